@@ -6,6 +6,7 @@
 
 #include "hq_device.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -74,45 +75,194 @@ __global__ void k_norm(const cplx<R>* __restrict__ a, uint64_t n_amps, int targe
     if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
-// Sum of p_i, p_i * bit_q(i) and p_i * (bit_q ^ bit_{q+1}) per block.
-template <typename R>
-__global__ void k_expect_z(const cplx<R>* __restrict__ a, int n, double* __restrict__ out)
+// ---- <Z_q>, <Z_q Z_{q+1}> -------------------------------------------------------------
+// Row layout of a block's partials: sum p, sum p bit_q (RED_MAXQ columns),
+// sum p (bit_q xor bit_{q+1}) (RED_MAXQ columns); columns of absent qubits
+// hold zeros.
+constexpr int RED_Z_BLOCKS = 256;
+constexpr int RED_Z_STRIDE = 1 + 2 * RED_MAXQ;
+constexpr int EZ_THREADS = 1024;
+constexpr int EZ_CHUNK_BITS = 13;   // 1024 threads x 8 amplitudes
+
+// Sum over the 64 lanes of each of the N columns v[0..N) (N <= 64); lane L
+// returns column bitreverse6(L).  Every step folds pairs of columns into one,
+// each half of the wave keeping one of the pair: N shuffles instead of 6 N.
+template <int N, int M>
+__device__ __forceinline__ double wave_columns(double* v, int lane)
 {
-    __shared__ double sh[16];
-    double tot = 0, s1[RED_MAXQ], s2[RED_MAXQ];
+    if constexpr (M == 0) {
+        return v[0];
+    } else {
+        const bool up = (lane & M) != 0;
 #pragma unroll
-    for (int q = 0; q < RED_MAXQ; q++) { s1[q] = 0; s2[q] = 0; }
-    uint64_t n_amps = (uint64_t)1 << n;
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_amps; i += stride) {
-        cplx<R> v = a[i];
-        double p = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
-        tot += p;
-#pragma unroll
-        for (int q = 0; q < RED_MAXQ; q++) {
-            if (q < n) {
-                uint64_t b = (i >> q) & 1, b2 = (i >> (q + 1)) & 1;
-                s1[q] += b ? p : 0.0;
-                s2[q] += (b ^ b2) ? p : 0.0;
+        for (int i = 0; i < (N + 1) / 2; i++) {
+            if (2 * i + 1 < N) {
+                const double keep = up ? v[2 * i + 1] : v[2 * i];
+                const double send = up ? v[2 * i] : v[2 * i + 1];
+                v[i] = keep + __shfl_xor(send, M);
+            } else {
+                v[i] = v[2 * i] + __shfl_xor(v[2 * i], M);
             }
         }
+        return wave_columns<(N + 1) / 2, M / 2>(v, lane);
     }
-    int stride_out = 1 + 2 * RED_MAXQ;
-    double r = block_sum(tot, sh);
-    if (threadIdx.x == 0) out[blockIdx.x * stride_out] = r;
+}
+
+// One row of partials per block, one read of the state.  HBM-bound by
+// construction: an index bit's weight is a constant of the place that holds
+// it, so per amplitude only p is formed and added to one of the thread's
+// eight accumulators; nothing is added per qubit and amplitude (that form
+// spent 2 n additions on every amplitude: 64.6 ms at 30 qubits complex128,
+// 129 ms at 31 qubits complex64; this one 2.92 ms = 5.9 TB/s and 3.22 ms =
+// 5.3 TB/s).
+//   index bits   held by
+//   0..12        lane (6), register (3), wave (4): weighted once at the end
+//   13..12+l     the block's loop over its 2^l consecutive chunks (l <= LB):
+//                one conditional add per chunk, thread and bit
+//   above        the block index: weighted in the row
+// A lane moves 16 bytes per load: one complex128 amplitude, or two
+// neighbouring complex64 ones (bit 0 is then a register bit).
+template <typename R, int LB>
+__global__ __launch_bounds__(EZ_THREADS) void k_expect_z(const cplx<R>* __restrict__ a, int n, int l,
+                                                         double* __restrict__ out)
+{
+    constexpr bool PAIR = sizeof(R) == 4;
+    constexpr int NCOL = 20 + 2 * LB;
+    __shared__ double sh[EZ_THREADS / 64][NCOL];
+    const uint64_t amps = (uint64_t)1 << n;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t blk = blockIdx.x;
+    double acc[8];
 #pragma unroll
-    for (int q = 0; q < RED_MAXQ; q++) {
-        if (q < n) {
-            double r1 = block_sum(s1[q], sh);
-            if (threadIdx.x == 0) out[blockIdx.x * stride_out + 1 + q] = r1;
-            double r2 = block_sum(s2[q], sh);
-            if (threadIdx.x == 0) out[blockIdx.x * stride_out + 1 + RED_MAXQ + q] = r2;
-        } else if (threadIdx.x == 0) {
-            // columns of absent qubits hold zeros: every column is defined
-            out[blockIdx.x * stride_out + 1 + q] = 0.0;
-            out[blockIdx.x * stride_out + 1 + RED_MAXQ + q] = 0.0;
+    for (int j = 0; j < 8; j++) acc[j] = 0;
+    double s[LB > 0 ? LB : 1], zz[LB > 0 ? LB : 1], zw = 0;
+#pragma unroll
+    for (int b = 0; b < LB; b++) { s[b] = 0; zz[b] = 0; }
+    const uint64_t c0 = blk << l, c1 = c0 + ((uint64_t)1 << l);
+    for (uint64_t c = c0; c < c1; c++) {
+        double p[8];
+        const uint64_t base = (c << EZ_CHUNK_BITS) | ((uint64_t)wave << 9);
+        if constexpr (PAIR) {
+            struct alignas(16) Two { cplx<R> v[2]; };
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint64_t i = base | (uint64_t)(k << 7 | lane << 1);
+                Two t = {};
+                if (i < amps) t = *(const Two*)(a + i);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    p[2 * k + h] = (double)t.v[h].x * (double)t.v[h].x + (double)t.v[h].y * (double)t.v[h].y;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint64_t i = base | (uint64_t)(j << 6 | lane);
+                cplx<R> t = {};
+                if (i < amps) t = a[i];
+                p[j] = (double)t.x * (double)t.x + (double)t.y * (double)t.y;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[j] += p[j];
+        const double t = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        // uniform conditions: scalar branches
+        const uint64_t x = c ^ (c >> 1);
+        if (((uint64_t)(wave >> 3) ^ c) & 1) zw += t;
+#pragma unroll
+        for (int b = 0; b < LB; b++) {
+            if ((c >> b) & 1) s[b] += t;
+            if ((x >> b) & 1) zz[b] += t;
         }
     }
+    // thread columns: 0 total; 1..6 lane bits; 7..11 neighbouring lane bits;
+    // 12..14 register bits; 15 register bits 1,2; 16, 17 the two pairs between
+    // lane and register bits (complex128: register bits 0,1 take 16); 18 the
+    // last register and the first wave bit; 19 the last wave bit and chunk bit
+    // 0; then the chunk bits and their pairs
+    {
+        double v[NCOL];
+        double half[3][2];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                double t = 0;
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (((j >> r) & 1) == h) t += acc[j];
+                half[r][h] = t;
+            }
+        auto cross = [&](int r0, int r1) {
+            double t = 0;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (((j >> r0) ^ (j >> r1)) & 1) t += acc[j];
+            return t;
+        };
+        const double T = half[0][0] + half[0][1];
+        v[0] = T;
+#pragma unroll
+        for (int k = 0; k < 6; k++) v[1 + k] = ((lane >> k) & 1) ? T : 0.0;
+#pragma unroll
+        for (int k = 0; k < 5; k++) v[7 + k] = (((lane ^ (lane >> 1)) >> k) & 1) ? T : 0.0;
+#pragma unroll
+        for (int r = 0; r < 3; r++) v[12 + r] = half[r][1];
+        v[15] = cross(1, 2);
+        if constexpr (PAIR) {
+            v[16] = (lane & 1) ? half[0][0] : half[0][1];
+            v[17] = (lane >> 5) ? half[1][0] : half[1][1];
+        } else {
+            v[16] = cross(0, 1);
+            v[17] = (lane >> 5) ? half[0][0] : half[0][1];
+        }
+        v[18] = (wave & 1) ? half[2][0] : half[2][1];
+        v[19] = zw;
+#pragma unroll
+        for (int b = 0; b < LB; b++) { v[20 + b] = s[b]; v[20 + LB + b] = zz[b]; }
+        const double r = wave_columns<NCOL, 32>(v, lane);
+        const int col = (int)(__brev((unsigned)lane) >> 26);
+        if (col < NCOL) sh[wave][col] = r;
+    }
+    __syncthreads();
+    const int o = threadIdx.x;
+    if (o >= RED_Z_STRIDE) return;
+    // row column o: qubit q's bit (pair = 0) or the pair q, q+1
+    const bool pair = o > RED_MAXQ;
+    const int q = o == 0 ? -1 : pair ? o - 1 - RED_MAXQ : o - 1;
+    int col = 0;            // thread column summed over the waves with weight 1 ...
+    int wmask = -1;         // ... or, >= 0: over the waves whose index has odd parity under it
+    bool zero = false;
+    constexpr int LANE0 = PAIR ? 1 : 0;   // qubit of lane bit 0
+    if (q < 0) {
+        col = 0;
+    } else if (q + (pair ? 1 : 0) >= n) {
+        zero = true;
+    } else if (q >= EZ_CHUNK_BITS + LB) {
+        const uint64_t c = blk << l;      // constant over the block
+        const uint64_t y = pair ? c ^ (c >> 1) : c;
+        zero = !((y >> (q - EZ_CHUNK_BITS)) & 1);
+    } else if (q >= EZ_CHUNK_BITS) {
+        col = 20 + (pair ? LB : 0) + (q - EZ_CHUNK_BITS);
+    } else if (!pair) {
+        if (q >= 9) wmask = 1 << (q - 9);
+        else if (q >= 7) col = 12 + (q - 6);
+        else if (PAIR && q == 0) col = 12;
+        else if (!PAIR && q == 6) col = 12;
+        else col = 1 + (q - LANE0);
+    } else {
+        if (q == 12) col = 19;
+        else if (q >= 9) wmask = 3 << (q - 9);
+        else if (q == 8) col = 18;
+        else if (q == 7) col = 15;
+        else if (PAIR) col = q == 6 ? 17 : q == 0 ? 16 : 7 + (q - 1);
+        else col = q == 6 ? 16 : q == 5 ? 17 : 7 + q;
+    }
+    double r = 0;
+    if (!zero)
+        for (int w = 0; w < EZ_THREADS / 64; w++)
+            if (wmask < 0 || (__popc(w & wmask) & 1)) r += sh[w][col];
+    out[blk * RED_Z_STRIDE + o] = r;
 }
 
 template <typename RA, typename RB>
@@ -135,23 +285,24 @@ __global__ void k_inner(const cplx<RA>* __restrict__ a, const cplx<RB>* __restri
     if (threadIdx.x == 0) out[2 * blockIdx.x + 1] = r2;
 }
 
-// Fixed-order Kahan sum of column c of `count` partial rows (row stride
-// `stride`) into fin[c], one thread per column: the same operations in the
-// same order as the host-side sum of the partials (sum_partials), so both
-// give the same FP64 result bit for bit.
-__global__ void k_sum_columns(const double* __restrict__ part, int count, int stride, int cols,
-                              double* __restrict__ fin)
+// Column sums of `count` rows (row stride `stride`) into fin, one wave per
+// column: lane i takes rows i, i + 64, ... with a Kahan sum, then a fixed tree
+// over the lanes.  fin may be host memory the device can write.
+__global__ __launch_bounds__(64) void k_sum_columns(const double* __restrict__ part, int count, int stride,
+                                                    double* __restrict__ fin)
 {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
+    const int c = blockIdx.x;
     double sum = 0, comp = 0;
-    for (int b = 0; b < count; b++) {
+#pragma unroll 4
+    for (int b = threadIdx.x; b < count; b += 64) {
         double y = part[(size_t)b * stride + c] - comp;
         double t = sum + y;
         comp = (t - sum) - y;
         sum = t;
     }
-    fin[c] = sum;
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) sum += __shfl_xor(sum, m);
+    if (threadIdx.x == 0) fin[c] = sum;
 }
 
 // ---- allocation-free readout -----------------------------------------------------------
@@ -160,8 +311,6 @@ __global__ void k_sum_columns(const double* __restrict__ part, int count, int st
 // column sums.  One copy per device, held until the process ends; host code
 // addresses it only through the pointer hipGetSymbolAddress returns for the
 // device (noalloc_scratch below).
-constexpr int RED_Z_BLOCKS = 256;
-constexpr int RED_Z_STRIDE = 1 + 2 * RED_MAXQ;
 constexpr size_t NOALLOC_SCRATCH_DOUBLES = (size_t)(RED_Z_BLOCKS + 1) * RED_Z_STRIDE;   // 147 KiB
 static __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 
@@ -426,14 +575,41 @@ hq_status hq_measure_zero(hq_state s, int target, double* p0)
     return run_norm(s, target, p0);
 }
 
-static void launch_expect_z(hq_state s, unsigned g, double* partials)
+// Column sums of the state (the layout of a k_expect_z row) into fin, device
+// or device-writable host memory; rows: RED_Z_BLOCKS rows of device scratch,
+// unused by a state of one chunk.  Asynchronous.
+static hq_status launch_expect_z(hq_state s, double* rows, double* fin)
 {
-    if (s->precision == HQ_C128)
-        hipLaunchKernelGGL(k_expect_z<double>, dim3(g), dim3(RED_THREADS), 0, s->stream,
-                           (const cplx<double>*)s->data, s->n, partials);
-    else
-        hipLaunchKernelGGL(k_expect_z<float>, dim3(g), dim3(RED_THREADS), 0, s->stream,
-                           (const cplx<float>*)s->data, s->n, partials);
+    // one chunk per block up to RED_Z_BLOCKS blocks (2^21 amplitudes), then
+    // 2^l consecutive chunks per block: 16 waves on every CU, and at most
+    // RED_Z_BLOCKS rows.  LB, the loop bits a kernel has columns for, costs
+    // registers (two doubles a thread each) and reduction steps, so it is
+    // 0, 10 or 15 by size
+    const int cb = std::max(0, s->n - EZ_CHUNK_BITS);
+    const int l = std::max(0, cb - 8);
+    const unsigned g = 1u << (cb - l);
+    static_assert(RED_Z_BLOCKS == 1 << 8, "block bits");
+    double* part = g > 1 ? rows : fin;
+#define HQ_EZ(RV, LBV)                                                                                          \
+    hipLaunchKernelGGL((k_expect_z<RV, LBV>), dim3(g), dim3(EZ_THREADS), 0, s->stream, (const cplx<RV>*)s->data, \
+                       s->n, l, part)
+    if (s->precision == HQ_C128) {
+        if (l == 0) HQ_EZ(double, 0);
+        else if (l <= 10) HQ_EZ(double, 10);
+        else HQ_EZ(double, 15);
+    } else {
+        if (l == 0) HQ_EZ(float, 0);
+        else if (l <= 10) HQ_EZ(float, 10);
+        else HQ_EZ(float, 15);
+    }
+#undef HQ_EZ
+    HQ_HIP(hipGetLastError());
+    if (g > 1) {
+        hipLaunchKernelGGL(k_sum_columns, dim3(RED_Z_STRIDE), dim3(64), 0, s->stream, (const double*)rows, (int)g,
+                           RED_Z_STRIDE, fin);
+        HQ_HIP(hipGetLastError());
+    }
+    return HQ_OK;
 }
 
 // z[q] = <Z_q>, zz[q] = <Z_q Z_{q+1}> from the column sums of k_expect_z
@@ -451,18 +627,13 @@ hq_status hq_expect_z(hq_state s, double* z, double* zz)
 {
     HQ_CHECK(s, HQ_ERR_ARG, "hq_expect_z: null state");
     HQ_CHECK(s->n <= RED_MAXQ, HQ_ERR_UNSUPPORTED, "hq_expect_z: at most 36 qubits");
-    const int stride = RED_Z_STRIDE;
-    unsigned g = grid_for(s->amps, RED_THREADS, RED_Z_BLOCKS);
-    hq_status st = ensure_red(s, (size_t)g * stride);
+    hq_status st = ensure_red(s, (size_t)RED_Z_BLOCKS * RED_Z_STRIDE);
     if (st != HQ_OK) return st;
-    launch_expect_z(s, g, s->d_red);
-    HQ_HIP(hipGetLastError());
-    HQ_HIP(hipMemcpyAsync(s->h_red, s->d_red, (size_t)g * stride * sizeof(double), hipMemcpyDeviceToHost,
-                          s->stream));
+    // the sums go straight to the pinned buffer: no copy to wait for
+    st = launch_expect_z(s, s->d_red, s->h_red);
+    if (st != HQ_OK) return st;
     HQ_HIP(hipStreamSynchronize(s->stream));
-    double col[RED_Z_STRIDE];
-    for (int c = 0; c < stride; c++) sum_partials(s, (int)g, stride, c, &col[c]);
-    finish_expect_z(s->n, col, z, zz);
+    finish_expect_z(s->n, s->h_red, z, zz);
     return HQ_OK;
 }
 
@@ -470,24 +641,16 @@ hq_status hq_expect_z_noalloc(hq_state s, double* z, double* zz)
 {
     HQ_CHECK(s, HQ_ERR_ARG, "hq_expect_z_noalloc: null state");
     HQ_CHECK(s->n <= RED_MAXQ, HQ_ERR_UNSUPPORTED, "hq_expect_z_noalloc: at most 36 qubits");
-    const int stride = RED_Z_STRIDE;
-    unsigned g = grid_for(s->amps, RED_THREADS, RED_Z_BLOCKS);
-    HQ_CHECK((size_t)(g + 1) * stride <= NOALLOC_SCRATCH_DOUBLES, HQ_ERR_ARG,
-             "hq_expect_z_noalloc: partials exceed the " + std::to_string(NOALLOC_SCRATCH_DOUBLES) +
-                 "-double scratch");
     double* ptr = nullptr;
     hq_status st = noalloc_scratch(s->device, &ptr);
     if (st != HQ_OK) return st;
     // every partial row and the column-sum row are written before they are
     // read: nothing in the scratch has to start at zero
-    launch_expect_z(s, g, ptr);
-    HQ_HIP(hipGetLastError());
-    double* fin = ptr + (size_t)g * stride;
-    hipLaunchKernelGGL(k_sum_columns, dim3(1), dim3(128), 0, s->stream, (const double*)ptr, (int)g, stride,
-                       stride, fin);
-    HQ_HIP(hipGetLastError());
+    double* fin = ptr + (size_t)RED_Z_BLOCKS * RED_Z_STRIDE;
+    st = launch_expect_z(s, ptr, fin);
+    if (st != HQ_OK) return st;
     double col[RED_Z_STRIDE];
-    HQ_HIP(hipMemcpyAsync(col, fin, stride * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    HQ_HIP(hipMemcpyAsync(col, fin, RED_Z_STRIDE * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HQ_HIP(hipStreamSynchronize(s->stream));
     finish_expect_z(s->n, col, z, zz);
     return HQ_OK;

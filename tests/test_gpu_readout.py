@@ -1,0 +1,55 @@
+"""Readouts of a device state at the edges of their kernels' tiles, against
+numpy in float64 on the same amplitudes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(gpu, n, prec, seed):
+    """A state with uploaded random amplitudes; (state, |a|^2 in float64)."""
+    rs = np.random.default_rng([seed, n, prec])
+    psi = rs.standard_normal((1 << n, 2)) / np.sqrt(2.0 * (1 << n))
+    psi = (psi[:, 0] + 1j * psi[:, 1]).astype(np.complex128 if prec == 0 else np.complex64)
+    s = gpu.State(n, gpu.HQ_C128 if prec == 0 else gpu.HQ_C64)
+    s.upload(psi)
+    a = psi.astype(np.complex128)
+    return s, a.real ** 2 + a.imag ** 2
+
+
+# below, at and above one 13-bit chunk; 8 chunk bits fill the grid at 21
+# qubits, the loop over chunks starts at 22
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [1, 2, 6, 7, 9, 10, 12, 13, 14, 17, 21, 22, 24])
+def test_expect_z_tiles(gpu, n, prec):
+    s, p = _state(gpu, n, prec, 11)
+    z, zz = s.expect_z()
+    # sums of at most 2^24 terms that total about 1, in trees: far below 1e-13
+    for q in range(n):
+        m = p.reshape(-1, 2, 1 << q).sum((0, 2))
+        assert abs(z[q] - (m[0] - m[1])) <= 1e-13, (n, q)
+        if q + 1 < n:
+            m = p.reshape(-1, 2, 2, 1 << q).sum((0, 3))
+            assert abs(zz[q] - (m[0, 0] + m[1, 1] - m[0, 1] - m[1, 0])) <= 1e-13, (n, q)
+    s.close()
+
+
+def test_expect_z_largest_loop(gpu):
+    """32 qubits: more than 10 loop bits.  A product state: RY(theta) on every
+    third qubit, X on every seventh, |0> elsewhere."""
+    n = 32
+    s = gpu.State(n, gpu.HQ_C64)
+    gates, want = [], np.ones(n)
+    for q in range(n):
+        if q % 7 == 3:
+            gates.append(gpu.Gate.X(q))
+            want[q] *= -1
+        if q % 3 == 1:
+            gates.append(gpu.Gate.RY(q, 0.3 + 0.05 * q))
+            want[q] *= np.cos(0.3 + 0.05 * q)
+    s.apply_plain(gates)
+    z, zz = s.expect_z()
+    s.close()
+    # single-precision gates: one rounding of 6e-8 per coefficient and product, 15 gates
+    assert np.max(np.abs(z - want)) <= 5e-6
+    assert np.max(np.abs(zz - want[:-1] * want[1:])) <= 5e-6
