@@ -82,9 +82,10 @@ template <typename R, int RB, int TB>
 __global__ __launch_bounds__(1 << TB) void k_batch_sharemem(const BatchItem* __restrict__ items, uint32_t count)
 {
     __shared__ cplx<R> lds[1 << (RB + TB)];
+    __shared__ __align__(16) char win[SHM_WINDOW_LDS];
     const uint64_t b = blockIdx.x;
     const BatchItem* it = items + find_item(items, count, b);
-    tile_pass<R, RB, TB>((cplx<R>*)it->psi, (const char*)it->prog, b - it->first_block, lds, it->mode, (int)it->n,
+    tile_pass<R, RB, TB>((cplx<R>*)it->psi, (const char*)it->prog, b - it->first_block, lds, win, it->mode, (int)it->n,
                          (double*)it->part);
 }
 
@@ -476,21 +477,17 @@ static int tile_for(const EngineOptions& o, int n)
 static hq_status append_blob(JobPlan* jp, const ShmPlan& plan)
 {
     for (const ShmOp& op : plan.ops)
-        HQ_CHECK(op.cls <= SHM_SCALE, HQ_ERR_UNSUPPORTED, "engine: op class the interpreter does not implement");
+        HQ_CHECK(op.cls != SHM_SHEAR && op.cls != SHM_SHEARX, HQ_ERR_UNSUPPORTED,
+                 "engine: op class the interpreter does not implement");
     GroupPlan g;
     g.rb = plan.rb;
     g.tb = plan.tb;
     g.k = plan.k;
-    g.nops = (uint32_t)plan.ops.size();
-    size_t off = (jp->blobs.size() + 255) & ~(size_t)255;
-    const size_t bytes = sizeof(ShmHeader) + plan.stages.size() * sizeof(ShmStage) + plan.ops.size() * sizeof(ShmOp);
-    jp->blobs.resize(off + bytes);
-    char* d = jp->blobs.data() + off;
-    memcpy(d, &plan.hdr, sizeof(ShmHeader));
-    memcpy(d + sizeof(ShmHeader), plan.stages.data(), plan.stages.size() * sizeof(ShmStage));
-    if (!plan.ops.empty())
-        memcpy(d + sizeof(ShmHeader) + plan.stages.size() * sizeof(ShmStage), plan.ops.data(),
-               plan.ops.size() * sizeof(ShmOp));
+    g.nops = plan.hdr.num_ops;
+    const std::vector<char> blob = encode_program(plan);
+    const size_t off = (jp->blobs.size() + 255) & ~(size_t)255;
+    jp->blobs.resize(off + blob.size());
+    memcpy(jp->blobs.data() + off, blob.data(), blob.size());
     g.blob_off = off;
     jp->groups.push_back(g);
     return HQ_OK;
@@ -504,7 +501,7 @@ static void append_jit(JobPlan* jp, const ShmPlan& plan, const std::vector<doubl
     g.rb = plan.rb;
     g.tb = plan.tb;
     g.k = plan.k;
-    g.nops = (uint32_t)plan.ops.size();
+    g.nops = plan.hdr.num_ops;
     g.fn = fn;
     const size_t rbytes = plan.precision == HQ_C128 ? 8 : 4;
     size_t off = (jp->blobs.size() + 255) & ~(size_t)255;
@@ -532,7 +529,7 @@ static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<
     const double live = first ? 0.5 : std::ldexp(1.0, -__builtin_popcountll(zero_mask & ~mask));
     // groups of more than kJitMaxOps ops stay with the interpreter (compile time)
     constexpr size_t kJitMaxOps = 512;
-    if (kc && plan.ops.size() <= kJitMaxOps) {
+    if (kc && plan.hdr.num_ops <= kJitMaxOps) {
         plan.init = first;
         std::vector<double> coef;
         const std::string src = jit_source(plan, &coef, true, last);

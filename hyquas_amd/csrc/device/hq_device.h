@@ -89,26 +89,40 @@ enum ShmClass : uint8_t {
     // shears, a = m[0], b = m[2], |a|, |b| <= 1
     SHM_SHEAR = 13,  // lo += a hi, hi += b lo, lo += a hi        (RY)
     SHM_SHEARX = 14, // lo += i a hi, hi -= i b lo, lo += i a hi  (RX)
+    // diagonal factors of a stage, merged by the planner (SHM_DIAG and
+    // SHM_PHASE are gate classes only: no op of a plan carries them)
+    SHM_TAB = 15,    // amplitude of register index j *= table[j]
+    SHM_MIX = 16,    // (m[0], m[1]) where register, thread and block bits match
+    SHM_LANE = 17,   // the lane's factor *= (m[0], m[1]) where thread and block bits match
+    SHM_LANEMUL = 18 // every amplitude *= the lane's factor * (m[0], m[1]); the factor is 1 again
 };
 
-enum ShmWhere : uint8_t { SHM_IN_REG = 0, SHM_IN_THREAD = 1, SHM_IN_BLOCK = 2 };
-
+// One op of a stage.  A condition is a mask and the value the masked bits
+// must have; pair updates (SHM_SWAP..SHM_RXB and the shears, target register
+// bit tpos) take all-ones values: their controls.
 struct ShmOp {
-    uint8_t cls;
-    uint8_t where;      // ShmWhere of the target
-    uint8_t tpos;       // register-index bit / thread-index bit / block-index bit
-    uint8_t pad0;
-    uint32_t creg;      // control mask over register-index bits
-    uint32_t cthr;      // control mask over thread-index bits
-    uint32_t flags;     // SHM_FLAG_*
-    uint64_t cblk;      // control mask over block-index bits
-    double m[8];        // coefficients, re/im interleaved, row-major 2x2
+    uint8_t cls = 0;
+    uint8_t tpos = 0;        // pair updates: register-index bit of the target
+    uint8_t creg = 0, cregv = 0;     // over register-index bits
+    uint16_t cthr = 0, cthrv = 0;    // over thread-index bits
+    uint32_t cblk = 0, cblkv = 0;    // over block-index bits (at most 29)
+    uint32_t flags = 0;      // SHM_FLAG_*
+    uint32_t tab = 0;        // SHM_TAB: first entry in ShmPlan::tabs (2^rb entries)
+    uint64_t jmask = 0;      // SHM_TAB: register indices whose entry is not 1 by structure
+    uint64_t jprod = 0;      // SHM_TAB, precise plans: entries that are products of several gates' factors
+    uint32_t jdep = 0;       // SHM_TAB: register-index bits the table depends on
+    double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // re/im interleaved, row-major 2x2
 };
-static_assert(sizeof(ShmOp) == 88, "ShmOp layout");
 
 // the op's coefficients are fixed by its gate type (H, T, CNOT, ...), so a
 // specialised kernel may embed them as constants
 constexpr uint32_t SHM_FLAG_CONST = 1;
+// SHM_MIX, SHM_LANE, SHM_LANEMUL: the factor is real by structure (Z, CZ signs)
+constexpr uint32_t SHM_FLAG_REAL = 2;
+// SHM_LANEMUL: (m[0], m[1]) is exactly 1 by structure
+constexpr uint32_t SHM_FLAG_UNIT = 4;
+// SHM_LANEMUL: no SHM_LANE op before it (the lane's factor is 1)
+constexpr uint32_t SHM_FLAG_NOLANE = 8;
 
 constexpr int SHM_MAX_TILE = 14;
 constexpr int SHM_MAX_TB = 9;
@@ -126,14 +140,76 @@ struct ShmHeader {
     uint32_t swz_col[SHM_MAX_TILE];    // LDS swizzle column of tile bit i
     uint32_t num_block_bits;
     uint32_t num_stages;
-    uint32_t num_ops;
+    uint32_t num_ops;          // lowered gates and the final scale (before diagonal factors are merged)
     uint32_t pad;
     // tiles whose block address has a bit in zero_mask hold only zeros before
     // the pass (the run started from |0...0> and no earlier group reached
     // those qubits) and keep them: the pass skips them
     uint64_t zero_mask;
-    // followed by ShmStage[num_stages], ShmOp[num_ops] (8-byte aligned)
 };
+
+// ---- the interpreter's program: header, op slots, lane tables ---------------------------
+// A slot is 16 bytes of decoded fields and eight coefficients in the state's
+// precision.  The kernel copies slots to LDS a window at a time (one memory
+// latency per window instead of several per op) and reads the next slot while
+// it executes one.
+struct ShmSlot {
+    uint8_t kind, aux;           // SlotKind; target register bit, or table slots that follow
+    uint8_t creg, cregv;
+    uint16_t cthr, cthrv;
+    uint32_t cblk, cblkv;
+};
+static_assert(sizeof(ShmSlot) == 16, "ShmSlot layout");
+
+enum SlotKind : uint8_t {
+    // pair updates: the ShmClass value (SHM_SWAP..SHM_GEN, SHM_HADD..SHM_RXB)
+    SLOT_CSWAP = 32,     // SHM_SWAP under a thread-bit control
+    SLOT_SCALE = 33,     // every amplitude *= (m[0], m[1])
+    SLOT_TAB = 34,       // complex table of the 2^RB register indices in the next `aux` slots
+    SLOT_TABMASK = 35,   // the same; only register indices in cblkv:cblk are multiplied
+    SLOT_MIX = 36,
+    SLOT_MIXSIGN = 37,   // factor -1
+    SLOT_LANE = 38,
+    SLOT_LANETAB = 39,   // the lane's factor = thread's entry of the lane table cblk (of this program)
+    SLOT_LANEMUL = 40,   // every amplitude *= the lane's factor
+    SLOT_XCHG = 41,      // LDS exchange into the next stage's split
+    SLOT_REFILL = 42,    // copy the next window of slots to LDS
+    SLOT_END = 43,
+};
+
+constexpr int SHM_WINDOW_BYTES = 7680;   // 96 slots of complex128, 160 of complex64
+template <typename R> constexpr int shm_slot_bytes() { return 16 + 8 * (int)sizeof(R); }
+template <typename R> constexpr int shm_window_slots() { return SHM_WINDOW_BYTES / shm_slot_bytes<R>(); }
+constexpr int SHM_WINDOW_COPY = 8192;    // copied at a time, in whole 16-byte pieces of 64 to 512 threads
+constexpr int SHM_WINDOW_LDS = SHM_WINDOW_COPY;
+static_assert(SHM_WINDOW_COPY >= SHM_WINDOW_BYTES + 80, "the slot behind a window's last one is read ahead");
+
+// exchange slots: swizzled LDS index of each thread and register bit of the
+// stage they lead to
+struct ShmXchg {
+    uint16_t thr[SHM_MAX_TB];
+    uint16_t reg[SHM_MAX_RB];
+};
+static_assert(sizeof(ShmXchg) <= 32, "an exchange fits the coefficients of a complex64 slot");
+
+struct ShmRun {                // base |= ((block >> src) & mask) << dst
+    uint32_t src, dst;
+    uint64_t mask;
+};
+
+struct ShmProg {
+    uint32_t num_runs, num_slots;
+    uint32_t lane_off;         // lane tables, bytes from the program's start
+    uint32_t pad;
+    uint64_t zero_mask;
+    uint8_t ld_thr[SHM_MAX_TB + 1], ld_reg[SHM_MAX_RB];   // physical position of each bit, first stage
+    uint8_t st_thr[SHM_MAX_TB + 1], st_reg[SHM_MAX_RB];   // last stage
+    ShmXchg first;             // the first stage's LDS indices
+    uint16_t pad2;
+    ShmRun run[SHM_MAX_TILE + 1];   // block bits in runs of consecutive positions
+};
+constexpr size_t SHM_PROG_HEADER = 512;
+static_assert(sizeof(ShmProg) <= SHM_PROG_HEADER, "ShmProg header size");
 
 // Host-side result of lowering + register-stage planning of one group.
 struct ShmPlan {
@@ -141,11 +217,19 @@ struct ShmPlan {
     bool init = false;        // start from |0...0> instead of loading (first group of a run)
     bool nt_load = false;     // specialised kernel: non-temporal HBM loads
     bool nt_store = false;    // specialised kernel: non-temporal HBM stores
+    // complex64: a merged diagonal factor is held and applied as a sum of two
+    // floats.  Rounded to one float, the moduli of its entries are each off by
+    // up to 2^-24 in a pattern over the index bits, the same in every tile, and
+    // <Z_q> of a large state (of order 2^(-n/2)) reads that pattern: at 31
+    // qubits it moved <Z> by 4e-4 of its size.  Gate by gate the rounded
+    // products average out over the amplitudes.
+    bool precise = false;
     bool whole_line = false;  // planned with the whole-line HBM stages (io = 3)
     uint64_t shared_mask = 0;
     ShmHeader hdr;
     std::vector<ShmStage> stages;
     std::vector<ShmOp> ops;
+    std::vector<double> tabs;  // SHM_TAB entries, re/im interleaved
 };
 
 }  // namespace hq
@@ -185,10 +269,14 @@ int sharemem_default_rb(int precision, int tile);
 // io: bit 0 adds a leading, bit 1 a trailing stage without gates where the
 // first / last stage holds one of the three lowest tile bits in registers
 // (the HBM access then covers whole 128-byte lines per wave instruction).
+// merge: diagonal gates merged across the stage (false: applied gate by gate).
 // shared_code: op classes that do not depend on gate angles (rotations keep
 // their full 2x2 form), so same-structure groups share a specialised kernel.
 hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gates, uint64_t shared_mask,
-                        int rb, ShmPlan* out, bool init = false, int io = 0, bool shared_code = false);
+                        int rb, ShmPlan* out, bool init = false, int io = 0, bool shared_code = false,
+                        bool merge = true);
+// The interpreter's program of a plan (ShmProg header, slots, lane tables).
+std::vector<char> encode_program(const ShmPlan& plan);
 // Specialised kernel for a planned group: generate, compile (cached), load.
 hq_status jit_sharemem(const ShmPlan& plan, hq_program p);
 hq_status launch_sharemem_jit(hq_state s, hq_program p);

@@ -75,6 +75,33 @@ __device__ __forceinline__ void scale(cplx<R>& v, R re, R im)
     v.y = re * y + im * x;
 }
 
+// A merged diagonal factor: complex128 as it is, complex64 as the sum of two
+// floats per part (ShmPlan::precise).
+template <typename R>
+struct Factor;
+template <>
+struct alignas(16) Factor<double> {
+    double x, y;
+    static __host__ __device__ Factor of(double re, double im) { return Factor{re, im}; }
+};
+template <>
+struct alignas(16) Factor<float> {
+    float x, y, lx, ly;
+    static __host__ __device__ Factor of(double re, double im)
+    {
+        const float x = (float)re, y = (float)im;
+        return Factor{x, y, (float)(re - (double)x), (float)(im - (double)y)};
+    }
+};
+
+__device__ __forceinline__ void scale(cplx<double>& v, const Factor<double>& f) { scale<double>(v, f.x, f.y); }
+__device__ __forceinline__ void scale(cplx<float>& v, const Factor<float>& f)
+{
+    const float x = v.x, y = v.y;
+    v.x = f.x * x - (f.y * y - (f.lx * x - f.ly * y));
+    v.y = f.x * y + (f.y * x + (f.lx * y + f.ly * x));
+}
+
 }  // namespace hq
 
 // Host-side classification (defined in pergate.hip).

@@ -243,25 +243,198 @@ struct Emitter {
           << r(j) << ".y = " << fr << " * v.y + " << fi << " * v.x; }\n";
     }
 
+    // `if` around an op under a block condition; true when one was opened
+    bool block_if(const ShmOp& op)
+    {
+        if (!op.cblk) return false;
+        o << "     if ((b & " << hex64(op.cblk) << ") == " << hex64(op.cblkv) << ") {\n";
+        return true;
+    }
+
+    // factor of a diagonal op: literals, or two runtime coefficients
+    void factor(const ShmOp& op, std::string* fr, std::string* fi)
+    {
+        if (op.flags & SHM_FLAG_CONST) {
+            *fr = lit(op.m[0], f32);
+            *fi = lit(op.m[1], f32);
+            return;
+        }
+        const size_t base = coef->size();
+        coef->push_back(op.m[0]);
+        coef->push_back(op.m[1]);
+        *fr = "cf[" + std::to_string(base) + "]";
+        *fi = "cf[" + std::to_string(base + 1) + "]";
+    }
+
+    // by the sum of two floats (precise complex64 plans): four operations more
+    void pair_scale_stmt(int j, const std::string& x, const std::string& y, const std::string& lx,
+                         const std::string& ly)
+    {
+        o << "      { const C v = " << r(j) << "; " << r(j) << ".x = " << x << " * v.x - (" << y << " * v.y - (" << lx
+          << " * v.x - " << ly << " * v.y)); " << r(j) << ".y = " << x << " * v.y + (" << y << " * v.x + (" << lx
+          << " * v.y + " << ly << " * v.x)); }\n";
+    }
+
+    void real_scale_stmt(int j, const std::string& f)
+    {
+        o << "      " << r(j) << ".x *= " << f << "; " << r(j) << ".y *= " << f << ";\n";
+    }
+
+    // one complex factor per register index, uniform over the block: only the
+    // entries the table's bits distinguish are loaded
+    void emit_tab(const ShmOp& op)
+    {
+        o << "    {\n";
+        std::vector<int> bits;
+        for (int i = 0; i < P.rb; i++)
+            if ((op.jdep >> i) & 1) bits.push_back(i);
+        for (uint32_t sub = 0; sub < (1u << bits.size()); sub++) {
+            int j = 0;
+            for (size_t i = 0; i < bits.size(); i++)
+                if ((sub >> i) & 1) j |= 1 << bits[i];
+            if (!((op.jmask >> j) & 1)) continue;
+            const size_t base = coef->size();
+            const double x = P.tabs[2 * (op.tab + j)], y = P.tabs[2 * (op.tab + j) + 1];
+            coef->push_back(x);
+            coef->push_back(y);
+            o << "      const R dx" << j << " = cf[" << base << "], dy" << j << " = cf[" << base + 1 << "];\n";
+            if (!((op.jprod >> j) & 1)) continue;
+            coef->push_back(x - (double)(float)x);
+            coef->push_back(y - (double)(float)y);
+            o << "      const R ex" << j << " = cf[" << base + 2 << "], ey" << j << " = cf[" << base + 3 << "];\n";
+        }
+        for (int j = 0; j < NR; j++)
+            if ((op.jmask >> j) & 1) {
+                const int e = j & (int)op.jdep;
+                const std::string d = std::to_string(e);
+                if ((op.jprod >> e) & 1) pair_scale_stmt(j, "dx" + d, "dy" + d, "ex" + d, "ey" + d);
+                else scale_stmt(j, "dx" + d, "dy" + d);
+            }
+        o << "    }\n";
+    }
+
+    void emit_mix(const ShmOp& op)
+    {
+        o << "    {\n";
+        const bool blockc = block_if(op);
+        std::string fr, fi;
+        factor(op, &fr, &fi);
+        const bool real = op.flags & SHM_FLAG_REAL;
+        if (op.cthr) {
+            o << "      const bool pc = (t & " << hex32(op.cthr) << ") == " << hex32(op.cthrv) << ";\n";
+            o << "      const R fr = pc ? " << fr << " : (R)1;\n";
+            if (!real) o << "      const R fi = pc ? " << fi << " : (R)0;\n";
+        } else {
+            o << "      const R fr = " << fr << ";\n";
+            if (!real) o << "      const R fi = " << fi << ";\n";
+        }
+        for (int j = 0; j < NR; j++) {
+            if ((j & op.creg) != op.cregv) continue;
+            if (real) real_scale_stmt(j, "fr");
+            else scale_stmt(j, "fr", "fi");
+        }
+        if (blockc) o << "     }\n";
+        o << "    }\n";
+    }
+
+    // the lane's factor (lx<n>, ly<n>): a few operations per lane and term in
+    // place of one product per amplitude and diagonal gate
+    int lane_id = 0;
+    enum { LANE_NONE, LANE_REAL, LANE_CPLX } lane = LANE_NONE;
+    void emit_lane(const ShmOp& op)
+    {
+        const std::string lx = "lx" + std::to_string(lane_id), ly = "ly" + std::to_string(lane_id);
+        if (lane == LANE_NONE) {
+            // precise plans form it in double: a few operations per lane
+            o << "    " << (P.precise ? "double " : "R ") << lx << " = 1, " << ly << " = 0;\n";
+            lane = LANE_REAL;
+        }
+        const bool real = op.flags & SHM_FLAG_REAL;
+        std::string fr, fi, pc;
+        factor(op, &fr, &fi);
+        if (op.cblk) pc = "(b & " + hex64(op.cblk) + ") == " + hex64(op.cblkv);
+        if (op.cthr) pc += std::string(pc.empty() ? "" : " && ") + "(t & " + hex32(op.cthr) + ") == " + hex32(op.cthrv);
+        o << "    {\n      const bool pc = " << pc << ";\n      const R fr = pc ? " << fr << " : (R)1;\n";
+        if (real) {
+            o << "      " << lx << " *= fr;";
+            if (lane == LANE_CPLX) o << " " << ly << " *= fr;";
+            o << "\n    }\n";
+            return;
+        }
+        o << "      const R fi = pc ? " << fi << " : (R)0;\n";
+        lane_times("fr", "fi");
+        o << "    }\n";
+    }
+    void lane_times(const std::string& fr, const std::string& fi)
+    {
+        const std::string lx = "lx" + std::to_string(lane_id), ly = "ly" + std::to_string(lane_id);
+        if (lane == LANE_REAL)
+            o << "      " << ly << " = " << lx << " * " << fi << "; " << lx << " = " << lx << " * " << fr << ";\n";
+        else
+            o << "      { const " << (P.precise ? "double" : "R") << " vx = " << lx << ", vy = " << ly << "; " << lx << " = " << fr << " * vx - " << fi
+              << " * vy; " << ly << " = " << fr << " * vy + " << fi << " * vx; }\n";
+        lane = LANE_CPLX;
+    }
+    void emit_lanemul(const ShmOp& op)
+    {
+        const std::string lx = "lx" + std::to_string(lane_id), ly = "ly" + std::to_string(lane_id);
+        o << "    {\n";
+        if (op.flags & SHM_FLAG_NOLANE) {
+            std::string fr, fi;
+            factor(op, &fr, &fi);
+            o << "      const R fr = " << fr << ", fi = " << fi << ";\n";
+            for (int j = 0; j < NR; j++) scale_stmt(j, "fr", "fi");
+        } else {
+            if (!(op.flags & SHM_FLAG_UNIT)) {
+                std::string fr, fi;
+                factor(op, &fr, &fi);
+                o << "      const R fr = " << fr << ", fi = " << fi << ";\n";
+                lane_times("fr", "fi");
+            }
+            if (P.precise) {
+                o << "      const R hx = (R)" << lx << ", hy = (R)" << ly << ";\n";
+                if (lane != LANE_REAL)
+                    o << "      const R ex = (R)(" << lx << " - (double)hx), ey = (R)(" << ly << " - (double)hy);\n";
+            }
+            for (int j = 0; j < NR; j++) {
+                if (lane == LANE_REAL) real_scale_stmt(j, P.precise ? "hx" : lx);   // signs alone
+                else if (P.precise) pair_scale_stmt(j, "hx", "hy", "ex", "ey");
+                else scale_stmt(j, lx, ly);
+            }
+            lane = LANE_NONE;
+            lane_id++;
+        }
+        o << "    }\n";
+    }
+
     void emit_op(const ShmOp& op, bool identity_ok_renaming)
     {
-        std::vector<std::string> m = coeffs(op);
+        switch (op.cls) {
+        case SHM_TAB: emit_tab(op); return;
+        case SHM_MIX: emit_mix(op); return;
+        case SHM_LANE: emit_lane(op); return;
+        case SHM_LANEMUL: emit_lanemul(op); return;
+        default: break;
+        }
+        // X, CNOT and CCX have no coefficients
+        std::vector<std::string> m = op.cls == SHM_SWAP ? std::vector<std::string>(8, "(R)0") : coeffs(op);
         const bool const_op = op.flags & SHM_FLAG_CONST;
         o << "    {\n";
-        bool blockc = op.cblk != 0;
-        if (blockc) o << "     if ((b & " << hex64(op.cblk) << ") == " << hex64(op.cblk) << ") {\n";
+        const bool blockc = block_if(op);
         // per-lane identity where a thread-bit control is 0
         std::vector<std::string> mv(8);
         static const char* ident[8] = {"(R)1", "(R)0", "(R)0", "(R)0", "(R)0", "(R)0", "(R)1", "(R)0"};
         if (op.cthr) {
-            o << "      const bool pc = (t & " << hex32(op.cthr) << ") == " << hex32(op.cthr) << ";\n";
-            for (int i = 0; i < 8; i++) {
-                o << "      const R m" << i << " = pc ? " << m[i] << " : " << ident[i] << ";\n";
-                mv[i] = "m" + std::to_string(i);
+            o << "      const bool pc = (t & " << hex32(op.cthr) << ") == " << hex32(op.cthrv) << ";\n";
+            if (op.cls != SHM_SWAP) {
+                for (int i = 0; i < 8; i++) {
+                    o << "      const R m" << i << " = pc ? " << m[i] << " : " << ident[i] << ";\n";
+                    mv[i] = "m" + std::to_string(i);
+                }
             }
         } else {
             for (int i = 0; i < 8; i++) {
-                if (const_op) {
+                if (const_op || op.cls == SHM_SWAP) {
                     mv[i] = m[i];
                 } else {
                     o << "      const R m" << i << " = " << m[i] << ";\n";
@@ -269,22 +442,25 @@ struct Emitter {
                 }
             }
         }
-        const bool rename = identity_ok_renaming && !blockc;
+        const bool rename = identity_ok_renaming && !blockc && !op.cthr;
         // the shear forms come from uncontrolled gates only; a per-lane
         // identity select would not express the identity for them
         if (op.cthr && (op.cls == SHM_SHEAR || op.cls == SHM_SHEARX))
             throw std::runtime_error("shear op with a thread-bit control");
-        if (op.cls == SHM_SCALE) {
-            for (int j = 0; j < NR; j++) scale_stmt(j, mv[0], mv[1]);
-        } else if (op.where == SHM_IN_REG) {
+        {
             const int Pb = op.tpos;
             for (int j = 0; j < NR; j++) {
                 if (j & (1 << Pb)) continue;
-                if ((j & op.creg) != op.creg) continue;
+                if ((j & op.creg) != op.cregv) continue;
                 const int jh = j | (1 << Pb);
                 switch (op.cls) {
                 case SHM_SWAP:
                     if (rename) std::swap(name[j], name[jh]);
+                    else if (op.cthr)
+                        // selects: half the VALU work of a 2x2 update with per-lane coefficients in complex64
+                        o << "      { const C lo = " << r(j) << ", hi = " << r(jh) << "; "
+                          << r(j) << ".x = pc ? hi.x : lo.x; " << r(j) << ".y = pc ? hi.y : lo.y; "
+                          << r(jh) << ".x = pc ? lo.x : hi.x; " << r(jh) << ".y = pc ? lo.y : hi.y; }\n";
                     else o << "      { const C tmp = " << r(j) << "; " << r(j) << " = " << r(jh) << "; " << r(jh) << " = tmp; }\n";
                     break;
                 case SHM_Y:
@@ -311,10 +487,6 @@ struct Emitter {
                       << r(j) << ".y = (" << mv[0] << " * lo.y + " << mv[1] << " * lo.x) + (" << mv[2] << " * hi.y + " << mv[3] << " * hi.x); "
                       << r(jh) << ".x = (" << mv[4] << " * lo.x - " << mv[5] << " * lo.y) + (" << mv[6] << " * hi.x - " << mv[7] << " * hi.y); "
                       << r(jh) << ".y = (" << mv[4] << " * lo.y + " << mv[5] << " * lo.x) + (" << mv[6] << " * hi.y + " << mv[7] << " * hi.x); }\n";
-                    break;
-                case SHM_DIAG:
-                    scale_stmt(j, mv[0], mv[1]);
-                    scale_stmt(jh, mv[6], mv[7]);
                     break;
                 case SHM_HADD:
                     o << "      { const C lo = " << r(j) << ", hi = " << r(jh) << "; " << r(j) << ".x = lo.x + hi.x; "
@@ -354,22 +526,9 @@ struct Emitter {
                       << "lo.x -= " << mv[0] << " * hi.y; lo.y += " << mv[0] << " * hi.x; "
                       << r(j) << " = lo; " << r(jh) << " = hi; }\n";
                     break;
-                default:  // SHM_PHASE
-                    scale_stmt(jh, mv[6], mv[7]);
-                    break;
+                default:
+                    throw std::runtime_error("op class without a specialised form");
                 }
-            }
-        } else {
-            // diagonal on a thread bit (per lane) or a block bit (uniform)
-            if (op.where == SHM_IN_THREAD)
-                o << "      const bool hb = (t >> " << (int)op.tpos << ") & 1u;\n";
-            else
-                o << "      const bool hb = (b >> " << (int)op.tpos << ") & 1ull;\n";
-            o << "      const R fr = hb ? " << mv[6] << " : " << mv[0] << ";\n";
-            o << "      const R fi = hb ? " << mv[7] << " : " << mv[1] << ";\n";
-            for (int j = 0; j < NR; j++) {
-                if ((j & op.creg) != op.creg) continue;
-                scale_stmt(j, "fr", "fi");
             }
         }
         if (blockc) o << "     }\n";

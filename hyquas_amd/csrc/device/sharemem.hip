@@ -36,7 +36,8 @@ __global__ __launch_bounds__(1 << TB) void k_sharemem(cplx<R>* __restrict__ psi,
                                                      uint32_t mode)
 {
     __shared__ cplx<R> lds[1 << (RB + TB)];
-    tile_pass<R, RB, TB>(psi, prog, blockIdx.x, lds, mode, 0, nullptr);
+    __shared__ __align__(16) char win[SHM_WINDOW_LDS];
+    tile_pass<R, RB, TB>(psi, prog, blockIdx.x, lds, win, mode, 0, nullptr);
 }
 
 // ---- launch table -------------------------------------------------------------------------
@@ -103,6 +104,7 @@ struct Lowered {
     int t_tile, t_block;  // target as tile bit or block bit (-1 if not)
     int c_tile[2], c_block[2];
     double m[8];
+    std::complex<double> scale{1.0, 0.0};   // factored out of m (applied later in the pass)
 };
 
 // Rotation [[c, -s], [s, c]] (c >= 0 after the sign is moved into the
@@ -209,10 +211,336 @@ int rank3(const std::vector<uint32_t>& v)
     return r;
 }
 
+// Turns the gates of the register stages into ops.  Diagonal gates are not
+// emitted where they stand: each is one or two factors ("terms") on the
+// amplitudes whose bits match, and a term commutes with every other term and
+// with every gate whose target is not one of its bits.  Terms stay pending
+// until a gate mixes one of their bits (or the pass ends) and are then applied
+// together:
+//   terms on register bits alone       one table over the register index
+//   terms on thread and block bits     one factor per lane, commuting with all
+//                                      of a stage's ops; in the last stage it
+//                                      carries the scale of the factored gates
+//   terms on both                      SHM_MIX, only if still mixed when forced
+// Register-controlled X permutes a pending table instead of forcing it.  One
+// table or lane factor costs 4 operations per amplitude whatever it merges; a
+// diagonal gate by itself costs 2 (register bit) or 4 (thread or block bit).
+class StageLowering {
+public:
+    StageLowering(const std::vector<Lowered>& low, const std::vector<int>& type, int precision, int rb, int tb,
+                  bool shared, bool precise, bool merge)
+        : low_(low), type_(type), rb_(rb), tb_(tb), nr_(1 << rb), shared_(shared), precise_(precise),
+          merge_(merge),          limit_(precision == HQ_C128 ? 480.0 : 48.0)
+    {
+    }
+
+    void stage(const ShmStage& st, const ShmStage* next, const std::vector<int>& gates, bool factored,
+               std::vector<ShmOp>* ops, std::vector<double>* tabs)
+    {
+        ops_ = ops;
+        tabs_ = tabs;
+        regset_ = set_of(st.reg_bits, rb_);
+        for (int i = 0; i < SHM_MAX_TILE; i++) reg_[i] = thr_[i] = -1;
+        for (int i = 0; i < rb_; i++) reg_[st.reg_bits[i]] = i;
+        for (int i = 0; i < tb_; i++) thr_[st.thr_bits[i]] = i;
+        reset_table();
+        for (int idx : gates) {
+            const Lowered& L = low_[idx];
+            if (L.needs_reg) mixing(L, type_[idx]);
+            else diagonal(L, type_[idx]);
+            add_scale(L);
+        }
+        std::vector<Term> lane;
+        if (!next) {
+            take([&](const Term& t) { return !(t.tmask & regset_); }, &lane);
+            take_mixed(~0u);
+            flush_table();
+            if (!lane.empty() || factored) emit_lane(lane, true, factored);
+            return;
+        }
+        // terms of one bit stay pending; terms of several are applied in the
+        // form they have if they would be mixed in the next stage
+        const uint32_t nreg = set_of(next->reg_bits, rb_);
+        auto mixed_next = [&](const Term& t) { return (t.tmask & nreg) && ((t.tmask & ~nreg) || t.bmask); };
+        std::vector<Term> now;
+        take([&](const Term& t) { return reg_only(t) && mixed_next(t); }, &now);
+        for (auto& t : now) table_add(t);
+        if (tactive_) flush_table();
+        bool need = false;
+        for (auto& t : pend_) need = need || (!(t.tmask & regset_) && mixed_next(t));
+        if (need) {
+            take([&](const Term& t) { return !(t.tmask & regset_); }, &lane);
+            emit_lane(lane, false, false);
+        }
+    }
+
+private:
+    struct Term {
+        uint32_t tmask, tval;   // tile bits
+        uint32_t bmask, bval;   // block bits
+        std::complex<double> f;
+        bool konst, real;
+        int gates;              // factors multiplied into f
+    };
+
+    // a gate's factor as one float: what the gate alone would multiply by
+    std::complex<double> rounded(const std::complex<double>& f) const
+    {
+        return precise_ ? std::complex<double>((float)f.real(), (float)f.imag()) : f;
+    }
+
+    static uint32_t set_of(const uint32_t* bits, int n)
+    {
+        uint32_t s = 0;
+        for (int i = 0; i < n; i++) s |= 1u << bits[i];
+        return s;
+    }
+    static bool const_type(int type)
+    {
+        switch (type) {
+        case HQ_CCX: case HQ_CNOT: case HQ_CY: case HQ_CZ: case HQ_H: case HQ_X: case HQ_Y: case HQ_Z:
+        case HQ_S: case HQ_SDG: case HQ_T: case HQ_TDG: case HQ_ID: case HQ_GII: case HQ_GZZ:
+            return true;
+        default:
+            return false;
+        }
+    }
+    bool reg_only(const Term& t) const { return !t.bmask && !(t.tmask & ~regset_) && t.tmask; }
+
+    // masks of tile bits over the stage's register / thread index
+    uint32_t to_reg(uint32_t tile) const
+    {
+        uint32_t r = 0;
+        for (int b = 0; b < SHM_MAX_TILE; b++)
+            if (((tile >> b) & 1) && reg_[b] >= 0) r |= 1u << reg_[b];
+        return r;
+    }
+    uint32_t to_thr(uint32_t tile) const
+    {
+        uint32_t r = 0;
+        for (int b = 0; b < SHM_MAX_TILE; b++)
+            if (((tile >> b) & 1) && thr_[b] >= 0) r |= 1u << thr_[b];
+        return r;
+    }
+
+    template <typename Pred>
+    void take(Pred pred, std::vector<Term>* out)
+    {
+        std::vector<Term> keep;
+        for (auto& t : pend_) (pred(t) ? *out : keep).push_back(t);
+        pend_.swap(keep);
+    }
+
+    void diagonal(const Lowered& L, int type)
+    {
+        for (int v = 0; v < 2; v++) {
+            const std::complex<double> f(v ? L.m[6] : L.m[0], v ? L.m[7] : L.m[1]);
+            // the |0> half of a phase is 1 by the gate's form
+            if (!v && L.cls == SHM_PHASE) continue;
+            Term t{0, 0, 0, 0, rounded(f), const_type(type), type == HQ_Z || type == HQ_CZ, 1};
+            if (L.t_tile >= 0) { t.tmask |= 1u << L.t_tile; t.tval |= (uint32_t)v << L.t_tile; }
+            else { t.bmask |= 1u << L.t_block; t.bval |= (uint32_t)v << L.t_block; }
+            for (int c = 0; c < 2; c++) {
+                if (L.c_tile[c] >= 0) { t.tmask |= 1u << L.c_tile[c]; t.tval |= 1u << L.c_tile[c]; }
+                if (L.c_block[c] >= 0) { t.bmask |= 1u << L.c_block[c]; t.bval |= 1u << L.c_block[c]; }
+            }
+            if (!merge_) {
+                push_mix(t);
+                continue;
+            }
+            bool merged = false;
+            for (auto& p : pend_) {
+                if (precise_) break;   // a product would be rounded once more
+                if (p.tmask != t.tmask || p.tval != t.tval || p.bmask != t.bmask || p.bval != t.bval) continue;
+                p.f *= t.f;
+                p.gates++;
+                p.konst = p.konst && t.konst;
+                p.real = p.real && t.real;
+                merged = true;
+                break;
+            }
+            if (!merged) pend_.push_back(t);
+        }
+    }
+
+    void mixing(const Lowered& L, int type)
+    {
+        const uint32_t pbit = 1u << L.t_tile;
+        const int P = reg_[L.t_tile];
+        uint32_t ct = 0, cb = 0;
+        for (int c = 0; c < 2; c++) {
+            if (L.c_tile[c] >= 0) ct |= 1u << L.c_tile[c];
+            if (L.c_block[c] >= 0) cb |= 1u << L.c_block[c];
+        }
+        ShmOp o;
+        o.cls = (uint8_t)L.cls;
+        o.tpos = (uint8_t)P;
+        o.creg = o.cregv = (uint8_t)to_reg(ct);
+        o.cthr = o.cthrv = (uint16_t)to_thr(ct);
+        o.cblk = o.cblkv = cb;
+        memcpy(o.m, L.m, sizeof(o.m));
+        // a thread-bit control makes the op the identity on some lanes: Y
+        // takes an update form whose coefficients can express the identity
+        if (o.cthr && o.cls == SHM_Y) o.cls = SHM_RX;
+        if (const_type(type)) o.flags |= SHM_FLAG_CONST;
+        const bool perm = L.cls == SHM_SWAP && !o.cthr && !cb;
+        if (perm && !ct) {
+            // X: the value a term asks of this bit flips
+            for (auto& t : pend_) t.tval ^= t.tmask & pbit;
+        } else {
+            take_mixed(pbit);
+            std::vector<Term> now;
+            if (perm) {
+                take([&](const Term& t) { return (t.tmask & pbit) != 0; }, &now);
+                for (auto& t : now) table_add(t);
+            } else {
+                bool need = tactive_ && ((tdep_ >> P) & 1);
+                for (auto& t : pend_) need = need || (t.tmask & pbit);
+                if (need) flush_table();
+            }
+        }
+        if (perm && tactive_) {
+            for (int j = 0; j < nr_; j++) {
+                if ((j >> P) & 1 || (j & o.creg) != o.creg) continue;
+                std::swap(table_[j], table_[j | (1 << P)]);
+                std::swap(used_[j], used_[j | (1 << P)]);
+            }
+            if ((tdep_ >> P) & 1) tdep_ |= o.creg;
+        }
+        ops_->push_back(o);
+    }
+
+    // applies the mixed terms on any of `bits` now
+    void take_mixed(uint32_t bits)
+    {
+        std::vector<Term> now;
+        take([&](const Term& t) { return (t.tmask & bits) && (t.tmask & regset_) && !reg_only(t); }, &now);
+        for (auto& t : now) push_mix(t);
+    }
+    void push_mix(const Term& t)
+    {
+        ShmOp o;
+        o.cls = SHM_MIX;
+        o.creg = (uint8_t)to_reg(t.tmask);
+        o.cregv = (uint8_t)to_reg(t.tval);
+        lane_cond(t, &o);
+        ops_->push_back(o);
+    }
+
+    void lane_cond(const Term& t, ShmOp* o) const
+    {
+        o->cthr = (uint16_t)to_thr(t.tmask);
+        o->cthrv = (uint16_t)to_thr(t.tval);
+        o->cblk = t.bmask;
+        o->cblkv = t.bval;
+        o->m[0] = t.f.real();
+        o->m[1] = t.real ? 0.0 : t.f.imag();
+        if (t.konst) o->flags |= SHM_FLAG_CONST;
+        if (t.real) o->flags |= SHM_FLAG_REAL;
+    }
+
+    void reset_table()
+    {
+        table_.assign(nr_, 1.0);
+        used_.assign(nr_, 0);
+        tdep_ = 0;
+        tactive_ = false;
+    }
+    void table_add(const Term& t)
+    {
+        const uint32_t m = to_reg(t.tmask), v = to_reg(t.tval);
+        for (int j = 0; j < nr_; j++)
+            if ((j & m) == v) { table_[j] *= t.f; used_[j] += t.real ? 0x100 : t.gates; }
+        tdep_ |= m;
+        tactive_ = true;
+    }
+    // applies the table, every pending term on register bits alone with it
+    void flush_table()
+    {
+        std::vector<Term> now;
+        take([&](const Term& t) { return reg_only(t); }, &now);
+        for (auto& t : now) table_add(t);
+        if (!tactive_) return;
+        ShmOp o;
+        o.cls = SHM_TAB;
+        o.tab = (uint32_t)(tabs_->size() / 2);
+        o.jdep = tdep_;
+        for (int j = 0; j < nr_; j++) {
+            if (used_[j]) o.jmask |= 1ull << j;
+            if (precise_ && (used_[j] & 0xff) > 1) o.jprod |= 1ull << j;
+            tabs_->push_back(table_[j].real());
+            tabs_->push_back(table_[j].imag());
+        }
+        ops_->push_back(o);
+        reset_table();
+    }
+
+    void emit_lane(const std::vector<Term>& lane, bool scale, bool factored)
+    {
+        bool real = true;
+        for (auto& t : lane) {
+            ShmOp o;
+            o.cls = SHM_LANE;
+            lane_cond(t, &o);
+            ops_->push_back(o);
+            real = real && t.real;
+        }
+        push_scale(scale && factored, lane.empty(), real);
+    }
+    void push_scale(bool scale, bool nolane, bool real)
+    {
+        ShmOp o;
+        o.cls = SHM_LANEMUL;
+        o.m[0] = 1.0;
+        if (nolane) o.flags |= SHM_FLAG_NOLANE;
+        if (scale) {
+            const std::complex<double> f = rounded(scale_);
+            o.m[0] = f.real();
+            o.m[1] = f.imag();
+            scale_ = 1.0;
+            logs_ = 0.0;
+        } else {
+            o.flags |= SHM_FLAG_UNIT;
+            if (real) o.flags |= SHM_FLAG_REAL;
+        }
+        // nothing to multiply by: unless same-structure groups share the code
+        if (nolane && !shared_ && o.m[0] == 1.0 && o.m[1] == 0.0) return;
+        ops_->push_back(o);
+    }
+    // The amplitudes grow by 1 / |scale| until the scale is applied: a group of
+    // hundreds of factored gates would leave float's range, so the scale is
+    // also applied whenever that growth reaches 2^48 (2^480 in double).  Shared
+    // code counts what the gates' types alone imply: 2^(1/2) per H.
+    void add_scale(const Lowered& L)
+    {
+        if (L.scale == std::complex<double>(1.0, 0.0)) return;
+        scale_ *= L.scale;
+        logs_ += shared_ ? (L.cls == SHM_HADD ? -0.5 : 0.0) : std::log2(std::abs(L.scale));
+        if (std::fabs(logs_) >= limit_) push_scale(true, true, false);
+    }
+
+    const std::vector<Lowered>& low_;
+    const std::vector<int>& type_;
+    const int rb_, tb_, nr_;
+    const bool shared_, precise_, merge_;
+    const double limit_;
+    std::vector<Term> pend_;
+    std::vector<ShmOp>* ops_ = nullptr;
+    std::vector<double>* tabs_ = nullptr;
+    uint32_t regset_ = 0;
+    int reg_[SHM_MAX_TILE], thr_[SHM_MAX_TILE];
+    std::vector<std::complex<double>> table_;
+    std::vector<int> used_;     // gates in each entry (signs count 0x100 each)
+    uint32_t tdep_ = 0;
+    bool tactive_ = false;
+    std::complex<double> scale_{1.0, 0.0};
+    double logs_ = 0.0;
+};
+
 }  // namespace
 
 hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gates, uint64_t shared_mask, int rb_req,
-                        ShmPlan* plan, bool init, int io, bool shared_code)
+                        ShmPlan* plan, bool init, int io, bool shared_code, bool merge)
 {
     HQ_CHECK(num_gates >= 0 && (num_gates == 0 || gates), HQ_ERR_ARG, "sharemem: bad gate array");
     const size_t amp_bytes = precision == HQ_C128 ? 16 : 8;
@@ -236,9 +564,8 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
     std::vector<int> low_type;
     low.reserve(num_gates);
     // uncontrolled H, RX, RY and unit diagonals lose a scalar factor; the
-    // product S is applied once at the end of the pass (HQ_SHM_FACTOR=0: off)
+    // factors' product is applied at the end of the pass (HQ_SHM_FACTOR=0: off)
     static const bool factor = !getenv("HQ_SHM_FACTOR") || atoi(getenv("HQ_SHM_FACTOR")) != 0;
-    std::complex<double> S(1.0, 0.0);
     bool factored = false;
     for (int i = 0; i < num_gates; i++) {
         const hq_gate& g = gates[i];
@@ -260,7 +587,7 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
             L.c_block[c] = cs[c] >= 0 ? block_of[cs[c]] : -1;
         }
         memcpy(L.m, g.mat, sizeof(L.m));
-        if (factor && g.control < 0 && g.control2 < 0 && factor_scalar(L, &S, shared_code)) factored = true;
+        if (factor && g.control < 0 && g.control2 < 0 && factor_scalar(L, &L.scale, shared_code)) factored = true;
         low.push_back(L);
         low_type.push_back(g.type);
     }
@@ -371,62 +698,25 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
     if ((io & 1) && !init && short_runs(stages.front())) stages.insert(stages.begin(), make_io(stages.front()));
     if ((io & 2) && short_runs(stages.back())) stages.push_back(make_io(stages.back()));
 
-    // serialize
-    std::vector<ShmOp> ops;
+    // lower the stages' gates to ops, diagonal gates merged (StageLowering)
     std::vector<ShmStage> dst;
+    // batched kernels return sums over a circuit's qubits, which the one-float
+    // form serves, and are bound by the operations it saves
+    const bool precise = precision == HQ_C64 && !shared_code;
+    StageLowering lo(low, low_type, precision, rb, tb, shared_code, precise, merge);
     for (auto& S : stages) {
         ShmStage d;
         memset(&d, 0, sizeof(d));
-        int reg_index[SHM_MAX_TILE], thr_index[SHM_MAX_TILE];
-        for (int i = 0; i < SHM_MAX_TILE; i++) reg_index[i] = thr_index[i] = -1;
-        for (int i = 0; i < rb; i++) { d.reg_bits[i] = S.reg_bits[i]; reg_index[S.reg_bits[i]] = i; }
-        for (int i = 0; i < tb; i++) { d.thr_bits[i] = S.thr_bits[i]; thr_index[S.thr_bits[i]] = i; }
-        d.op_begin = (uint32_t)ops.size();
-        for (int idx : S.ops) {
-            const Lowered& L = low[idx];
-            ShmOp o;
-            memset(&o, 0, sizeof(o));
-            o.cls = (uint8_t)L.cls;
-            if (L.t_tile >= 0 && reg_index[L.t_tile] >= 0) { o.where = SHM_IN_REG; o.tpos = (uint8_t)reg_index[L.t_tile]; }
-            else if (L.t_tile >= 0) { o.where = SHM_IN_THREAD; o.tpos = (uint8_t)thr_index[L.t_tile]; }
-            else { o.where = SHM_IN_BLOCK; o.tpos = (uint8_t)L.t_block; }
-            for (int c = 0; c < 2; c++) {
-                if (L.c_tile[c] >= 0) {
-                    if (reg_index[L.c_tile[c]] >= 0) o.creg |= 1u << reg_index[L.c_tile[c]];
-                    else o.cthr |= 1u << thr_index[L.c_tile[c]];
-                } else if (L.c_block[c] >= 0) {
-                    o.cblk |= 1ull << L.c_block[c];
-                }
-            }
-            memcpy(o.m, L.m, sizeof(o.m));
-            // a thread-bit control makes the op the identity on some lanes:
-            // use an update form that can express the identity
-            if (o.cthr && o.cls == SHM_SWAP) o.cls = SHM_REAL;
-            if (o.cthr && o.cls == SHM_Y) o.cls = SHM_RX;
-            switch (low_type[idx]) {
-            case HQ_CCX: case HQ_CNOT: case HQ_CY: case HQ_CZ: case HQ_H: case HQ_X: case HQ_Y: case HQ_Z:
-            case HQ_S: case HQ_SDG: case HQ_T: case HQ_TDG: case HQ_ID: case HQ_GII: case HQ_GZZ:
-                o.flags |= SHM_FLAG_CONST;
-                break;
-            default:
-                break;
-            }
-            ops.push_back(o);
-        }
-        d.op_end = (uint32_t)ops.size();
+        for (int i = 0; i < rb; i++) d.reg_bits[i] = S.reg_bits[i];
+        for (int i = 0; i < tb; i++) d.thr_bits[i] = S.thr_bits[i];
         dst.push_back(d);
     }
-    // shared code: the scale op whenever a gate was factored (a structural
-    // fact), even where the angles make the product exactly 1
-    if (S != std::complex<double>(1.0, 0.0) || (shared_code && factored)) {
-        ShmOp o;
-        memset(&o, 0, sizeof(o));
-        o.cls = SHM_SCALE;
-        o.where = SHM_IN_REG;
-        o.m[0] = S.real();
-        o.m[1] = S.imag();
-        ops.push_back(o);
-        dst.back().op_end = (uint32_t)ops.size();
+    std::vector<ShmOp> ops;
+    std::vector<double> tabs;
+    for (size_t s = 0; s < dst.size(); s++) {
+        dst[s].op_begin = (uint32_t)ops.size();
+        lo.stage(dst[s], s + 1 < dst.size() ? &dst[s + 1] : nullptr, stages[s].ops, factored, &ops, &tabs);
+        dst[s].op_end = (uint32_t)ops.size();
     }
 
     ShmHeader hdr;
@@ -435,7 +725,8 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
     for (int i = 0; i < k; i++) { hdr.tile_phys[i] = 1ull << tile_pos[i]; hdr.swz_col[i] = swz_column(i); }
     hdr.num_block_bits = (uint32_t)block_pos.size();
     hdr.num_stages = (uint32_t)dst.size();
-    hdr.num_ops = (uint32_t)ops.size();
+    // lowered gates, plus the final scale when a gate was factored
+    hdr.num_ops = (uint32_t)(low.size() + (factored ? 1 : 0));
 
     plan->n = n;
     plan->precision = precision;
@@ -446,11 +737,200 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
     plan->hdr = hdr;
     plan->stages = std::move(dst);
     plan->ops = std::move(ops);
+    plan->tabs = std::move(tabs);
+    plan->precise = precise;
     return HQ_OK;
 }
 
+// ---- the interpreter's program ------------------------------------------------------------
+
+namespace {
+
+template <typename R>
+struct Encoder {
+    const ShmPlan& P;
+    std::vector<char> slots;
+    std::vector<Factor<R>> lanes;   // 2^tb entries per lane table
+    static constexpr int SLOT = shm_slot_bytes<R>();
+    static_assert(SHM_WINDOW_BYTES % SLOT == 0, "windows hold whole slots");
+
+    size_t count() const { return slots.size() / SLOT; }
+
+    // room for `need` consecutive slots before the window's last one, which
+    // is kept for the refill
+    void room(size_t need)
+    {
+        const size_t W = (size_t)shm_window_slots<R>();
+        if (count() % W + need <= W - 1) return;
+        ShmSlot none{};
+        none.kind = SLOT_END;       // never reached: a refill comes first
+        ShmSlot refill{};
+        refill.kind = SLOT_REFILL;
+        put(refill, nullptr, 0);
+        while (count() % W) put(none, nullptr, 0);
+    }
+    void put(const ShmSlot& h, const void* payload, size_t bytes)
+    {
+        const size_t at = slots.size();
+        slots.resize(at + SLOT, 0);
+        memcpy(slots.data() + at, &h, sizeof(h));
+        if (bytes) memcpy(slots.data() + at + sizeof(h), payload, bytes);
+    }
+    void op(const ShmSlot& h, const double* m, int nm)
+    {
+        R c[8] = {};
+        for (int i = 0; i < nm; i++) c[i] = (R)m[i];
+        room(1);
+        put(h, c, sizeof(c));
+    }
+    static ShmSlot head(const ShmOp& o, int kind)
+    {
+        ShmSlot h{};
+        h.kind = (uint8_t)kind;
+        h.aux = o.tpos;
+        h.creg = o.creg; h.cregv = o.cregv;
+        h.cthr = o.cthr; h.cthrv = o.cthrv;
+        h.cblk = o.cblk; h.cblkv = o.cblkv;
+        return h;
+    }
+
+    ShmXchg xchg(const ShmStage& st) const
+    {
+        ShmXchg x{};
+        auto swz = [&](uint32_t bit) { return (uint16_t)(bit < 3 ? 1u << bit : (1u << bit) ^ P.hdr.swz_col[bit]); };
+        for (int i = 0; i < P.tb; i++) x.thr[i] = swz(st.thr_bits[i]);
+        for (int i = 0; i < P.rb; i++) x.reg[i] = swz(st.reg_bits[i]);
+        return x;
+    }
+
+    void stage(const ShmStage& st)
+    {
+        // the lane factor of the stage: what depends on the thread bits alone
+        // (and the scale) as a table, loaded before the stage's ops
+        const int NT = 1 << P.tb;
+        bool table = false;
+        std::vector<std::complex<double>> f;
+        const ShmOp* mul = nullptr;
+        for (uint32_t i = st.op_begin; i < st.op_end; i++) {
+            const ShmOp& o = P.ops[i];
+            if (o.cls == SHM_LANEMUL && !(o.flags & SHM_FLAG_NOLANE)) mul = &o;
+            if (o.cls != SHM_LANE || o.cblk) continue;
+            if (!table) { f.assign(NT, 1.0); table = true; }
+            for (int t = 0; t < NT; t++)
+                if ((t & o.cthr) == o.cthrv) f[t] *= std::complex<double>(o.m[0], o.m[1]);
+        }
+        if (table) {
+            const std::complex<double> S(mul->m[0], mul->m[1]);
+            ShmSlot h{};
+            h.kind = SLOT_LANETAB;
+            h.cblk = (uint32_t)(lanes.size() / NT);
+            for (int t = 0; t < NT; t++) {
+                const std::complex<double> v = f[t] * S;
+                lanes.push_back(Factor<R>::of(v.real(), v.imag()));
+            }
+            op(h, nullptr, 0);
+        }
+        for (uint32_t i = st.op_begin; i < st.op_end; i++) {
+            const ShmOp& o = P.ops[i];
+            switch (o.cls) {
+            case SHM_TAB: {
+                const size_t bytes = ((size_t)1 << P.rb) * sizeof(Factor<R>);
+                const size_t more = (bytes + SLOT - 1) / SLOT;
+                std::vector<Factor<R>> t((size_t)1 << P.rb);
+                for (size_t j = 0; j < t.size(); j++)
+                    t[j] = Factor<R>::of(P.tabs[2 * (o.tab + j)], P.tabs[2 * (o.tab + j) + 1]);
+                ShmSlot h{};
+                // per-index branches pay when at least half of the indices keep their amplitude
+                const bool mask = 2 * __builtin_popcountll(o.jmask) <= (1 << P.rb);
+                h.kind = mask ? SLOT_TABMASK : SLOT_TAB;
+                h.aux = (uint8_t)more;
+                if (mask) { h.cblk = (uint32_t)o.jmask; h.cblkv = (uint32_t)(o.jmask >> 32); }
+                room(1 + more);
+                put(h, nullptr, 0);
+                const size_t at = slots.size();
+                slots.resize(at + more * SLOT, 0);
+                memcpy(slots.data() + at, t.data(), bytes);
+                break;
+            }
+            case SHM_MIX:
+                op(head(o, (o.flags & SHM_FLAG_REAL) && o.m[0] == -1.0 ? SLOT_MIXSIGN : SLOT_MIX), o.m, 2);
+                break;
+            case SHM_LANE:
+                if (o.cblk) op(head(o, SLOT_LANE), o.m, 2);
+                break;
+            case SHM_LANEMUL:
+                if (o.flags & SHM_FLAG_NOLANE) {
+                    op(head(o, SLOT_SCALE), o.m, 2);
+                } else {
+                    if (!table && !(o.flags & SHM_FLAG_UNIT)) op(head(o, SLOT_LANE), o.m, 2);
+                    op(head(o, SLOT_LANEMUL), nullptr, 0);
+                }
+                break;
+            case SHM_SWAP:
+                op(head(o, o.cthr ? (int)SLOT_CSWAP : (int)SHM_SWAP), nullptr, 0);
+                break;
+            default:
+                op(head(o, o.cls), o.m, 8);
+                break;
+            }
+        }
+    }
+
+    std::vector<char> run()
+    {
+        ShmProg H{};
+        for (size_t s = 0; s < P.stages.size(); s++) {
+            if (s > 0) {
+                ShmSlot h{};
+                h.kind = SLOT_XCHG;
+                const ShmXchg x = xchg(P.stages[s]);
+                room(1);
+                put(h, &x, sizeof(x));
+            }
+            stage(P.stages[s]);
+        }
+        ShmSlot end{};
+        end.kind = SLOT_END;
+        room(1);
+        put(end, nullptr, 0);
+        // runs of consecutive block positions
+        const uint32_t nb = P.hdr.num_block_bits;
+        for (uint32_t j = 0; j < nb;) {
+            const int p = __builtin_ctzll(P.hdr.block_phys[j]);
+            uint32_t len = 1;
+            while (j + len < nb && __builtin_ctzll(P.hdr.block_phys[j + len]) == p + (int)len) len++;
+            H.run[H.num_runs++] = ShmRun{j, (uint32_t)p, (1ull << len) - 1};
+            j += len;
+        }
+        H.num_slots = (uint32_t)count();
+        H.zero_mask = P.hdr.zero_mask;
+        auto pos = [&](uint32_t tile) { return (uint8_t)__builtin_ctzll(P.hdr.tile_phys[tile]); };
+        const ShmStage &f = P.stages.front(), &l = P.stages.back();
+        for (int i = 0; i < P.tb; i++) { H.ld_thr[i] = pos(f.thr_bits[i]); H.st_thr[i] = pos(l.thr_bits[i]); }
+        for (int i = 0; i < P.rb; i++) { H.ld_reg[i] = pos(f.reg_bits[i]); H.st_reg[i] = pos(l.reg_bits[i]); }
+        H.first = xchg(f);
+        // the last window is copied whole
+        const size_t tail = slots.size() - slots.size() % (size_t)SHM_WINDOW_BYTES + SHM_WINDOW_COPY;
+        const size_t lane_off = (SHM_PROG_HEADER + tail + 255) & ~(size_t)255;
+        H.lane_off = (uint32_t)lane_off;
+        std::vector<char> out(lane_off + lanes.size() * sizeof(Factor<R>), 0);
+        memcpy(out.data(), &H, sizeof(H));
+        memcpy(out.data() + SHM_PROG_HEADER, slots.data(), slots.size());
+        if (!lanes.empty()) memcpy(out.data() + lane_off, lanes.data(), lanes.size() * sizeof(Factor<R>));
+        return out;
+    }
+};
+
+}  // namespace
+
+std::vector<char> encode_program(const ShmPlan& plan)
+{
+    if (plan.precision == HQ_C128) return Encoder<double>{plan, {}, {}}.run();
+    return Encoder<float>{plan, {}, {}}.run();
+}
+
 hq_status build_sharemem_program(hq_state s, const hq_gate* gates, int num_gates, uint64_t shared_mask, int rb_req,
-                                 hq_program* out, bool init, int variant, uint64_t zero_mask)
+                                 hq_program* out, bool init, int variant, uint64_t zero_mask, bool merge)
 {
     HQ_CHECK(s && out, HQ_ERR_ARG, "sharemem: null argument");
     *out = nullptr;
@@ -459,21 +939,15 @@ hq_status build_sharemem_program(hq_state s, const hq_gate* gates, int num_gates
     // non-temporal loads
     const bool whole_line = variant & 1;
     hq_status st = plan_sharemem(s->n, s->precision, gates, num_gates, shared_mask, rb_req, &plan, init,
-                                 whole_line ? 3 : 0);
+                                 whole_line ? 3 : 0, false, merge);
     if (st != HQ_OK) return st;
     plan.init = init;
     plan.whole_line = whole_line;
     plan.nt_store = (variant & 2) != 0;
     plan.nt_load = (variant & 4) != 0;
     plan.hdr.zero_mask = init ? 0 : zero_mask;
-    const auto& dst = plan.stages;
-    const auto& ops = plan.ops;
-    size_t bytes = sizeof(ShmHeader) + dst.size() * sizeof(ShmStage) + ops.size() * sizeof(ShmOp);
-    std::vector<char> blob(bytes);
-    memcpy(blob.data(), &plan.hdr, sizeof(ShmHeader));
-    memcpy(blob.data() + sizeof(ShmHeader), dst.data(), dst.size() * sizeof(ShmStage));
-    if (!ops.empty())
-        memcpy(blob.data() + sizeof(ShmHeader) + dst.size() * sizeof(ShmStage), ops.data(), ops.size() * sizeof(ShmOp));
+    const std::vector<char> blob = encode_program(plan);
+    const size_t bytes = blob.size();
 
     hq_program p = new hq_program_s();
     p->kind = 1;
@@ -482,8 +956,8 @@ hq_status build_sharemem_program(hq_state s, const hq_gate* gates, int num_gates
     p->tile = plan.k;
     p->rb = plan.rb;
     p->tb = plan.tb;
-    p->num_stages = (int)dst.size();
-    p->num_ops = (int)ops.size();
+    p->num_stages = (int)plan.stages.size();
+    p->num_ops = (int)plan.hdr.num_ops;
     p->shared_mask = shared_mask;
     p->prog_bytes = bytes;
     p->plan = new ShmPlan(std::move(plan));

@@ -44,94 +44,59 @@ __device__ __forceinline__ void reg_pairs(cplx<R> (&a)[1 << RB], uint32_t creg, 
         }
         return;
     }
+    // the factored forms come from uncontrolled gates only
+    if constexpr (CLS < SHM_HADD) {
+#pragma unroll
+        for (int j = 0; j < (1 << RB); j++) {
+            if (j & (1 << P)) continue;
+            if ((j & creg) != creg) continue;
+            pair_update<CLS, R>(a[j], a[j | (1 << P)], m);
+        }
+    }
+}
+
+// X where the lane's thread-bit controls are set: selects, no arithmetic
+template <typename R, int RB, int P>
+__device__ __forceinline__ void lane_swap(cplx<R> (&a)[1 << RB], uint32_t creg, bool on)
+{
 #pragma unroll
     for (int j = 0; j < (1 << RB); j++) {
         if (j & (1 << P)) continue;
         if ((j & creg) != creg) continue;
-        pair_update<CLS, R>(a[j], a[j | (1 << P)], m);
+        const cplx<R> lo = a[j], hi = a[j | (1 << P)];
+        a[j].x = on ? hi.x : lo.x;
+        a[j].y = on ? hi.y : lo.y;
+        a[j | (1 << P)].x = on ? lo.x : hi.x;
+        a[j | (1 << P)].y = on ? lo.y : hi.y;
     }
 }
 
 template <typename R, int RB, int P>
-__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int cls, uint32_t creg, const R* m)
+__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool on, const R* m)
 {
-    switch (cls) {
+    switch (kind) {
     case SHM_SWAP: reg_pairs<R, RB, SHM_SWAP, P>(a, creg, m); break;
     case SHM_Y: reg_pairs<R, RB, SHM_Y, P>(a, creg, m); break;
     case SHM_REAL: reg_pairs<R, RB, SHM_REAL, P>(a, creg, m); break;
     case SHM_RX: reg_pairs<R, RB, SHM_RX, P>(a, creg, m); break;
     case SHM_GEN: reg_pairs<R, RB, SHM_GEN, P>(a, creg, m); break;
-    case SHM_DIAG: reg_pairs<R, RB, SHM_DIAG, P>(a, creg, m); break;
     case SHM_HADD: reg_pairs<R, RB, SHM_HADD, P>(a, creg, m); break;
     case SHM_ROTA: reg_pairs<R, RB, SHM_ROTA, P>(a, creg, m); break;
     case SHM_ROTB: reg_pairs<R, RB, SHM_ROTB, P>(a, creg, m); break;
     case SHM_RXA: reg_pairs<R, RB, SHM_RXA, P>(a, creg, m); break;
     case SHM_RXB: reg_pairs<R, RB, SHM_RXB, P>(a, creg, m); break;
-    default: reg_pairs<R, RB, SHM_PHASE, P>(a, creg, m); break;
+    default: lane_swap<R, RB, P>(a, creg, on); break;
     }
 }
 
-template <typename R, int RB>
-__device__ __forceinline__ void apply_op(cplx<R> (&a)[1 << RB], const HQ_GLOBAL ShmOp* __restrict__ op, uint32_t tid,
-                                         uint64_t blk)
-{
-    // Every branch below is uniform over the block (the op fields and the
-    // block index are): a lane whose thread-bit controls are not all set gets
-    // the identity's coefficients instead of leaving the op, so no branch
-    // depends on the lane (a per-lane exit made every later dispatch a
-    // divergent branch).  Thread-controlled ops only use classes that can
-    // express the identity (the planner turns SWAP into REAL and Y into RX).
-    const uint64_t cblk = op->cblk;
-    if ((blk & cblk) != cblk) return;                 // block control not set (uniform)
-    const uint32_t cthr = op->cthr;
-    const bool on = (tid & cthr) == cthr;
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+// a slot as it sits in LDS
+template <typename R>
+struct alignas(16) SlotRegs {
+    uint4 h;
     R m[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const R id = (i == 0 || i == 6) ? R(1) : R(0);
-        const R v = (R)op->m[i];
-        m[i] = on ? v : id;
-    }
-    const uint32_t creg = op->creg;
-    const int cls = op->cls;
-    const int tpos = op->tpos;
-    if (cls == SHM_SCALE) {
-#pragma unroll
-        for (int j = 0; j < (1 << RB); j++) scale(a[j], m[0], m[1]);
-        return;
-    }
-    if (op->where == SHM_IN_REG) {
-        switch (tpos) {
-        case 0: reg_op<R, RB, 0>(a, cls, creg, m); break;
-        case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, cls, creg, m); break;
-        case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, cls, creg, m); break;
-        case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, cls, creg, m); break;
-        case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, cls, creg, m); break;
-        default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, cls, creg, m); break;
-        }
-        static_assert(RB <= 6, "register positions above 5 are not dispatched");
-        return;
-    }
-    // diagonal gate whose target is a thread bit or a block bit: one factor
-    // per lane for every register amplitude (a phase leaves the |0> half alone)
-    const uint32_t hb = op->where == SHM_IN_THREAD ? (tid >> tpos) & 1u : (uint32_t)((blk >> tpos) & 1u);
-    const R fr = hb ? m[6] : (cls == SHM_PHASE ? R(1) : m[0]);
-    const R fi = hb ? m[7] : (cls == SHM_PHASE ? R(0) : m[1]);
-#pragma unroll
-    for (int j = 0; j < (1 << RB); j++) {
-        if ((j & creg) != creg) continue;
-        scale(a[j], fr, fi);
-    }
-}
-
-template <int K>
-__device__ __forceinline__ uint32_t swz(uint32_t x, const uint32_t* __restrict__ col)
-{
-    uint32_t f = 0;
-#pragma unroll
-    for (int i = 3; i < K; i++) f ^= ((x >> i) & 1u) ? col[i] : 0u;
-    return x ^ f;
-}
+};
 
 // Z-sum and nearest-neighbour ZZ-sum eigenvalues of basis state idx over n qubits:
 // sum_q (1 - 2 b_q) and sum_{q<n-1} (1 - 2 (b_q xor b_{q+1})).
@@ -145,56 +110,70 @@ __device__ __forceinline__ void zsums(uint64_t idx, int n, double* z, double* zz
 
 // One OShareMem pass of tile `blk` of the group program `prog` over `psi`.
 // `mode` is uniform over the grid; the single-state kernel passes 0.
+//
+// The program is a list of slots executed in order.  A pass over a small state
+// is a chain of ops run by one wave per SIMD, so what an op costs is its fetch
+// and dispatch: read from HBM through the scalar cache, each op's fields were
+// three dependent misses.  Slots are copied to
+// LDS a window at a time, together with the tile's loads, and the next slot is
+// read while one executes.  With diagonal gates merged on top, passes of the
+// 17-qubit complex64 and 20-qubit complex128 random circuits (32 and 256
+// blocks) went from 61 and 67.5 us to 37 and 38 us, the 174 gates of a
+// 10-qubit ansatz (one wave) from 132 to 51 us.
 template <typename R, int RB, int TB>
 __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const char* __restrict__ prog_any,
-                                          uint64_t blk, cplx<R>* __restrict__ lds, uint32_t mode, int n,
-                                          double* __restrict__ part_any)
+                                          uint64_t blk, cplx<R>* __restrict__ lds, char* __restrict__ win,
+                                          uint32_t mode, int n, double* __restrict__ part_any)
 {
     HQ_GLOBAL cplx<R>* __restrict__ psi = to_global(psi_any);
     const HQ_GLOBAL char* __restrict__ prog = to_global(prog_any);
     HQ_GLOBAL double* __restrict__ part = to_global(part_any);
     constexpr int NR = 1 << RB;
-    constexpr int K = RB + TB;
+    constexpr int NT = 1 << TB;
+    constexpr int SLOT = shm_slot_bytes<R>();
 
-    const HQ_GLOBAL ShmHeader* __restrict__ H = (const HQ_GLOBAL ShmHeader*)prog;
-    const HQ_GLOBAL ShmStage* __restrict__ ST = (const HQ_GLOBAL ShmStage*)(prog + sizeof(ShmHeader));
-    const uint32_t nst = H->num_stages;
-    const HQ_GLOBAL ShmOp* __restrict__ OP =
-        (const HQ_GLOBAL ShmOp*)(prog + sizeof(ShmHeader) + nst * sizeof(ShmStage));
+    const HQ_GLOBAL ShmProg* __restrict__ H = (const HQ_GLOBAL ShmProg*)prog;
     const uint32_t tid = threadIdx.x;
 
-    // block base address: pdep(blk, block bits)
+    // block base address: the block index scattered to the block bits
     uint64_t base = 0;
-    const uint32_t nbb = H->num_block_bits;
-    for (uint32_t j = 0; j < nbb; j++)
-        if ((blk >> j) & 1) base |= H->block_phys[j];
+    const uint32_t nruns = H->num_runs;
+    for (uint32_t j = 0; j < nruns; j++) base |= ((blk >> H->run[j].src) & H->run[j].mask) << H->run[j].dst;
     // a tile known to be zero stays zero (uniform over the block)
     if (!(mode & TILE_READ) && (base & H->zero_mask)) return;
 
-    uint32_t col[K];
+    // a window of slots, global -> registers -> LDS, in pieces of 16 bytes a
+    // thread (every window is readable to SHM_WINDOW_COPY bytes).  No branch
+    // here or in the loop below depends on the lane: one that did would make
+    // the compiler rebuild the whole loop with copies of every amplitude at
+    // its joins (17 qubits complex64: 12 200 VALU instructions per wave and
+    // pass instead of 6 200).
+    const uint32_t nbytes = H->num_slots * SLOT;
+    constexpr int WIN_BYTES = shm_window_slots<R>() * SLOT;
+    constexpr int PIECES = SHM_WINDOW_COPY / (16 * NT);
+    const HQ_GLOBAL char* __restrict__ slots = prog + SHM_PROG_HEADER;
+    uint4 piece[PIECES];
+    auto fetch = [&](uint32_t from) {
 #pragma unroll
-    for (int i = 0; i < K; i++) col[i] = H->swz_col[i];
+        for (int i = 0; i < PIECES; i++)
+            if (from + (uint32_t)(i * NT) * 16u < nbytes)
+                piece[i] = *(const HQ_GLOBAL uint4*)(slots + from + (uint32_t)(i * NT + tid) * 16u);
+    };
+    auto fill = [&]() {
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) *(uint4*)(win + (uint32_t)(i * NT + tid) * 16u) = piece[i];
+    };
 
     cplx<R> a[NR];
-
-    // mapping of stage 0
-    uint32_t rbit[RB];
     uint64_t rphys[RB];
-#pragma unroll
-    for (int i = 0; i < RB; i++) {
-        rbit[i] = 1u << ST[0].reg_bits[i];
-        rphys[i] = H->tile_phys[ST[0].reg_bits[i]];
-    }
-    uint32_t et = 0;
-    uint64_t pt = 0;
-#pragma unroll
-    for (int i = 0; i < TB; i++) {
-        uint32_t b = ST[0].thr_bits[i];
-        if ((tid >> i) & 1) { et |= 1u << b; pt |= H->tile_phys[b]; }
-    }
     if (mode == TILE_INIT && base != 0) {
         // first pass of a run: a tile other than the origin's starts at zero
         // and stays zero under the group's linear gates
+        uint64_t pt = 0;
+#pragma unroll
+        for (int i = 0; i < TB; i++) pt |= (uint64_t)((tid >> i) & 1u) << H->st_thr[i];
+#pragma unroll
+        for (int i = 0; i < RB; i++) rphys[i] = (uint64_t)1 << H->st_reg[i];
         HQ_GLOBAL cplx<R>* __restrict__ dst = psi + (base | pt);
         cplx<R> z;
         z.x = R(0);
@@ -208,71 +187,191 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
         }
         return;
     }
-    if (mode & TILE_INIT) {
-        const bool origin = (base | pt) == 0;
+    // issued before the tile's loads, so that it can be stored while they are in flight
+    fetch(0);
+    {
+        uint64_t pt = 0;
 #pragma unroll
-        for (int j = 0; j < NR; j++) {
-            a[j].x = (origin && j == 0) ? R(1) : R(0);
-            a[j].y = R(0);
-        }
-    } else {
-        const HQ_GLOBAL cplx<R>* __restrict__ src = psi + (base | pt);
+        for (int i = 0; i < TB; i++) pt |= (uint64_t)((tid >> i) & 1u) << H->ld_thr[i];
+        if (mode & TILE_INIT) {
+            const bool origin = (base | pt) == 0;
 #pragma unroll
-        for (int j = 0; j < NR; j++) {
-            uint64_t off = 0;
+            for (int j = 0; j < NR; j++) {
+                a[j].x = (origin && j == 0) ? R(1) : R(0);
+                a[j].y = R(0);
+            }
+        } else {
 #pragma unroll
-            for (int i = 0; i < RB; i++) if ((j >> i) & 1) off |= rphys[i];
-            a[j] = src[off];
+            for (int i = 0; i < RB; i++) rphys[i] = (uint64_t)1 << H->ld_reg[i];
+            const HQ_GLOBAL cplx<R>* __restrict__ src = psi + (base | pt);
+#pragma unroll
+            for (int j = 0; j < NR; j++) {
+                uint64_t off = 0;
+#pragma unroll
+                for (int i = 0; i < RB; i++) if ((j >> i) & 1) off |= rphys[i];
+                a[j] = src[off];
+            }
         }
     }
-
-    for (uint32_t s = 0; s < nst; s++) {
-        if (s > 0) {
-            // exchange: write under the old mapping, read under the new one.
-            // The swizzle is linear over xor, so a register's LDS index is the
-            // lane's swizzled index xor the swizzled bits of the register index
-            const uint32_t st = swz<K>(et, col);
-            uint32_t srb[RB];
+    fill();
+    // LDS indices of the current stage
+    uint32_t at, reg_at[RB];
+    {
+        uint32_t r = 0;
 #pragma unroll
-            for (int i = 0; i < RB; i++) srb[i] = swz<K>(rbit[i], col);
+        for (int i = 0; i < TB; i++) r ^= (0u - ((tid >> i) & 1u)) & (uint32_t)H->first.thr[i];
+        at = r;
+#pragma unroll
+        for (int i = 0; i < RB; i++) reg_at[i] = H->first.reg[i];
+    }
+    __syncthreads();
+
+    double lx = 1, ly = 0;    // the lane's factor
+    uint32_t window = 0;      // bytes of the current window's start in the program
+    const char* pc = win;
+    SlotRegs<R> next = *(const SlotRegs<R>*)pc;
+    for (;;) {
+        const SlotRegs<R> s = next;
+        pc += SLOT;
+        next = *(const SlotRegs<R>*)pc;   // (behind the last slot of a window: unused)
+        const uint32_t w0 = uniform(s.h.x), w1 = uniform(s.h.y);
+        const uint32_t cb = uniform(s.h.z), cbv = uniform(s.h.w);
+        const int kind = (int)(w0 & 255u), aux = (int)((w0 >> 8) & 255u);
+        const uint32_t creg = (w0 >> 16) & 255u, cregv = w0 >> 24;
+        const uint32_t cthr = w1 & 0xffffu, cthrv = w1 >> 16;
+        const bool on = (tid & cthr) == cthrv;
+        // Every branch below is uniform over the block: a lane whose
+        // thread-bit condition does not hold gets the identity's coefficients
+        // or keeps its values by selects instead of leaving the op.
+        if (kind <= SLOT_CSWAP) {
+            if (((uint32_t)blk & cb) != cbv) continue;
+            R m[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) m[i] = s.m[i];
+            if (cthr) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) m[i] = on ? m[i] : (i == 0 || i == 6) ? R(1) : R(0);
+            }
+            switch (aux) {
+            case 0: reg_op<R, RB, 0>(a, kind, creg, on, m); break;
+            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, on, m); break;
+            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, on, m); break;
+            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, on, m); break;
+            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, on, m); break;
+            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, on, m); break;
+            }
+            static_assert(RB <= 6, "register positions above 5 are not dispatched");
+            continue;
+        }
+        if (kind == SLOT_XCHG) {
+            // write under the old split, read under the new one; a register's
+            // LDS index is the lane's xor its register bits' entries
+            auto entry = [&](int e) -> uint32_t {   // e-th 16-bit field of the ShmXchg in s.m
+                uint32_t w;
+                if constexpr (sizeof(R) == 4) w = __float_as_uint(s.m[e / 2]);
+                else w = (e & 2) ? (uint32_t)__double2hiint(s.m[e / 4]) : (uint32_t)__double2loint(s.m[e / 4]);
+                return (e & 1) ? w >> 16 : w & 0xffffu;
+            };
 #pragma unroll
             for (int j = 0; j < NR; j++) {
                 uint32_t so = 0;
 #pragma unroll
-                for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= srb[i];
-                lds[st ^ so] = a[j];
+                for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= reg_at[i];
+                lds[at ^ so] = a[j];
             }
+            at = 0;
+#pragma unroll
+            for (int i = 0; i < TB; i++) at ^= (0u - ((tid >> i) & 1u)) & entry(i);
+#pragma unroll
+            for (int i = 0; i < RB; i++) reg_at[i] = uniform(entry(SHM_MAX_TB + i));
             __syncthreads();
 #pragma unroll
-            for (int i = 0; i < RB; i++) rbit[i] = 1u << ST[s].reg_bits[i];
-            et = 0;
-#pragma unroll
-            for (int i = 0; i < TB; i++)
-                if ((tid >> i) & 1) et |= 1u << ST[s].thr_bits[i];
-            const uint32_t st2 = swz<K>(et, col);
-#pragma unroll
-            for (int i = 0; i < RB; i++) srb[i] = swz<K>(rbit[i], col);
-#pragma unroll
             for (int j = 0; j < NR; j++) {
                 uint32_t so = 0;
 #pragma unroll
-                for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= srb[i];
-                a[j] = lds[st2 ^ so];
+                for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= reg_at[i];
+                a[j] = lds[at ^ so];
             }
             // the next exchange overwrites lds: every lane must have read first
-            if (s + 1 < nst) __syncthreads();
+            __syncthreads();
+            continue;
         }
-        const uint32_t ob = ST[s].op_begin, oe = ST[s].op_end;
-        for (uint32_t o = ob; o < oe; o++) apply_op<R, RB>(a, OP + o, tid, blk);
+        if (kind == SLOT_TAB) {
+            const Factor<R>* __restrict__ tab = (const Factor<R>*)pc;
+#pragma unroll
+            for (int j = 0; j < NR; j++) scale(a[j], tab[j]);
+            pc += aux * SLOT;
+            next = *(const SlotRegs<R>*)pc;
+            continue;
+        }
+        if (kind == SLOT_TABMASK) {
+            const Factor<R>* __restrict__ tab = (const Factor<R>*)pc;
+            const uint64_t jm = (uint64_t)cbv << 32 | cb;
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if ((jm >> j) & 1) scale(a[j], tab[j]);
+            pc += aux * SLOT;
+            next = *(const SlotRegs<R>*)pc;
+            continue;
+        }
+        if (kind == SLOT_SCALE) {
+#pragma unroll
+            for (int j = 0; j < NR; j++) scale(a[j], s.m[0], s.m[1]);
+            continue;
+        }
+        if (kind == SLOT_LANEMUL) {
+            const Factor<R> f = Factor<R>::of(lx, ly);
+#pragma unroll
+            for (int j = 0; j < NR; j++) scale(a[j], f);
+            lx = 1;
+            ly = 0;
+            continue;
+        }
+        if (kind == SLOT_LANETAB) {
+            const HQ_GLOBAL Factor<R>* __restrict__ t =
+                (const HQ_GLOBAL Factor<R>*)(prog + H->lane_off) + (size_t)cb * NT;
+            const Factor<R> f = t[tid];
+            lx = f.x;
+            ly = f.y;
+            if constexpr (sizeof(R) == 4) { lx += f.lx; ly += f.ly; }
+            continue;
+        }
+        if (kind == SLOT_REFILL) {
+            window += (uint32_t)WIN_BYTES;
+            __syncthreads();   // every lane has read this window's last slot
+            fetch(window);
+            fill();
+            __syncthreads();
+            pc = win;
+            next = *(const SlotRegs<R>*)pc;
+            continue;
+        }
+        if (kind == SLOT_END) break;
+        if (((uint32_t)blk & cb) != cbv) continue;
+        if (kind == SLOT_LANE) {
+            const double fr = on ? (double)s.m[0] : 1.0, fi = on ? (double)s.m[1] : 0.0;
+            const double x = lx, y = ly;
+            lx = fr * x - fi * y;
+            ly = fr * y + fi * x;
+        } else if (kind == SLOT_MIXSIGN) {
+            const R f = on ? R(-1) : R(1);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if ((j & creg) == cregv) { a[j].x *= f; a[j].y *= f; }
+        } else {   // SLOT_MIX
+            const R fr = on ? s.m[0] : R(1), fi = on ? s.m[1] : R(0);
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if ((j & creg) == cregv) scale(a[j], fr, fi);
+        }
     }
 
     // mapping of the last stage
-    pt = 0;
+    uint64_t pt = 0;
 #pragma unroll
-    for (int i = 0; i < TB; i++)
-        if ((et >> ST[nst - 1].thr_bits[i]) & 1) pt |= H->tile_phys[ST[nst - 1].thr_bits[i]];
+    for (int i = 0; i < TB; i++) pt |= (uint64_t)((tid >> i) & 1u) << H->st_thr[i];
 #pragma unroll
-    for (int i = 0; i < RB; i++) rphys[i] = H->tile_phys[ST[nst - 1].reg_bits[i]];
+    for (int i = 0; i < RB; i++) rphys[i] = (uint64_t)1 << H->st_reg[i];
 
     if (mode & TILE_READ) {
         double s0 = 0, s1 = 0, s2 = 0;
