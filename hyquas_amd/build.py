@@ -35,6 +35,11 @@ INCLUDES = ["-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(CSRC, "hos
 # packed-FP32 instructions are disabled for every HIP file (-packed-fp32-ops)
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"] + INCLUDES
+# The interpreter's dispatch loop branches on values uniform over the block
+# only; left as it is, the structurizer rewrites such a loop as if its branches
+# diverged, with copies of every amplitude at each join.
+INTERPRETER_FLAGS = ["-mllvm", "-structurizecfg-skip-uniform-regions=1"]
+INTERPRETER_FILES = ("sharemem.hip", "engine.hip")
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-fopenmp"] + INCLUDES
 
 
@@ -63,6 +68,11 @@ def _obj(src):
     return os.path.join(BUILD, rel + ".o")
 
 
+def device_command(src):
+    extra = INTERPRETER_FLAGS if os.path.basename(src) in INTERPRETER_FILES else []
+    return [HIPCC] + HIP_FLAGS + extra + ["-c", src, "-o", _obj(src)]
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> str:
     if shutil.which(HIPCC) is None and not os.path.exists(HIPCC):
         raise RuntimeError("hipcc not found; the HIP toolchain is required to build hyquas_amd")
@@ -70,7 +80,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
     dev, host = _sources()
     cmds = []
     for s in dev:
-        cmds.append([HIPCC] + HIP_FLAGS + ["-c", s, "-o", _obj(s)])
+        cmds.append(device_command(s))
     for s in host:
         cmds.append([CXX] + CXX_FLAGS + ["-c", s, "-o", _obj(s)])
     main_src = os.path.join(CSRC, "host", "main.cpp")
