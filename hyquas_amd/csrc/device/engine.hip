@@ -85,7 +85,7 @@ __global__ __launch_bounds__(1 << TB) void k_batch_sharemem(const BatchItem* __r
     __shared__ __align__(16) char win[SHM_WINDOW_LDS];
     const uint64_t b = blockIdx.x;
     const BatchItem* it = items + find_item(items, count, b);
-    tile_pass<R, RB, TB>((cplx<R>*)it->psi, (const char*)it->prog, b - it->first_block, lds, win, it->mode, (int)it->n,
+    tile_pass<R, RB, TB, false>((cplx<R>*)it->psi, (const char*)it->prog, b - it->first_block, lds, win, it->mode, (int)it->n,
                          (double*)it->part);
 }
 
@@ -520,8 +520,11 @@ static void append_jit(JobPlan* jp, const ShmPlan& plan, const std::vector<doubl
 static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<hq_gate>& hg, uint64_t mask,
                            bool first, bool last, uint64_t zero_mask, KernelCache* kc)
 {
+    // an engine returns sums over a circuit's qubits, which merged factors in
+    // one float serve; its passes are bound by the operations they save
     ShmPlan plan;
-    hq_status st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, kc && first, 0, kc != nullptr);
+    hq_status st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, kc && first, 0, kc != nullptr,
+                                 DiagMode::MERGED);
     if (st != HQ_OK) return st;
     plan.hdr.zero_mask = zero_mask;
     // the first pass only writes; later ones skip the tiles whose block
@@ -545,7 +548,7 @@ static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<
         // in the interpreter's op forms (the shared-code forms are the
         // specialised kernels' own)
         plan = ShmPlan();
-        st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, false, 0, false);
+        st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, false, 0, false, DiagMode::MERGED);
         if (st != HQ_OK) return st;
         plan.hdr.zero_mask = zero_mask;
     }

@@ -150,7 +150,8 @@ struct ShmHeader {
 
 // ---- the interpreter's program: header, op slots, lane tables ---------------------------
 // A slot is 16 bytes of decoded fields and eight coefficients in the state's
-// precision.  The kernel copies slots to LDS a window at a time (one memory
+// precision; the coefficients of a pair update are its 2x2 matrix's real parts,
+// then the imaginary ones.  The kernel copies slots to LDS a window at a time (one memory
 // latency per window instead of several per op) and reads the next slot while
 // it executes one.
 struct ShmSlot {
@@ -258,6 +259,10 @@ struct hq_program_s {
 };
 
 namespace hq {
+// How a plan applies diagonal gates: gate by gate; merged across the stage; or
+// merged with complex64 factors kept as two floats (ShmPlan::precise).
+enum class DiagMode { APART, MERGED, PRECISE };
+
 // Launchers implemented in the .hip files.
 hq_status launch_sharemem(hq_state s, hq_program p);
 hq_status transpose_prepare(hq_state s, const int* perm, void** dev_args);
@@ -269,12 +274,11 @@ int sharemem_default_rb(int precision, int tile);
 // io: bit 0 adds a leading, bit 1 a trailing stage without gates where the
 // first / last stage holds one of the three lowest tile bits in registers
 // (the HBM access then covers whole 128-byte lines per wave instruction).
-// merge: diagonal gates merged across the stage (false: applied gate by gate).
 // shared_code: op classes that do not depend on gate angles (rotations keep
 // their full 2x2 form), so same-structure groups share a specialised kernel.
 hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gates, uint64_t shared_mask,
                         int rb, ShmPlan* out, bool init = false, int io = 0, bool shared_code = false,
-                        bool merge = true);
+                        DiagMode diag = DiagMode::PRECISE);
 // The interpreter's program of a plan (ShmProg header, slots, lane tables).
 std::vector<char> encode_program(const ShmPlan& plan);
 // Specialised kernel for a planned group: generate, compile (cached), load.

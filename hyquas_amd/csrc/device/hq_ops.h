@@ -75,17 +75,15 @@ __device__ __forceinline__ void scale(cplx<R>& v, R re, R im)
     v.y = re * y + im * x;
 }
 
-// A merged diagonal factor: complex128 as it is, complex64 as the sum of two
-// floats per part (ShmPlan::precise).
-template <typename R>
-struct Factor;
-template <>
-struct alignas(16) Factor<double> {
-    double x, y;
-    static __host__ __device__ Factor of(double re, double im) { return Factor{re, im}; }
+// A merged diagonal factor: in the state's precision, or for complex64 as the
+// sum of two floats per part (ShmPlan::precise).
+template <typename R, bool PRECISE>
+struct alignas(2 * sizeof(R)) Factor {
+    R x, y;
+    static __host__ __device__ Factor of(double re, double im) { return Factor{(R)re, (R)im}; }
 };
 template <>
-struct alignas(16) Factor<float> {
+struct alignas(16) Factor<float, true> {
     float x, y, lx, ly;
     static __host__ __device__ Factor of(double re, double im)
     {
@@ -94,8 +92,9 @@ struct alignas(16) Factor<float> {
     }
 };
 
-__device__ __forceinline__ void scale(cplx<double>& v, const Factor<double>& f) { scale<double>(v, f.x, f.y); }
-__device__ __forceinline__ void scale(cplx<float>& v, const Factor<float>& f)
+template <typename R>
+__device__ __forceinline__ void scale(cplx<R>& v, const Factor<R, false>& f) { scale<R>(v, f.x, f.y); }
+__device__ __forceinline__ void scale(cplx<float>& v, const Factor<float, true>& f)
 {
     const float x = v.x, y = v.y;
     v.x = f.x * x - (f.y * y - (f.lx * x - f.ly * y));

@@ -1103,7 +1103,8 @@ extern "C" hq_status hq_sharemem_source(int n, int precision, const hq_gate* gat
     HQ_CHECK(batch || !readout, HQ_ERR_ARG, "hq_sharemem_source: the readout fold needs the batched form");
     hq::ShmPlan plan;
     hq_status st = hq::plan_sharemem(n, precision, gates, num_gates, shared_mask, reg_qubits, &plan, init,
-                                     whole_line ? 3 : 0, shared_code);
+                                     whole_line ? 3 : 0, shared_code,
+                                     shared_code ? hq::DiagMode::MERGED : hq::DiagMode::PRECISE);
     if (st != HQ_OK) return st;
     // bit 0 alone: whole-line stages with non-temporal loads and stores; with
     // bit 5: whole-line stages, non-temporal stores only; bit 5 alone: the

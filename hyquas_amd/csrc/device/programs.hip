@@ -330,7 +330,7 @@ hq_status build_sharemem_programs(hq_state s, const std::vector<SharememRequest>
     // is of the order of what one rounding of a merged factor moves it by
     // (ShmPlan::precise), and the pass is not bound by the operations saved
     // (31 qubits, 18 groups: 128 ms merged, 126 ms apart)
-    const bool merge = !(jit && s->precision == HQ_C64);
+    const bool apart = jit && s->precision == HQ_C64;
     auto destroy_all = [&]() {
         for (auto& v : built)
             for (auto p : v) hq_program_destroy(p);
@@ -340,7 +340,7 @@ hq_status build_sharemem_programs(hq_state s, const std::vector<SharememRequest>
         for (size_t i = 0; i < reqs.size(); i++) {
             hq_status st = build_sharemem_program(s, reqs[i].gates.data(), (int)reqs[i].gates.size(), reqs[i].mask,
                                                   reg_qubits, &built[v][i], reqs[i].init, tune ? kTuned[v] : only,
-                                                  reqs[i].zero_mask, merge);
+                                                  reqs[i].zero_mask, apart);
             if (st != HQ_OK) { destroy_all(); return st; }
         }
     }

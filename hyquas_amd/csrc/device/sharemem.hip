@@ -37,7 +37,7 @@ __global__ __launch_bounds__(1 << TB) void k_sharemem(cplx<R>* __restrict__ psi,
 {
     __shared__ cplx<R> lds[1 << (RB + TB)];
     __shared__ __align__(16) char win[SHM_WINDOW_LDS];
-    tile_pass<R, RB, TB>(psi, prog, blockIdx.x, lds, win, mode, 0, nullptr);
+    tile_pass<R, RB, TB, sizeof(R) == 4>(psi, prog, blockIdx.x, lds, win, mode, 0, nullptr);
 }
 
 // ---- launch table -------------------------------------------------------------------------
@@ -540,7 +540,7 @@ private:
 }  // namespace
 
 hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gates, uint64_t shared_mask, int rb_req,
-                        ShmPlan* plan, bool init, int io, bool shared_code, bool merge)
+                        ShmPlan* plan, bool init, int io, bool shared_code, DiagMode diag)
 {
     HQ_CHECK(num_gates >= 0 && (num_gates == 0 || gates), HQ_ERR_ARG, "sharemem: bad gate array");
     const size_t amp_bytes = precision == HQ_C128 ? 16 : 8;
@@ -700,10 +700,8 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
 
     // lower the stages' gates to ops, diagonal gates merged (StageLowering)
     std::vector<ShmStage> dst;
-    // batched kernels return sums over a circuit's qubits, which the one-float
-    // form serves, and are bound by the operations it saves
-    const bool precise = precision == HQ_C64 && !shared_code;
-    StageLowering lo(low, low_type, precision, rb, tb, shared_code, precise, merge);
+    const bool precise = precision == HQ_C64 && diag == DiagMode::PRECISE;
+    StageLowering lo(low, low_type, precision, rb, tb, shared_code, precise, diag != DiagMode::APART);
     for (auto& S : stages) {
         ShmStage d;
         memset(&d, 0, sizeof(d));
@@ -746,11 +744,11 @@ hq_status plan_sharemem(int n, int precision, const hq_gate* gates, int num_gate
 
 namespace {
 
-template <typename R>
+template <typename R, bool PRECISE>
 struct Encoder {
     const ShmPlan& P;
     std::vector<char> slots;
-    std::vector<Factor<R>> lanes;   // 2^tb entries per lane table
+    std::vector<Factor<R, PRECISE>> lanes;   // 2^tb entries per lane table
     static constexpr int SLOT = shm_slot_bytes<R>();
     static_assert(SHM_WINDOW_BYTES % SLOT == 0, "windows hold whole slots");
 
@@ -779,7 +777,8 @@ struct Encoder {
     void op(const ShmSlot& h, const double* m, int nm)
     {
         R c[8] = {};
-        for (int i = 0; i < nm; i++) c[i] = (R)m[i];
+        // a matrix: real parts first (real updates read half of the slot)
+        for (int i = 0; i < nm; i++) c[nm == 8 ? (i & 1) * 4 + i / 2 : i] = (R)m[i];
         room(1);
         put(h, c, sizeof(c));
     }
@@ -826,7 +825,7 @@ struct Encoder {
             h.cblk = (uint32_t)(lanes.size() / NT);
             for (int t = 0; t < NT; t++) {
                 const std::complex<double> v = f[t] * S;
-                lanes.push_back(Factor<R>::of(v.real(), v.imag()));
+                lanes.push_back(Factor<R, PRECISE>::of(v.real(), v.imag()));
             }
             op(h, nullptr, 0);
         }
@@ -834,11 +833,11 @@ struct Encoder {
             const ShmOp& o = P.ops[i];
             switch (o.cls) {
             case SHM_TAB: {
-                const size_t bytes = ((size_t)1 << P.rb) * sizeof(Factor<R>);
+                const size_t bytes = ((size_t)1 << P.rb) * sizeof(Factor<R, PRECISE>);
                 const size_t more = (bytes + SLOT - 1) / SLOT;
-                std::vector<Factor<R>> t((size_t)1 << P.rb);
+                std::vector<Factor<R, PRECISE>> t((size_t)1 << P.rb);
                 for (size_t j = 0; j < t.size(); j++)
-                    t[j] = Factor<R>::of(P.tabs[2 * (o.tab + j)], P.tabs[2 * (o.tab + j) + 1]);
+                    t[j] = Factor<R, PRECISE>::of(P.tabs[2 * (o.tab + j)], P.tabs[2 * (o.tab + j) + 1]);
                 ShmSlot h{};
                 // per-index branches pay when at least half of the indices keep their amplitude
                 const bool mask = 2 * __builtin_popcountll(o.jmask) <= (1 << P.rb);
@@ -913,10 +912,10 @@ struct Encoder {
         const size_t tail = slots.size() - slots.size() % (size_t)SHM_WINDOW_BYTES + SHM_WINDOW_COPY;
         const size_t lane_off = (SHM_PROG_HEADER + tail + 255) & ~(size_t)255;
         H.lane_off = (uint32_t)lane_off;
-        std::vector<char> out(lane_off + lanes.size() * sizeof(Factor<R>), 0);
+        std::vector<char> out(lane_off + lanes.size() * sizeof(Factor<R, PRECISE>), 0);
         memcpy(out.data(), &H, sizeof(H));
         memcpy(out.data() + SHM_PROG_HEADER, slots.data(), slots.size());
-        if (!lanes.empty()) memcpy(out.data() + lane_off, lanes.data(), lanes.size() * sizeof(Factor<R>));
+        if (!lanes.empty()) memcpy(out.data() + lane_off, lanes.data(), lanes.size() * sizeof(Factor<R, PRECISE>));
         return out;
     }
 };
@@ -925,21 +924,23 @@ struct Encoder {
 
 std::vector<char> encode_program(const ShmPlan& plan)
 {
-    if (plan.precision == HQ_C128) return Encoder<double>{plan, {}, {}}.run();
-    return Encoder<float>{plan, {}, {}}.run();
+    if (plan.precision == HQ_C128) return Encoder<double, false>{plan, {}, {}}.run();
+    if (plan.precise) return Encoder<float, true>{plan, {}, {}}.run();
+    return Encoder<float, false>{plan, {}, {}}.run();
 }
 
 hq_status build_sharemem_program(hq_state s, const hq_gate* gates, int num_gates, uint64_t shared_mask, int rb_req,
-                                 hq_program* out, bool init, int variant, uint64_t zero_mask, bool merge)
+                                 hq_program* out, bool init, int variant, uint64_t zero_mask, bool apart)
 {
     HQ_CHECK(s && out, HQ_ERR_ARG, "sharemem: null argument");
     *out = nullptr;
     ShmPlan plan;
+    const DiagMode diag = apart ? DiagMode::APART : DiagMode::PRECISE;
     // variant bit 0: whole-line stages; bit 1: non-temporal stores; bit 2:
     // non-temporal loads
     const bool whole_line = variant & 1;
     hq_status st = plan_sharemem(s->n, s->precision, gates, num_gates, shared_mask, rb_req, &plan, init,
-                                 whole_line ? 3 : 0, false, merge);
+                                 whole_line ? 3 : 0, false, diag);
     if (st != HQ_OK) return st;
     plan.init = init;
     plan.whole_line = whole_line;

@@ -71,15 +71,29 @@ __device__ __forceinline__ void lane_swap(cplx<R> (&a)[1 << RB], uint32_t creg, 
     }
 }
 
+// c: the matrix's real parts, rest: its imaginary ones in LDS (read by the
+// forms that have any); lane: some thread-bit control, `on` where it holds
 template <typename R, int RB, int P>
-__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool on, const R* m)
+__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool lane, bool on,
+                                       const R (&c)[4], const R* rest)
 {
+    R m[8];
+    auto matrix = [&](bool imag) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) { m[2 * i] = c[i]; m[2 * i + 1] = imag ? rest[i] : R(0); }
+        if (lane) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (imag || !(i & 1)) m[i] = on ? m[i] : (i == 0 || i == 6) ? R(1) : R(0);
+        }
+    };
+    m[0] = c[0];
     switch (kind) {
     case SHM_SWAP: reg_pairs<R, RB, SHM_SWAP, P>(a, creg, m); break;
     case SHM_Y: reg_pairs<R, RB, SHM_Y, P>(a, creg, m); break;
-    case SHM_REAL: reg_pairs<R, RB, SHM_REAL, P>(a, creg, m); break;
-    case SHM_RX: reg_pairs<R, RB, SHM_RX, P>(a, creg, m); break;
-    case SHM_GEN: reg_pairs<R, RB, SHM_GEN, P>(a, creg, m); break;
+    case SHM_REAL: matrix(false); reg_pairs<R, RB, SHM_REAL, P>(a, creg, m); break;
+    case SHM_RX: matrix(true); reg_pairs<R, RB, SHM_RX, P>(a, creg, m); break;
+    case SHM_GEN: matrix(true); reg_pairs<R, RB, SHM_GEN, P>(a, creg, m); break;
     case SHM_HADD: reg_pairs<R, RB, SHM_HADD, P>(a, creg, m); break;
     case SHM_ROTA: reg_pairs<R, RB, SHM_ROTA, P>(a, creg, m); break;
     case SHM_ROTB: reg_pairs<R, RB, SHM_ROTB, P>(a, creg, m); break;
@@ -90,13 +104,6 @@ __device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t
 }
 
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-
-// a slot as it sits in LDS
-template <typename R>
-struct alignas(16) SlotRegs {
-    uint4 h;
-    R m[8];
-};
 
 // Z-sum and nearest-neighbour ZZ-sum eigenvalues of basis state idx over n qubits:
 // sum_q (1 - 2 b_q) and sum_{q<n-1} (1 - 2 (b_q xor b_{q+1})).
@@ -120,7 +127,7 @@ __device__ __forceinline__ void zsums(uint64_t idx, int n, double* z, double* zz
 // 17-qubit complex64 and 20-qubit complex128 random circuits (32 and 256
 // blocks) went from 61 and 67.5 us to 37 and 38 us, the 174 gates of a
 // 10-qubit ansatz (one wave) from 132 to 51 us.
-template <typename R, int RB, int TB>
+template <typename R, int RB, int TB, bool PRECISE>
 __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const char* __restrict__ prog_any,
                                           uint64_t blk, cplx<R>* __restrict__ lds, char* __restrict__ win,
                                           uint32_t mode, int n, double* __restrict__ part_any)
@@ -214,28 +221,32 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
         }
     }
     fill();
-    // LDS indices of the current stage
+    // LDS addresses (bytes) of the current stage
     uint32_t at, reg_at[RB];
     {
         uint32_t r = 0;
 #pragma unroll
         for (int i = 0; i < TB; i++) r ^= (0u - ((tid >> i) & 1u)) & (uint32_t)H->first.thr[i];
-        at = r;
+        at = r * (uint32_t)sizeof(cplx<R>);
 #pragma unroll
-        for (int i = 0; i < RB; i++) reg_at[i] = H->first.reg[i];
+        for (int i = 0; i < RB; i++) reg_at[i] = H->first.reg[i] * (uint32_t)sizeof(cplx<R>);
     }
     __syncthreads();
 
     double lx = 1, ly = 0;    // the lane's factor
     uint32_t window = 0;      // bytes of the current window's start in the program
     const char* pc = win;
-    SlotRegs<R> next = *(const SlotRegs<R>*)pc;
+    uint4 next = *(const uint4*)pc;   // fields of the next slot
+    char* const xlds = (char*)lds;
     for (;;) {
-        const SlotRegs<R> s = next;
+        const uint32_t w0 = uniform(next.x), w1 = uniform(next.y);
+        const uint32_t cb = uniform(next.z), cbv = uniform(next.w);
+        const R* const coef = (const R*)(pc + 16);
+        R c[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) c[i] = coef[i];
         pc += SLOT;
-        next = *(const SlotRegs<R>*)pc;   // (behind the last slot of a window: unused)
-        const uint32_t w0 = uniform(s.h.x), w1 = uniform(s.h.y);
-        const uint32_t cb = uniform(s.h.z), cbv = uniform(s.h.w);
+        next = *(const uint4*)pc;     // (behind the last slot of a window: unused)
         const int kind = (int)(w0 & 255u), aux = (int)((w0 >> 8) & 255u);
         const uint32_t creg = (w0 >> 16) & 255u, cregv = w0 >> 24;
         const uint32_t cthr = w1 & 0xffffu, cthrv = w1 >> 16;
@@ -245,82 +256,77 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
         // or keeps its values by selects instead of leaving the op.
         if (kind <= SLOT_CSWAP) {
             if (((uint32_t)blk & cb) != cbv) continue;
-            R m[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) m[i] = s.m[i];
-            if (cthr) {
-#pragma unroll
-                for (int i = 0; i < 8; i++) m[i] = on ? m[i] : (i == 0 || i == 6) ? R(1) : R(0);
-            }
+            const bool lane = cthr != 0;
             switch (aux) {
-            case 0: reg_op<R, RB, 0>(a, kind, creg, on, m); break;
-            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, on, m); break;
-            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, on, m); break;
-            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, on, m); break;
-            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, on, m); break;
-            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, on, m); break;
+            case 0: reg_op<R, RB, 0>(a, kind, creg, lane, on, c, coef + 4); break;
+            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, lane, on, c, coef + 4); break;
+            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, lane, on, c, coef + 4); break;
+            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, lane, on, c, coef + 4); break;
+            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, lane, on, c, coef + 4); break;
+            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, lane, on, c, coef + 4); break;
             }
             static_assert(RB <= 6, "register positions above 5 are not dispatched");
             continue;
         }
         if (kind == SLOT_XCHG) {
             // write under the old split, read under the new one; a register's
-            // LDS index is the lane's xor its register bits' entries
-            auto entry = [&](int e) -> uint32_t {   // e-th 16-bit field of the ShmXchg in s.m
-                uint32_t w;
-                if constexpr (sizeof(R) == 4) w = __float_as_uint(s.m[e / 2]);
-                else w = (e & 2) ? (uint32_t)__double2hiint(s.m[e / 4]) : (uint32_t)__double2loint(s.m[e / 4]);
-                return (e & 1) ? w >> 16 : w & 0xffffu;
-            };
+            // LDS address is the lane's xor its register bits' entries (all
+            // kept in bytes: one xor per access)
 #pragma unroll
             for (int j = 0; j < NR; j++) {
                 uint32_t so = 0;
 #pragma unroll
                 for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= reg_at[i];
-                lds[at ^ so] = a[j];
+                *(cplx<R>*)(xlds + (at ^ so)) = a[j];
             }
+            const ShmXchg* const x = (const ShmXchg*)coef;
+            uint32_t e[(SHM_MAX_TB + SHM_MAX_RB + 1) / 2];   // two 16-bit entries each
+#pragma unroll
+            for (int i = 0; i < (int)(sizeof(e) / 4); i++) e[i] = ((const uint32_t*)x)[i];
+            auto entry = [&](int i) { return (i & 1) ? e[i / 2] >> 16 : e[i / 2] & 0xffffu; };
             at = 0;
 #pragma unroll
             for (int i = 0; i < TB; i++) at ^= (0u - ((tid >> i) & 1u)) & entry(i);
+            at *= (uint32_t)sizeof(cplx<R>);
 #pragma unroll
-            for (int i = 0; i < RB; i++) reg_at[i] = uniform(entry(SHM_MAX_TB + i));
+            for (int i = 0; i < RB; i++) reg_at[i] = uniform(entry(SHM_MAX_TB + i)) * (uint32_t)sizeof(cplx<R>);
             __syncthreads();
 #pragma unroll
             for (int j = 0; j < NR; j++) {
                 uint32_t so = 0;
 #pragma unroll
                 for (int i = 0; i < RB; i++) if ((j >> i) & 1) so ^= reg_at[i];
-                a[j] = lds[at ^ so];
+                a[j] = *(const cplx<R>*)(xlds + (at ^ so));
             }
             // the next exchange overwrites lds: every lane must have read first
             __syncthreads();
             continue;
         }
         if (kind == SLOT_TAB) {
-            const Factor<R>* __restrict__ tab = (const Factor<R>*)pc;
+            const Factor<R, PRECISE>* __restrict__ tab = (const Factor<R, PRECISE>*)pc;
 #pragma unroll
             for (int j = 0; j < NR; j++) scale(a[j], tab[j]);
             pc += aux * SLOT;
-            next = *(const SlotRegs<R>*)pc;
+            next = *(const uint4*)pc;
             continue;
         }
         if (kind == SLOT_TABMASK) {
-            const Factor<R>* __restrict__ tab = (const Factor<R>*)pc;
+            const Factor<R, PRECISE>* __restrict__ tab = (const Factor<R, PRECISE>*)pc;
             const uint64_t jm = (uint64_t)cbv << 32 | cb;
 #pragma unroll
             for (int j = 0; j < NR; j++)
                 if ((jm >> j) & 1) scale(a[j], tab[j]);
             pc += aux * SLOT;
-            next = *(const SlotRegs<R>*)pc;
+            next = *(const uint4*)pc;
             continue;
         }
         if (kind == SLOT_SCALE) {
 #pragma unroll
-            for (int j = 0; j < NR; j++) scale(a[j], s.m[0], s.m[1]);
+            for (int j = 0; j < NR; j++) scale(a[j], c[0], c[1]);
             continue;
         }
         if (kind == SLOT_LANEMUL) {
-            const Factor<R> f = Factor<R>::of(lx, ly);
+            const Factor<R, PRECISE> f = Factor<R, PRECISE>::of(lx, ly);
 #pragma unroll
             for (int j = 0; j < NR; j++) scale(a[j], f);
             lx = 1;
@@ -328,12 +334,12 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             continue;
         }
         if (kind == SLOT_LANETAB) {
-            const HQ_GLOBAL Factor<R>* __restrict__ t =
-                (const HQ_GLOBAL Factor<R>*)(prog + H->lane_off) + (size_t)cb * NT;
-            const Factor<R> f = t[tid];
+            const HQ_GLOBAL Factor<R, PRECISE>* __restrict__ t =
+                (const HQ_GLOBAL Factor<R, PRECISE>*)(prog + H->lane_off) + (size_t)cb * NT;
+            const Factor<R, PRECISE> f = t[tid];
             lx = f.x;
             ly = f.y;
-            if constexpr (sizeof(R) == 4) { lx += f.lx; ly += f.ly; }
+            if constexpr (PRECISE) { lx += f.lx; ly += f.ly; }
             continue;
         }
         if (kind == SLOT_REFILL) {
@@ -343,13 +349,13 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             fill();
             __syncthreads();
             pc = win;
-            next = *(const SlotRegs<R>*)pc;
+            next = *(const uint4*)pc;
             continue;
         }
         if (kind == SLOT_END) break;
         if (((uint32_t)blk & cb) != cbv) continue;
         if (kind == SLOT_LANE) {
-            const double fr = on ? (double)s.m[0] : 1.0, fi = on ? (double)s.m[1] : 0.0;
+            const double fr = on ? (double)c[0] : 1.0, fi = on ? (double)c[1] : 0.0;
             const double x = lx, y = ly;
             lx = fr * x - fi * y;
             ly = fr * y + fi * x;
@@ -359,7 +365,7 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             for (int j = 0; j < NR; j++)
                 if ((j & creg) == cregv) { a[j].x *= f; a[j].y *= f; }
         } else {   // SLOT_MIX
-            const R fr = on ? s.m[0] : R(1), fi = on ? s.m[1] : R(0);
+            const R fr = on ? c[0] : R(1), fi = on ? c[1] : R(0);
 #pragma unroll
             for (int j = 0; j < NR; j++)
                 if ((j & creg) == cregv) scale(a[j], fr, fi);

@@ -13,11 +13,11 @@ void set_error(const std::string& msg);
 // (reg_qubits = 0: default for the tile size); init: the group builds
 // |0...0> in registers instead of loading the state; variant (specialised
 // kernel) bit 0: whole-line HBM stages (added stages without gates where
-// needed); bit 1: non-temporal stores; bit 2: non-temporal loads; merge:
-// diagonal gates of a stage merged into tables and lane factors.
+// needed); bit 1: non-temporal stores; bit 2: non-temporal loads; apart:
+// diagonal gates applied gate by gate, not merged.
 hq_status build_sharemem_program(hq_state s, const hq_gate* gates, int num_gates, uint64_t shared_mask,
                                  int reg_qubits, hq_program* out, bool init = false, int variant = 0,
-                                 uint64_t zero_mask = 0, bool merge = true);
+                                 uint64_t zero_mask = 0, bool apart = false);
 
 // Many OShareMem programs at once; with jit, every group also gets a
 // structure-specialised kernel, compiled in parallel.  tune_mode (jit only):
