@@ -520,10 +520,14 @@ static void append_jit(JobPlan* jp, const ShmPlan& plan, const std::vector<doubl
 static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<hq_gate>& hg, uint64_t mask,
                            bool first, bool last, uint64_t zero_mask, KernelCache* kc)
 {
+    // many circuits fill the chip together: the single-state rule for few
+    // blocks (n - tile small) does not apply here
+    const int tile = __builtin_popcountll((unsigned long long)mask);
+    const int irb = interpreter_rb(precision, tile, 64);
     // an engine returns sums over a circuit's qubits, which merged factors in
     // one float serve; its passes are bound by the operations they save
     ShmPlan plan;
-    hq_status st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, kc && first, 0, kc != nullptr,
+    hq_status st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, kc ? 0 : irb, &plan, kc && first, 0, kc != nullptr,
                                  DiagMode::MERGED);
     if (st != HQ_OK) return st;
     plan.hdr.zero_mask = zero_mask;
@@ -548,7 +552,7 @@ static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<
         // in the interpreter's op forms (the shared-code forms are the
         // specialised kernels' own)
         plan = ShmPlan();
-        st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, 0, &plan, false, 0, false, DiagMode::MERGED);
+        st = plan_sharemem(n, precision, hg.data(), (int)hg.size(), mask, irb, &plan, false, 0, false, DiagMode::MERGED);
         if (st != HQ_OK) return st;
         plan.hdr.zero_mask = zero_mask;
     }

@@ -271,6 +271,8 @@ hq_status launch_dense(hq_state s, const void* d_mat, int mat_qubits, void* in, 
 // U (rows in the order of the set bits of `rows`) on those qubits, in place.
 hq_status launch_dense_at(hq_state s, const void* d_mat, int mat_qubits, uint64_t rows);
 int sharemem_default_rb(int precision, int tile);
+// Register qubits of the interpreter's kernel on one n-qubit state.
+int interpreter_rb(int precision, int tile, int n);
 // io: bit 0 adds a leading, bit 1 a trailing stage without gates where the
 // first / last stage holds one of the three lowest tile bits in registers
 // (the HBM access then covers whole 128-byte lines per wave instruction).

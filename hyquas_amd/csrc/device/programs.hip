@@ -19,7 +19,9 @@ extern "C" {
 hq_status hq_program_create_sharemem(hq_state s, const hq_gate* gates, int num_gates, uint64_t shared_mask,
                                      hq_program* out)
 {
-    return build_sharemem_program(s, gates, num_gates, shared_mask, 0, out);
+    HQ_CHECK(s, HQ_ERR_ARG, "sharemem: null argument");
+    const int rb = interpreter_rb(s->precision, __builtin_popcountll((unsigned long long)shared_mask), s->n);
+    return build_sharemem_program(s, gates, num_gates, shared_mask, rb, out);
 }
 
 // U as split planes (re | im) in the state's precision: FP64 fusion, rounded
@@ -338,8 +340,10 @@ hq_status build_sharemem_programs(hq_state s, const std::vector<SharememRequest>
     out->assign(reqs.size(), nullptr);
     for (int v = 0; v < variants; v++) {
         for (size_t i = 0; i < reqs.size(); i++) {
+            const int tile = __builtin_popcountll((unsigned long long)reqs[i].mask);
+            const int rb = reg_qubits > 0 || jit ? reg_qubits : interpreter_rb(s->precision, tile, s->n);
             hq_status st = build_sharemem_program(s, reqs[i].gates.data(), (int)reqs[i].gates.size(), reqs[i].mask,
-                                                  reg_qubits, &built[v][i], reqs[i].init, tune ? kTuned[v] : only,
+                                                  rb, &built[v][i], reqs[i].init, tune ? kTuned[v] : only,
                                                   reqs[i].zero_mask, apart);
             if (st != HQ_OK) { destroy_all(); return st; }
         }

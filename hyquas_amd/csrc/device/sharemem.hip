@@ -94,6 +94,21 @@ int sharemem_default_rb(int precision, int tile)
     return tile >= 14 ? 6 : tile == 13 ? 5 : tile == 12 ? 4 : tile - 6;
 }
 
+int interpreter_rb(int precision, int tile, int n)
+{
+    // Up to a block or two per CU a pass is a chain of ops whose latency shows:
+    // 8 amplitudes on twice the threads take less of it per op than 16 and one
+    // more exchange per stage costs.  12-qubit tiles, 16 random layers, 16 and
+    // 8 amplitudes: complex64 17 qubits 212 and 165 us, 20 qubits 367 and 235,
+    // 21 qubits (512 blocks) 407 and 339; complex128 17 qubits 210 and 186, 20
+    // qubits 334 and 306, but 21 qubits 413 and 515.  10 qubits in one block: 103 and 87.
+    if (tile >= 10 && tile <= 12 && n - tile <= (precision == HQ_C128 ? 8 : 9)) return 3;
+    // 13-qubit complex64 blocks: 512 threads x 16 instead of 256 x 32 (100
+    // ansatz circuits of 10 to 14 qubits: 0.93 and 1.16 ms)
+    if (tile == 13 && precision == HQ_C64) return 4;
+    return sharemem_default_rb(precision, tile);
+}
+
 // ---- host side: lowering + register-stage planning -------------------------------------------
 
 namespace {
