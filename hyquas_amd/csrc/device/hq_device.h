@@ -55,6 +55,9 @@ struct hq_state_s {
     double* d_red = nullptr;  // reduction scratch (device)
     double* h_red = nullptr;  // reduction scratch (pinned host)
     size_t red_cap = 0;       // doubles
+    char* d_ws = nullptr;     // readout workspace (device, pinned host), see ensure_ws
+    char* h_ws = nullptr;
+    size_t ws_dev = 0, ws_host = 0;   // bytes
     bool profiling = false;
     std::vector<hq::ProfileEntry> prof;
     std::vector<hipEvent_t> free_events;
@@ -65,6 +68,12 @@ namespace hq {
 // Profiling helpers: bracket one launch with events when enabled.
 hq_status prof_begin(hq_state s, int kind, int* slot);
 hq_status prof_end(hq_state s, int slot);
+
+// Room for a readout in the state's workspace (grown on demand, freed with
+// the state); contents do not outlive a call.
+hq_status ensure_ws(hq_state s, size_t dev, size_t host);
+// Gives back workspace beyond `keep` bytes (no work of the state may use it).
+void trim_ws(hq_state s, size_t keep);
 
 // ---- OShareMem program (device-resident) ---------------------------------------------
 // Op classes of the register kernel.

@@ -5,6 +5,7 @@
 // throughout (the reference's int nVec overflows at n >= 33).
 
 #include "hq_device.h"
+#include "reduce_dev.h"
 
 #include <algorithm>
 #include <cmath>
@@ -83,30 +84,6 @@ constexpr int RED_Z_BLOCKS = 256;
 constexpr int RED_Z_STRIDE = 1 + 2 * RED_MAXQ;
 constexpr int EZ_THREADS = 1024;
 constexpr int EZ_CHUNK_BITS = 13;   // 1024 threads x 8 amplitudes
-
-// Sum over the 64 lanes of each of the N columns v[0..N) (N <= 64); lane L
-// returns column bitreverse6(L).  Every step folds pairs of columns into one,
-// each half of the wave keeping one of the pair: N shuffles instead of 6 N.
-template <int N, int M>
-__device__ __forceinline__ double wave_columns(double* v, int lane)
-{
-    if constexpr (M == 0) {
-        return v[0];
-    } else {
-        const bool up = (lane & M) != 0;
-#pragma unroll
-        for (int i = 0; i < (N + 1) / 2; i++) {
-            if (2 * i + 1 < N) {
-                const double keep = up ? v[2 * i + 1] : v[2 * i];
-                const double send = up ? v[2 * i] : v[2 * i + 1];
-                v[i] = keep + __shfl_xor(send, M);
-            } else {
-                v[i] = v[2 * i] + __shfl_xor(v[2 * i], M);
-            }
-        }
-        return wave_columns<(N + 1) / 2, M / 2>(v, lane);
-    }
-}
 
 // One row of partials per block, one read of the state.  HBM-bound by
 // construction: an index bit's weight is a constant of the place that holds
@@ -354,6 +331,33 @@ static hq_status ensure_red(hq_state s, size_t doubles)
     return HQ_OK;
 }
 
+// The state's readout workspace: at least `dev` bytes of device and `host` bytes
+// of pinned memory, kept for the next readout.
+hq_status ensure_ws(hq_state s, size_t dev, size_t host)
+{
+    if (s->ws_dev < dev) {
+        if (s->d_ws) (void)hipFree(s->d_ws);
+        s->d_ws = nullptr;
+        s->ws_dev = 0;
+        HQ_HIP(hipMalloc((void**)&s->d_ws, dev));
+        s->ws_dev = dev;
+    }
+    if (s->ws_host < host) {
+        if (s->h_ws) (void)hipHostFree(s->h_ws);
+        s->h_ws = nullptr;
+        s->ws_host = 0;
+        HQ_HIP(hipHostMalloc((void**)&s->h_ws, host, hipHostMallocDefault));
+        s->ws_host = host;
+    }
+    return HQ_OK;
+}
+
+void trim_ws(hq_state s, size_t keep)
+{
+    if (s->ws_dev > keep) { (void)hipFree(s->d_ws); s->d_ws = nullptr; s->ws_dev = 0; }
+    if (s->ws_host > keep) { (void)hipHostFree(s->h_ws); s->h_ws = nullptr; s->ws_host = 0; }
+}
+
 static unsigned grid_for(uint64_t work, unsigned threads, unsigned cap)
 {
     uint64_t g = (work + threads - 1) / threads;
@@ -458,6 +462,8 @@ hq_status hq_state_destroy(hq_state s)
     if (s->buf) (void)hipFree(s->buf);
     if (s->d_red) (void)hipFree(s->d_red);
     if (s->h_red) (void)hipHostFree(s->h_red);
+    if (s->d_ws) (void)hipFree(s->d_ws);
+    if (s->h_ws) (void)hipHostFree(s->h_ws);
     for (auto& e : s->prof) { (void)hipEventDestroy(e.start); (void)hipEventDestroy(e.stop); }
     for (auto& e : s->free_events) (void)hipEventDestroy(e);
     if (s->stream) (void)hipStreamDestroy(s->stream);

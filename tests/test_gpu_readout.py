@@ -53,3 +53,49 @@ def test_expect_z_largest_loop(gpu):
     # single-precision gates: one rounding of 6e-8 per coefficient and product, 15 gates
     assert np.max(np.abs(z - want)) <= 5e-6
     assert np.max(np.abs(zz - want[:-1] * want[1:])) <= 5e-6
+
+
+def _draws(p, shots, seed):
+    """The documented draw: the smallest index whose cumulative probability exceeds u * total."""
+    from helpers import Rng
+    cdf = np.cumsum(p)
+    r = Rng(seed)
+    u = np.array([r.uniform() for _ in range(shots)])
+    return np.searchsorted(cdf, u * cdf[-1], side="right")
+
+
+# one part, one chunk, several chunks, more than one and two steps of the 64-way prefix search
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [1, 5, 6, 11, 12, 13, 18, 19, 22])
+def test_sample_searches(gpu, n, prec):
+    s, p = _state(gpu, n, prec, 3)
+    assert np.array_equal(s.sample(5000, 21).astype(np.int64), _draws(p, 5000, 21))
+    s.close()
+
+
+def test_sample_sparse_and_batches(gpu):
+    """A state with 9 nonzero amplitudes (first and last of parts and chunks)
+    and more shots than one launch takes."""
+    n = 15
+    idx = np.array([0, 63, 64, 4095, 4096, 9000, 20479, 20480, (1 << n) - 1])
+    psi = np.zeros(1 << n, np.complex128)
+    psi[idx] = np.sqrt(np.arange(1, 10) / 45.0)
+    s = gpu.State(n)
+    s.upload(psi)
+    shots = (1 << 18) + 7
+    got = s.sample(shots, 5).astype(np.int64)
+    assert np.array_equal(got, _draws(np.abs(psi) ** 2, shots, 5))
+    assert set(got.tolist()) <= set(idx.tolist())
+    s.close()
+
+
+def test_sample_without_part_sums(gpu):
+    """30 qubits: a wave sums the parts of its chunk itself.  H on three qubits
+    of |0...0>: eight outcomes of probability 1/8 (to float rounding)."""
+    n = 30
+    s = gpu.State(n, gpu.HQ_C64)
+    s.apply_plain([gpu.Gate.H(q) for q in (0, 13, 29)])
+    got = s.sample(4000, 9).astype(np.int64)
+    s.close()
+    out = np.array([a | b << 13 | c << 29 for c in (0, 1) for b in (0, 1) for a in (0, 1)])
+    assert np.array_equal(got, out[_draws(np.full(8, 0.125), 4000, 9)])
