@@ -64,6 +64,7 @@ struct TopkItem {
     uint64_t count;        // elements in src
     uint64_t dst;          // 16 candidates per block
     uint64_t first_block;
+    uint64_t chunk;        // elements per block
     uint32_t kind, pad;
 };
 
@@ -116,90 +117,188 @@ __device__ __forceinline__ bool better(double pa, uint64_t ia, double pb, uint64
     return pa > pb || (pa == pb && ia < ib);
 }
 
-__device__ __forceinline__ void wave_best(double& p, uint64_t& i)
+constexpr int TOPK = 16;
+constexpr int TOPK_MIN_CHUNK = 4096;   // elements per block: 256 threads x 16 ...
+constexpr int TOPK_MAX_BLOCKS = 1024;  // ... up to this many blocks, then longer chunks
+
+__device__ __forceinline__ double read_lane(double v, int lane)
 {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t u, int lane)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return (uint64_t)hi << 32 | lo;
+}
+
+// the value of the lane below, within rows of 16 lanes
+__device__ __forceinline__ double lane_below(double v)
+{
+    const long long u = __double_as_longlong(v);
+    const int lo = (int)(uint32_t)u, hi = (int)(uint32_t)((uint64_t)u >> 32);
+    const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(lo, lo, 0x111 /* row_shr:1 */, 0xf, 0xf, false);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_update_dpp(hi, hi, 0x111, 0xf, 0xf, false);
+    return __longlong_as_double((long long)((uint64_t)h << 32 | l));
+}
+__device__ __forceinline__ uint64_t lane_below(uint64_t u)
+{
+    return (uint64_t)__double_as_longlong(lane_below(__longlong_as_double((long long)u)));
+}
+
+// The 16 best so far of what a wave has seen, in order, one per lane 0..15,
+// and the last of them as the bar an element has to pass.
+struct WaveTop {
+    double p = -1.0;
+    uint64_t i = ~0ull;
+    double bar_p = -1.0;
+    uint64_t bar_i = ~0ull;
+
+    // the elements (q, e) of the lanes where `may`: those that pass the bar
+    // inserted one by one
+    __device__ __forceinline__ void offer(double q, uint64_t e, bool may, int lane)
+    {
+        uint64_t m = __ballot(may && better(q, e, bar_p, bar_i));
+        while (m) {
+            const int f = __builtin_ctzll(m);
+            const double np = read_lane(q, f);
+            const uint64_t ni = read_lane(e, f);
+            // lanes the new element goes before move up by one
+            const bool after = better(np, ni, p, i);
+            const double up_p = lane_below(p);
+            const uint64_t up_i = lane_below(i);
+            const int at = __builtin_ctzll(__ballot(after));
+            if (after) { p = lane == at ? np : up_p; i = lane == at ? ni : up_i; }
+            bar_p = read_lane(p, TOPK - 1);
+            bar_i = read_lane(i, TOPK - 1);
+            m &= m - 1;
+            m &= __ballot(better(q, e, bar_p, bar_i));
+        }
+    }
+};
+
+// The 16 best (p, idx) of a chunk, in order; empty slots hold p = -1.  A pass
+// over n amplitudes offers each to its wave's list, which takes it only if it
+// beats the 16th: about 16 (1 + ln(n / 16)) do, so the pass is a read of the
+// state (28 qubits complex64, 2 GiB: 0.49 ms; selecting 16 times from every
+// 4096 elements took 2.1 ms).  Applied to the blocks' results once more.
+template <typename R>
+__device__ __forceinline__ void topk_chunk(const TopkItem& it, uint64_t chunk)
+{
+    const uint32_t t = threadIdx.x;
+    const int lane = (int)(t & 63), w = (int)(t >> 6);
+    const uint64_t e0 = chunk * it.chunk;
+    const uint64_t e1 = e0 + it.chunk < it.count ? e0 + it.chunk : it.count;
+    constexpr int U = 8;                 // elements per lane and step
+    constexpr bool PAIR = sizeof(R) == 4;
+    struct alignas(16) Two { cplx<R> v[PAIR ? 2 : 1]; };
+    WaveTop top;
+    bool first = true;
+    for (uint64_t b = e0 + (uint64_t)w * (64 * U); b < e1; b += 4 * 64 * U) {
+        double q[U];
+        uint64_t e[U];
+        if (it.kind == 0) {
+            if constexpr (PAIR) {
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        double op = __shfl_xor(p, o);
-        uint64_t oi = __shfl_xor(i, o);
-        if (better(op, oi, p, i)) { p = op; i = oi; }
+                for (int u = 0; u < U / 2; u++) {
+                    const uint64_t x = b + (uint64_t)(u * 128 + 2 * lane);
+                    Two v = {};
+                    const bool in = x < e1;      // counts are even
+                    if (in) v = *(const Two*)((const cplx<R>*)it.src + x);
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const double re = (double)v.v[h].x, im = (double)v.v[h].y;
+                        q[2 * u + h] = in ? re * re + im * im : -1.0;
+                        e[2 * u + h] = in ? x + (uint64_t)h : ~0ull;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const uint64_t x = b + (uint64_t)(u * 64 + lane);
+                    cplx<R> v = {};
+                    const bool in = x < e1;
+                    if (in) v = ((const cplx<R>*)it.src)[x];
+                    q[u] = in ? (double)v.x * (double)v.x + (double)v.y * (double)v.y : -1.0;
+                    e[u] = in ? x : ~0ull;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint64_t x = b + (uint64_t)(u * 64 + lane);
+                q[u] = -1.0;
+                e[u] = ~0ull;
+                if (x < e1) {
+                    const Cand c = ((const Cand*)it.src)[x];
+                    q[u] = c.p;
+                    e[u] = c.idx;
+                }
+            }
+        }
+        // of a wave's first elements only those that can be among its 16 best
+        // are offered: the bar is searched bit by bit in the upper halves of
+        // the probabilities (inserting one element costs as much as some
+        // three such steps, and 70 of 512 would beat a bar that starts at 0)
+        int key[U], cut = 0;
+        if (first) {
+            first = false;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int h = (int)(uint32_t)((uint64_t)__double_as_longlong(q[u]) >> 32);
+                key[u] = q[u] >= 0 ? h : -1;       // (not: empty, NaN)
+            }
+            for (int bit = 30; bit >= 0; bit--) {
+                const int t = cut | (1 << bit);
+                int n = 0;
+#pragma unroll
+                for (int u = 0; u < U; u++) n += (int)__popcll(__ballot(key[u] >= t));
+                if (n >= TOPK) cut = t;
+                if (n == TOPK) break;
+            }
+        } else {
+            double best = q[0];
+#pragma unroll
+            for (int u = 1; u < U; u++) best = q[u] > best ? q[u] : best;
+            if (!__ballot(best >= top.bar_p)) continue;
+#pragma unroll
+            for (int u = 0; u < U; u++) key[u] = 0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) top.offer(q[u], e[u], key[u] >= cut, lane);
+    }
+    // the waves' lists: each entry's place is the number of entries before it
+    __shared__ double sp[4 * TOPK];
+    __shared__ uint64_t si[4 * TOPK];
+    if (lane < TOPK) { sp[w * TOPK + lane] = top.p; si[w * TOPK + lane] = top.i; }
+    __syncthreads();
+    if (w == 0) {
+        const double mp = sp[lane];
+        const uint64_t mi = si[lane];
+        int rank = 0;
+        for (int k = 0; k < 4 * TOPK; k++) {
+            const bool same = sp[k] == mp && si[k] == mi;      // empty slots: by position
+            rank += better(sp[k], si[k], mp, mi) || (same && k < lane) ? 1 : 0;
+        }
+        if (rank < TOPK) ((Cand*)it.dst)[chunk * TOPK + rank] = Cand{mp, mi};
     }
 }
 
-constexpr int TOPK = 16;
-constexpr int TOPK_CHUNK = 4096;  // elements per block: 256 threads x 16
-
-// 16 best (p, idx) of each 4096-element chunk, in order.  Empty slots hold
-// p = -1.  Applied level by level until one chunk remains.
 template <typename R>
 __global__ __launch_bounds__(256) void k_topk(const TopkItem* __restrict__ items, uint32_t count)
 {
     const uint64_t b = blockIdx.x;
-    const TopkItem* it = items + find_item(items, count, b);
-    const uint64_t chunk = b - it->first_block;
-    const uint64_t e0 = chunk * TOPK_CHUNK;
-    const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
-    double p[16];
-    uint64_t id[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const uint64_t e = e0 + (uint64_t)j * 256 + t;
-        p[j] = -1.0;
-        id[j] = ~0ull;
-        if (e < it->count) {
-            if (it->kind == 0) {
-                const cplx<R> a = ((const cplx<R>*)it->src)[e];
-                const double re = (double)a.x, im = (double)a.y;
-                p[j] = re * re + im * im;
-                id[j] = e;
-            } else {
-                const Cand c = ((const Cand*)it->src)[e];
-                p[j] = c.p;
-                id[j] = c.idx;
-            }
-        }
-    }
-    double kp = -1.0;
-    uint64_t ki = ~0ull;
-    for (int r = 0; r < TOPK; r++) {
-        double bp = p[0];
-        uint64_t bi = id[0];
-        int bj = 0;
-#pragma unroll
-        for (int j = 1; j < 16; j++)
-            if (better(p[j], id[j], bp, bi)) { bp = p[j]; bi = id[j]; bj = j; }
-        double wp = bp;
-        uint64_t wi = bi;
-        wave_best(wp, wi);
-        if (bp == wp && bi == wi) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) if (j == bj) p[j] = -2.0;
-        }
-        if (lane == (uint32_t)r) { kp = wp; ki = wi; }
-    }
-    __shared__ double sp[64];
-    __shared__ uint64_t si[64];
-    if (lane < TOPK) { sp[w * TOPK + lane] = kp; si[w * TOPK + lane] = ki; }
-    __syncthreads();
-    if (w == 0) {
-        double q = sp[lane];
-        uint64_t qi = si[lane];
-        double op = -1.0;
-        uint64_t oi = ~0ull;
-        for (int r = 0; r < TOPK; r++) {
-            double wp = q;
-            uint64_t wi = qi;
-            wave_best(wp, wi);
-            if (q == wp && qi == wi) q = -2.0;
-            if (lane == (uint32_t)r) { op = wp; oi = wi; }
-        }
-        if (lane < TOPK) {
-            Cand c;
-            c.p = op < 0 ? -1.0 : op;
-            c.idx = oi;
-            ((Cand*)it->dst)[chunk * TOPK + lane] = c;
-        }
-    }
+    const TopkItem it = items[find_item(items, count, b)];
+    topk_chunk<R>(it, b - it.first_block);
+}
+
+template <typename R>
+__global__ __launch_bounds__(256) void k_topk_one(TopkItem it)
+{
+    topk_chunk<R>(it, blockIdx.x);
 }
 
 // ---- launch dispatch -----------------------------------------------------------------------
@@ -634,7 +733,7 @@ struct Job {
     enum Status { QUEUED, COMPILED, ADMITTED, DONE, FAILED } status = QUEUED;
     std::string error;
     std::vector<Block> blocks;
-    uint64_t d_blob = 0, d_state = 0, d_part = 0, d_cand[2] = {0, 0};
+    uint64_t d_blob = 0, d_state = 0, d_part = 0, d_cand = 0;
     int next_group = 0;
     double t_submit = 0, t_admit = 0, t_done = 0;
     double res[3] = {0, 0, 0};
@@ -646,18 +745,19 @@ struct Job {
     bool needs_state() const { return plan.groups.size() > 1 || wants_topk(); }
 };
 
-// top-k levels: element counts per level (the last level has one chunk)
-static std::vector<uint64_t> topk_levels(uint64_t elems)
+// Passes of the top-k over `elems` amplitudes: elements and elements per block
+// of each (the second, over at most 1024 x 16 candidates, is one block).
+struct TopkLevel {
+    uint64_t count, chunk;
+    uint64_t blocks() const { return (count + chunk - 1) / chunk; }
+};
+static std::vector<TopkLevel> topk_levels(uint64_t elems)
 {
-    std::vector<uint64_t> lv;
-    uint64_t c = elems;
-    for (;;) {
-        lv.push_back(c);
-        uint64_t blocks = (c + TOPK_CHUNK - 1) / TOPK_CHUNK;
-        if (blocks <= 1) break;
-        c = blocks * TOPK;
-    }
-    return lv;
+    TopkLevel l{elems, TOPK_MIN_CHUNK};
+    while (l.blocks() > TOPK_MAX_BLOCKS) l.chunk *= 2;
+    if (l.blocks() == 1) return {l};
+    const uint64_t cand = l.blocks() * TOPK;
+    return {l, TopkLevel{cand, cand}};
 }
 
 struct LaunchDesc {
@@ -754,7 +854,7 @@ static void build_round(const std::vector<Job*>& jobs, uint64_t res_dev, RoundBu
     rb->launches.push_back(d);
     // top-k, level by level across the finishing circuits
     size_t max_levels = 0;
-    std::vector<std::vector<uint64_t>> lv(rb->finishing.size());
+    std::vector<std::vector<TopkLevel>> lv(rb->finishing.size());
     for (size_t i = 0; i < rb->finishing.size(); i++) {
         if (!rb->finishing[i]->wants_topk()) continue;
         lv[i] = topk_levels(1ull << rb->finishing[i]->n);
@@ -769,11 +869,12 @@ static void build_round(const std::vector<Job*>& jobs, uint64_t res_dev, RoundBu
             TopkItem t;
             t.kind = L == 0 ? 0 : 1;
             t.pad = 0;
-            t.src = L == 0 ? j->d_state : j->d_cand[(L - 1) & 1];
-            t.count = lv[i][L];
-            t.dst = L + 1 == lv[i].size() ? res_dev + i * RES_BYTES + 64 : j->d_cand[L & 1];
+            t.src = L == 0 ? j->d_state : j->d_cand;
+            t.count = lv[i][L].count;
+            t.chunk = lv[i][L].chunk;
+            t.dst = L + 1 == lv[i].size() ? res_dev + i * RES_BYTES + 64 : j->d_cand;
             t.first_block = blocks;
-            blocks += (t.count + TOPK_CHUNK - 1) / TOPK_CHUNK;
+            blocks += lv[i][L].blocks();
             items.push_back(t);
         }
         LaunchDesc t{2, 0, 0, table_append(rb->table, items.data(), items.size() * sizeof(TopkItem)),
@@ -856,26 +957,25 @@ static hq_status issue_round(const RoundBuild& rb, uint64_t table_dev, int preci
 
 // device bytes a job needs: programs, state, partials, top-k candidates
 static void job_sizes(const Job& j, int precision, uint64_t* blob, uint64_t* state, uint64_t* part,
-                      uint64_t* cand0, uint64_t* cand1)
+                      uint64_t* cand)
 {
     const uint64_t amp = precision == HQ_C128 ? 16 : 8;
     *blob = j.plan.blobs.size();
     *state = j.needs_state() ? (1ull << j.n) * amp : 0;
     *part = j.tiles_last() * 3 * sizeof(double);
-    *cand0 = *cand1 = 0;
+    *cand = 0;
     if (j.wants_topk()) {
         auto lv = topk_levels(1ull << j.n);
-        if (lv.size() > 1) *cand0 = lv[1] * sizeof(Cand);
-        if (lv.size() > 2) *cand1 = lv[2] * sizeof(Cand);
+        if (lv.size() > 1) *cand = lv[1].count * sizeof(Cand);
     }
 }
 
 static bool job_alloc(Job* j, Arena& a, int precision)
 {
-    uint64_t sz[5];
-    job_sizes(*j, precision, &sz[0], &sz[1], &sz[2], &sz[3], &sz[4]);
-    uint64_t* dst[5] = {&j->d_blob, &j->d_state, &j->d_part, &j->d_cand[0], &j->d_cand[1]};
-    for (int i = 0; i < 5; i++) {
+    uint64_t sz[4];
+    job_sizes(*j, precision, &sz[0], &sz[1], &sz[2], &sz[3]);
+    uint64_t* dst[4] = {&j->d_blob, &j->d_state, &j->d_part, &j->d_cand};
+    for (int i = 0; i < 4; i++) {
         *dst[i] = 0;
         if (!sz[i]) continue;
         Block b;
@@ -892,8 +992,8 @@ static bool job_alloc(Job* j, Arena& a, int precision)
 
 static uint64_t job_bytes(const Job& j, int precision, uint64_t* largest)
 {
-    uint64_t sz[5], t = 0;
-    job_sizes(j, precision, &sz[0], &sz[1], &sz[2], &sz[3], &sz[4]);
+    uint64_t sz[4], t = 0;
+    job_sizes(j, precision, &sz[0], &sz[1], &sz[2], &sz[3]);
     *largest = 0;
     for (uint64_t s : sz)
         if (s) { t += 1ull << Arena::order_of(s); *largest = std::max(*largest, s); }
@@ -1634,40 +1734,29 @@ hq_status hq_state_topk(hq_state s, int k, uint64_t* idx, double* prob)
 {
     HQ_CHECK(s && (idx || prob), HQ_ERR_ARG, "hq_state_topk: null argument");
     HQ_CHECK(k >= 1 && k <= TOPK, HQ_ERR_ARG, "hq_state_topk: k must be in [1, 16]");
-    auto lv = topk_levels(s->amps);
-    size_t c0 = lv.size() > 1 ? lv[1] : 0, c1 = lv.size() > 2 ? lv[2] : 0;
-    char* d = nullptr;
-    const size_t bytes = (c0 + c1 + TOPK) * sizeof(Cand) + lv.size() * sizeof(TopkItem) + 1024;
-    HQ_HIP(hipMalloc((void**)&d, bytes));
-    Cand* cand[2] = {(Cand*)d, (Cand*)d + c0};
-    Cand* fin = (Cand*)d + c0 + c1;
-    TopkItem* items = (TopkItem*)(((uintptr_t)(fin + TOPK) + 63) & ~(uintptr_t)63);
-    std::vector<TopkItem> h(lv.size());
+    const auto lv = topk_levels(s->amps);
+    const size_t cand = lv.size() > 1 ? lv[1].count * sizeof(Cand) : 0;
+    // candidates stay on the device, the result goes straight to pinned memory
+    hq_status st = ensure_ws(s, cand, TOPK * sizeof(Cand));
+    if (st != HQ_OK) return st;
+    const Cand* res = (const Cand*)s->h_ws;
     for (size_t L = 0; L < lv.size(); L++) {
-        h[L].kind = L == 0 ? 0 : 1;
-        h[L].pad = 0;
-        h[L].src = L == 0 ? (uint64_t)(uintptr_t)s->data : (uint64_t)(uintptr_t)cand[(L - 1) & 1];
-        h[L].count = lv[L];
-        h[L].dst = L + 1 == lv.size() ? (uint64_t)(uintptr_t)fin : (uint64_t)(uintptr_t)cand[L & 1];
-        h[L].first_block = 0;
-    }
-    hipError_t e = hipMemcpyAsync(items, h.data(), h.size() * sizeof(TopkItem), hipMemcpyHostToDevice, s->stream);
-    for (size_t L = 0; L < lv.size() && e == hipSuccess; L++) {
-        const unsigned blocks = (unsigned)((lv[L] + TOPK_CHUNK - 1) / TOPK_CHUNK);
+        TopkItem it;
+        it.src = (uint64_t)(uintptr_t)(L == 0 ? s->data : (void*)s->d_ws);
+        it.count = lv[L].count;
+        it.chunk = lv[L].chunk;
+        it.dst = (uint64_t)(uintptr_t)(L + 1 == lv.size() ? s->h_ws : s->d_ws);
+        it.first_block = 0;
+        it.kind = L == 0 ? 0 : 1;
+        it.pad = 0;
+        const unsigned blocks = (unsigned)lv[L].blocks();
         if (s->precision == HQ_C128)
-            hipLaunchKernelGGL(k_topk<double>, dim3(blocks), dim3(256), 0, s->stream, items + L, 1u);
+            hipLaunchKernelGGL(k_topk_one<double>, dim3(blocks), dim3(256), 0, s->stream, it);
         else
-            hipLaunchKernelGGL(k_topk<float>, dim3(blocks), dim3(256), 0, s->stream, items + L, 1u);
-        e = hipGetLastError();
+            hipLaunchKernelGGL(k_topk_one<float>, dim3(blocks), dim3(256), 0, s->stream, it);
+        HQ_HIP(hipGetLastError());
     }
-    Cand res[TOPK];
-    if (e == hipSuccess) e = hipMemcpyAsync(res, fin, sizeof(res), hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    (void)hipFree(d);
-    if (e != hipSuccess) {
-        set_error(std::string("hq_state_topk: ") + hipGetErrorString(e));
-        return HQ_ERR_HIP;
-    }
+    HQ_HIP(hipStreamSynchronize(s->stream));
     for (int i = 0; i < k; i++) {
         if (idx) idx[i] = res[i].idx;
         if (prob) prob[i] = res[i].p;

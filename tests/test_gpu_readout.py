@@ -99,3 +99,24 @@ def test_sample_without_part_sums(gpu):
     s.close()
     out = np.array([a | b << 13 | c << 29 for c in (0, 1) for b in (0, 1) for a in (0, 1)])
     assert np.array_equal(got, out[_draws(np.full(8, 0.125), 4000, 9)])
+
+
+# one block, several, and (2^23 amplitudes) chunks longer than 4096
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [1, 3, 4, 9, 12, 13, 17, 23])
+def test_topk_lists(gpu, n, prec):
+    s, p = _state(gpu, n, prec, 4)
+    k = min(16, 1 << n)
+    idx, prob = s.topk(k)
+    order = np.lexsort((np.arange(1 << n), -p))[:k]
+    assert list(idx) == order.tolist()
+    np.testing.assert_allclose(prob, p[order], rtol=1e-14)
+    # few nonzero amplitudes: the rest of the list are the smallest indices of probability 0
+    if n >= 9:
+        psi = np.zeros(1 << n, np.complex128 if prec == 0 else np.complex64)
+        psi[[5, (1 << n) - 1, 300]] = [0.5, 0.5, 0.25]
+        s.upload(psi)
+        idx, prob = s.topk(16)
+        assert list(idx) == [5, (1 << n) - 1, 300, 0, 1, 2, 3, 4, 6, 7, 8, 9, 10, 11, 12, 13]
+        assert prob[3:] == [0.0] * 13
+    s.close()
