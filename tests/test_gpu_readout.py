@@ -120,3 +120,13 @@ def test_topk_lists(gpu, n, prec):
         assert list(idx) == [5, (1 << n) - 1, 300, 0, 1, 2, 3, 4, 6, 7, 8, 9, 10, 11, 12, 13]
         assert prob[3:] == [0.0] * 13
     s.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [1, 2, 9, 10, 13, 20, 21])
+def test_norm_and_measure_elements(gpu, n, prec):
+    s, p = _state(gpu, n, prec, 8)
+    assert abs(s.norm2() - p.sum()) <= 1e-13
+    for q in sorted({0, min(1, n - 1), n // 2, n - 1}):
+        assert abs(s.measure_zero(q) - p.reshape(-1, 2, 1 << q)[:, 0].sum()) <= 1e-13, (n, q)
+    s.close()
