@@ -18,31 +18,42 @@ namespace {
 
 int popc(qindex x) { return __builtin_popcountll((unsigned long long)x); }
 
+// A set of gates of the window; W words on the stack.
+template <int W>
 struct Bits {
-    std::vector<uint64_t> w;
-    explicit Bits(int nbits = 0) : w((nbits + 63) / 64, 0) {}
+    uint64_t w[W] = {};
     void set(int i) { w[i >> 6] |= 1ull << (i & 63); }
     bool test(int i) const { return (w[i >> 6] >> (i & 63)) & 1; }
-    int count() const
+    // the first `used` words hold every bit
+    int count(int used) const
     {
         int c = 0;
-        for (auto x : w) c += __builtin_popcountll(x);
+        for (int i = 0; i < used; i++) c += __builtin_popcountll(w[i]);
         return c;
     }
-    bool any() const
+    bool any(int used) const
     {
-        for (auto x : w) if (x) return true;
+        for (int i = 0; i < used; i++)
+            if (w[i]) return true;
         return false;
     }
-    void orWith(const Bits& o) { for (size_t i = 0; i < w.size(); i++) w[i] |= o.w[i]; }
-    void andNot(const Bits& o) { for (size_t i = 0; i < w.size(); i++) w[i] &= ~o.w[i]; }
+    void orWith(const Bits& o, int used) { for (int i = 0; i < used; i++) w[i] |= o.w[i]; }
+    void andNot(const Bits& o, int used) { for (int i = 0; i < used; i++) w[i] &= ~o.w[i]; }
 };
 
 }  // namespace
 
 GroupFinder::GroupFinder(int numQubits, const std::vector<Gate>& gates, int window)
-    : n_(numQubits), window_(window), gates_(gates)
+    : n_(numQubits), window_(window)
 {
+    // what the search reads of a gate, 8 bytes instead of a Gate: the search
+    // walks the window's gates thousands of times
+    auto brief = std::make_shared<std::vector<Brief>>(gates.size());
+    for (size_t i = 0; i < gates.size(); i++) {
+        const Gate& g = gates[i];
+        (*brief)[i] = Brief{(int8_t)g.targetQubit, (int8_t)g.controlQubit, (int8_t)g.controlQubit2, g.isDiagonal()};
+    }
+    gates_ = brief;
     remain_.resize(gates.size());
     for (size_t i = 0; i < gates.size(); i++) remain_[i] = (int)i;
 }
@@ -64,127 +75,136 @@ std::vector<std::vector<int>> GroupFinder::findAll(std::vector<char>& full, std:
                                                    bool enableGlobal, int localSize, qindex localQubits,
                                                    int starts) const
 {
+    // 8 words hold the default window; 64 the largest the option takes
+    return window_ <= 512 ? findAllIn<8>(full, related, enableGlobal, localSize, localQubits, starts)
+                          : findAllIn<64>(full, related, enableGlobal, localSize, localQubits, starts);
+}
+
+// GateGroup::newRelated on a Brief
+qindex GroupFinder::withGate(qindex rel, const Brief& g, qindex localQubits, bool enableGlobal)
+{
+    if (enableGlobal) return g.diagonal ? rel : rel | qindex(1) << g.t;
+    if (!g.diagonal || ((localQubits >> g.t) & 1)) rel |= qindex(1) << g.t;
+    if (g.c != -1 && ((localQubits >> g.c) & 1)) rel |= qindex(1) << g.c;
+    if (g.c2 != -1 && ((localQubits >> g.c2) & 1)) rel |= qindex(1) << g.c2;
+    return rel;
+}
+
+template <int W>
+std::vector<std::vector<int>> GroupFinder::findAllIn(std::vector<char>& full, std::vector<qindex>& related,
+                                                     bool enableGlobal, int localSize, qindex localQubits,
+                                                     int starts) const
+{
     const int n = n_;
+    const std::vector<Brief>& gates = *gates_;
     const int gate_num = std::min<int>((int)remain_.size(), window_);
-    std::vector<Bits> cur(n, Bits(gate_num));
-    Bits selected(gate_num);
+    const uint64_t all = n >= 64 ? ~0ull : (1ull << n) - 1;
+    std::vector<Bits<W>> cur(n);
+    int used = 1;   // words of the window the chains reach into
 
     // 1. per-qubit chains of gates that can join the group
-    for (int id = 0; id < gate_num; id++) {
-        if (id % 100 == 0) {
-            bool live = false;
-            for (int i = 0; i < n; i++) if (!full[i]) live = true;
-            if (!live) break;
-        }
-        const Gate& g = gates_[remain_[id]];
-        if (g.isControlGate()) {
-            const int c = g.controlQubit, t = g.targetQubit, c2 = g.controlQubit2;
-            if (!full[c] && !full[t] && (c2 < 0 || !full[c2])) {
-                qindex nr = related[c] | related[t] | (c2 >= 0 ? related[c2] : 0);
-                nr = GateGroup::newRelated(nr, g, localQubits, enableGlobal);
+    uint64_t fullMask = 0;
+    for (int i = 0; i < n; i++)
+        if (full[i]) fullMask |= 1ull << i;
+    for (int id = 0; id < gate_num && fullMask != all; id++) {
+        const Brief g = gates[remain_[id]];
+        const uint64_t bits = 1ull << g.t | (g.c >= 0 ? 1ull << g.c : 0) | (g.c2 >= 0 ? 1ull << g.c2 : 0);
+        if (g.c >= 0) {
+            if (!(fullMask & bits)) {
+                qindex nr = related[g.c] | related[g.t] | (g.c2 >= 0 ? related[g.c2] : 0);
+                nr = withGate(nr, g, localQubits, enableGlobal);
                 if (popc(nr) <= localSize) {
-                    Bits nc = cur[c];
-                    nc.orWith(cur[t]);
-                    if (c2 >= 0) nc.orWith(cur[c2]);
+                    used = (id >> 6) + 1;
+                    Bits<W>& nc = cur[g.c];
+                    nc.orWith(cur[g.t], used);
+                    if (g.c2 >= 0) nc.orWith(cur[g.c2], used);
                     nc.set(id);
-                    cur[c] = nc;
-                    cur[t] = nc;
-                    if (c2 >= 0) cur[c2] = nc;
-                    related[c] = related[t] = nr;
-                    if (c2 >= 0) related[c2] = nr;
+                    cur[g.t] = nc;
+                    if (g.c2 >= 0) cur[g.c2] = nc;
+                    related[g.c] = related[g.t] = nr;
+                    if (g.c2 >= 0) related[g.c2] = nr;
                     continue;
                 }
             }
-            full[c] = full[t] = 1;
-            if (c2 >= 0) full[c2] = 1;
-        } else {
-            if (!full[g.targetQubit]) {
-                cur[g.targetQubit].set(id);
-                related[g.targetQubit] = GateGroup::newRelated(related[g.targetQubit], g, localQubits, enableGlobal);
-            }
+            fullMask |= bits;
+        } else if (!(fullMask & bits)) {
+            used = (id >> 6) + 1;
+            cur[g.t].set(id);
+            related[g.t] = withGate(related[g.t], g, localQubits, enableGlobal);
         }
     }
+    for (int i = 0; i < n; i++)
+        if ((fullMask >> i) & 1) full[i] = 1;
 
     // 2. greedily merge the longest chains that fit.  With starts > 1 the
     // merge is repeated with each of the `starts` longest chains taken first,
     // and the largest group wins (a one-group lookahead; starts = 1 is the
     // reference's rule).
-    auto merge = [&](int first, Bits& sel) {
-        std::vector<Bits> cc = cur;
-        std::vector<char> blocked(n, 0);
+    auto merge = [&](int first, Bits<W>& sel) {
+        std::vector<Bits<W>> cc = cur;
+        uint64_t blocked = 0;
         qindex selRel = 0;
         bool forced = first >= 0;
         while (true) {
             int mx = 0, best = -1;
             if (forced) {
                 best = first;
-                mx = cc[first].count();
+                mx = cc[first].count(used);
                 forced = false;
             } else {
                 for (int i = 0; i < n; i++) {
-                    int cnt = cc[i].count();
-                    if (!blocked[i] && cnt > mx) {
+                    if ((blocked >> i) & 1) continue;
+                    const int cnt = cc[i].count(used);
+                    if (cnt > mx) {
                         if (popc(selRel | related[i]) <= localSize) { mx = cnt; best = i; }
-                        else blocked[i] = 1;
+                        else blocked |= 1ull << i;
                     }
                 }
             }
             if (mx == 0) break;
-            sel.orWith(cc[best]);
+            sel.orWith(cc[best], used);
             selRel |= related[best];
-            blocked[best] = 1;
+            blocked |= 1ull << best;
             for (int i = 0; i < n; i++) {
-                if (!blocked[i] && cc[i].any()) {
-                    if ((related[i] | selRel) == selRel) {
-                        sel.orWith(cc[i]);
-                        blocked[i] = 1;
-                    } else {
-                        cc[i].andNot(cc[best]);
-                    }
+                if (((blocked >> i) & 1) || !cc[i].any(used)) continue;
+                if ((related[i] | selRel) == selRel) {
+                    sel.orWith(cc[i], used);
+                    blocked |= 1ull << i;
+                } else {
+                    cc[i].andNot(cc[best], used);
                 }
             }
         }
     };
-    std::vector<Bits> cands;
-    merge(-1, selected);
-    cands.push_back(selected);
+    std::vector<Bits<W>> cands(1);
+    merge(-1, cands[0]);
     if (starts > 1) {
-        std::vector<int> order;
-        for (int i = 0; i < n; i++)
-            if (cur[i].any() && popc(related[i]) <= localSize) order.push_back(i);
-        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cur[a].count() > cur[b].count(); });
+        std::vector<int> order, len(n);
+        for (int i = 0; i < n; i++) {
+            len[i] = cur[i].count(used);
+            if (len[i] && popc(related[i]) <= localSize) order.push_back(i);
+        }
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return len[a] > len[b]; });
         for (int k = 1; k < starts && k < (int)order.size(); k++) {
-            Bits sel(gate_num);
+            Bits<W> sel;
             merge(order[k], sel);
             cands.push_back(sel);
         }
     }
-    std::vector<char> blocked(n, 0);
 
-    // 3. diagonal gates that commute into the group (OShareMem only)
-    auto sweep = [&](Bits& sel) {
-        std::fill(blocked.begin(), blocked.end(), 0);
-        int cnt = 0;
-        for (int id = 0; id < gate_num; id++) {
-            cnt++;
-            if (cnt % 100 == 0) {
-                bool live = false;
-                for (int i = 0; i < n; i++) if (!blocked[i]) live = true;
-                if (!live) break;
-            }
+    // 3. diagonal gates that commute into the group (OShareMem only); once
+    // every qubit is blocked no gate can
+    auto sweep = [&](Bits<W>& sel) {
+        uint64_t blocked = 0;
+        for (int id = 0; id < gate_num && blocked != all; id++) {
             if (sel.test(id)) continue;
-            const Gate& g = gates_[remain_[id]];
-            if (g.isDiagonal()) {
-                if (g.isControlGate()) {
-                    if (!blocked[g.controlQubit] && !blocked[g.targetQubit]) sel.set(id);
-                    else blocked[g.controlQubit] = blocked[g.targetQubit] = 1;
-                } else {
-                    if (!blocked[g.targetQubit]) sel.set(id);
-                }
+            const Brief g = gates[remain_[id]];
+            const uint64_t t = 1ull << g.t, c = g.c >= 0 ? 1ull << g.c : 0;
+            if (g.diagonal) {
+                if (!(blocked & (t | c))) sel.set(id);
+                else if (c) blocked |= t | c;
             } else {
-                if (g.isControlGate()) blocked[g.controlQubit] = 1;
-                if (g.isC2Gate()) blocked[g.controlQubit2] = 1;
-                blocked[g.targetQubit] = 1;
+                blocked |= t | c | (g.c2 >= 0 ? 1ull << g.c2 : 0);
             }
         }
     };
@@ -192,8 +212,9 @@ std::vector<std::vector<int>> GroupFinder::findAll(std::vector<char>& full, std:
     for (auto& sel : cands) {
         if (enableGlobal) sweep(sel);
         std::vector<int> ret;
-        for (int id = 0; id < gate_num; id++)
-            if (sel.test(id)) ret.push_back(remain_[id]);
+        ret.reserve(sel.count(W));
+        for (int k = 0; k < W; k++)
+            for (uint64_t m = sel.w[k]; m; m &= m - 1) ret.push_back(remain_[64 * k + __builtin_ctzll(m)]);
         bool dup = false;
         for (auto& o : out) if (o == ret) dup = true;
         if (!dup) out.push_back(std::move(ret));
@@ -321,10 +342,34 @@ static Schedule greedySchedule(int n, const std::vector<Gate>& gates, const Comp
 // TransMM groups, so the coalesced qubits are physical 0..coalesce-1.
 static std::vector<std::vector<int>> beamPerGate(int n, const std::vector<Gate>& gates, const CompilerParams& p)
 {
+    // groups of a partial partition, newest first, shared with its siblings
+    struct Link {
+        std::vector<int> group;
+        std::shared_ptr<const Link> before;
+    };
     struct Node {
         GroupFinder f;
-        std::vector<std::vector<int>> groups;
+        std::shared_ptr<const Link> groups;
         size_t done;
+        uint64_t hash;   // of the set of placed gates
+    };
+    struct Child {
+        size_t parent;
+        std::vector<int> group;
+        size_t done;
+        uint64_t hash;
+    };
+    auto mix = [](uint64_t x) {   // SplitMix64
+        x += 0x9e3779b97f4a7c15ull;
+        x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+        x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+        return x ^ (x >> 31);
+    };
+    auto unroll = [](const Link* l) {
+        std::vector<std::vector<int>> groups;
+        for (; l; l = l->before.get()) groups.push_back(l->group);
+        std::reverse(groups.begin(), groups.end());
+        return groups;
     };
     const qindex all = n >= 63 ? ~qindex(0) : ((qindex(1) << n) - 1);
     const int coalesce = std::min(p.coalesce, n);
@@ -332,38 +377,45 @@ static std::vector<std::vector<int>> beamPerGate(int n, const std::vector<Gate>&
     qindex co = 0;
     for (int j = 0; j < coalesce; j++) co |= qindex(1) << j;
     std::vector<Node> beam;
-    beam.push_back(Node{GroupFinder(n, gates, p.window), {}, 0});
+    beam.push_back(Node{GroupFinder(n, gates, p.window), nullptr, 0, 0});
     std::vector<char> full(n);
     std::vector<qindex> related(n);
     const int width = std::max(1, p.beam);
     const int starts = std::max(2, p.starts);
     while (true) {
         for (auto& nd : beam)
-            if (nd.f.empty()) return nd.groups;
-        std::vector<Node> next;
-        for (auto& nd : beam) {
+            if (nd.f.empty()) return unroll(nd.groups.get());
+        // children are ranked by what they place; only those kept are built
+        std::vector<Child> next;
+        for (size_t b = 0; b < beam.size(); b++) {
             std::fill(full.begin(), full.end(), 0);
             std::fill(related.begin(), related.end(), co);
-            auto cands = nd.f.findAll(full, related, true, localSize, all, starts);
+            auto cands = beam[b].f.findAll(full, related, true, localSize, all, starts);
             for (auto& c : cands) {
                 if (c.empty()) continue;
-                Node ch{nd.f, nd.groups, nd.done + c.size()};
-                ch.f.remove(c);
-                ch.groups.push_back(c);
-                next.push_back(std::move(ch));
+                uint64_t h = beam[b].hash;
+                for (int g : c) h ^= mix((uint64_t)g);
+                const size_t done = beam[b].done + c.size();
+                next.push_back(Child{b, std::move(c), done, h});
             }
         }
-        if (next.empty()) return beam.front().groups;   // cannot happen for valid parameters
+        if (next.empty()) return unroll(beam.front().groups.get());   // cannot happen for valid parameters
         std::vector<size_t> ord(next.size());
         for (size_t i = 0; i < ord.size(); i++) ord[i] = i;
         std::stable_sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return next[a].done > next[b].done; });
         std::vector<Node> kept;
         for (size_t i : ord) {
             if ((int)kept.size() >= width) break;
+            Child& ch = next[i];
+            GroupFinder f = beam[ch.parent].f;
+            f.remove(ch.group);
             bool dup = false;
             for (auto& k : kept)
-                if (k.done == next[i].done && k.f.remain() == next[i].f.remain()) { dup = true; break; }
-            if (!dup) kept.push_back(std::move(next[i]));
+                if (k.done == ch.done && k.hash == ch.hash && k.f.remain() == f.remain()) { dup = true; break; }
+            if (dup) continue;
+            kept.push_back(Node{std::move(f),
+                                std::make_shared<const Link>(Link{std::move(ch.group), beam[ch.parent].groups}),
+                                ch.done, ch.hash});
         }
         beam.swap(kept);
     }

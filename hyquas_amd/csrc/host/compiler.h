@@ -1,6 +1,8 @@
 // compiler.h -- the hybrid partitioner (src/compiler.h / compiler.cpp), single GPU.
 #pragma once
 
+#include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "evaluator.h"
@@ -43,9 +45,19 @@ public:
     const std::vector<int>& remain() const { return remain_; }
 
 private:
+    // what the search reads of a gate: target, controls (-1: none)
+    struct Brief {
+        int8_t t, c, c2;
+        bool diagonal;
+    };
+    static qindex withGate(qindex rel, const Brief& g, qindex localQubits, bool enableGlobal);
+    template <int W>
+    std::vector<std::vector<int>> findAllIn(std::vector<char>& full, std::vector<qindex>& related, bool enableGlobal,
+                                            int localSize, qindex localQubits, int starts) const;
+
     int n_;
     int window_;
-    const std::vector<Gate>& gates_;
+    std::shared_ptr<const std::vector<Brief>> gates_;   // shared by copies
     std::vector<int> remain_;   // ascending indices of ungrouped gates
 };
 
