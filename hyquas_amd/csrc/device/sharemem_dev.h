@@ -71,23 +71,23 @@ __device__ __forceinline__ void lane_swap(cplx<R> (&a)[1 << RB], uint32_t creg, 
     }
 }
 
-// c: the matrix's real parts, rest: its imaginary ones in LDS (read by the
-// forms that have any); lane: some thread-bit control, `on` where it holds
+// c0: the first coefficient, coef: all of them in LDS (a matrix's real parts,
+// then its imaginary ones); lane: some thread-bit control, `on` where it holds
 template <typename R, int RB, int P>
-__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool lane, bool on,
-                                       const R (&c)[4], const R* rest)
+__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool lane, bool on, R c0,
+                                       const R* coef)
 {
     R m[8];
     auto matrix = [&](bool imag) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) { m[2 * i] = c[i]; m[2 * i + 1] = imag ? rest[i] : R(0); }
+        for (int i = 0; i < 4; i++) { m[2 * i] = coef[i]; m[2 * i + 1] = imag ? coef[4 + i] : R(0); }
         if (lane) {
 #pragma unroll
             for (int i = 0; i < 8; i++)
                 if (imag || !(i & 1)) m[i] = on ? m[i] : (i == 0 || i == 6) ? R(1) : R(0);
         }
     };
-    m[0] = c[0];
+    m[0] = c0;
     switch (kind) {
     case SHM_SWAP: reg_pairs<R, RB, SHM_SWAP, P>(a, creg, m); break;
     case SHM_Y: reg_pairs<R, RB, SHM_Y, P>(a, creg, m); break;
@@ -143,9 +143,13 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
     const uint32_t tid = threadIdx.x;
 
     // block base address: the block index scattered to the block bits
+    // (the first runs without a branch, so that their loads go out together;
+    // unused runs have an empty mask)
     uint64_t base = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) base |= ((blk >> H->run[j].src) & H->run[j].mask) << H->run[j].dst;
     const uint32_t nruns = H->num_runs;
-    for (uint32_t j = 0; j < nruns; j++) base |= ((blk >> H->run[j].src) & H->run[j].mask) << H->run[j].dst;
+    for (uint32_t j = 4; j < nruns; j++) base |= ((blk >> H->run[j].src) & H->run[j].mask) << H->run[j].dst;
     // a tile known to be zero stays zero (uniform over the block)
     if (!(mode & TILE_READ) && (base & H->zero_mask)) return;
 
@@ -163,7 +167,7 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
     auto fetch = [&](uint32_t from) {
 #pragma unroll
         for (int i = 0; i < PIECES; i++)
-            if (from + (uint32_t)(i * NT) * 16u < nbytes)
+            if (i == 0 || from + (uint32_t)(i * NT) * 16u < nbytes)
                 piece[i] = *(const HQ_GLOBAL uint4*)(slots + from + (uint32_t)(i * NT + tid) * 16u);
     };
     auto fill = [&]() {
@@ -236,17 +240,23 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
     double lx = 1, ly = 0;    // the lane's factor
     uint32_t window = 0;      // bytes of the current window's start in the program
     const char* pc = win;
-    uint4 next = *(const uint4*)pc;   // fields of the next slot
+    // fields and first two coefficients of the next slot: all that most ops
+    // have (the rest is read when it is used)
+    uint4 next = *(const uint4*)pc;
+    R next0 = ((const R*)(pc + 16))[0], next1 = ((const R*)(pc + 16))[1];
+    auto read_next = [&]() {
+        next = *(const uint4*)pc;     // (behind the last slot of a window: unused)
+        next0 = ((const R*)(pc + 16))[0];
+        next1 = ((const R*)(pc + 16))[1];
+    };
     char* const xlds = (char*)lds;
     for (;;) {
         const uint32_t w0 = uniform(next.x), w1 = uniform(next.y);
         const uint32_t cb = uniform(next.z), cbv = uniform(next.w);
         const R* const coef = (const R*)(pc + 16);
-        R c[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) c[i] = coef[i];
+        const R c0 = next0, c1 = next1;
         pc += SLOT;
-        next = *(const uint4*)pc;     // (behind the last slot of a window: unused)
+        read_next();
         const int kind = (int)(w0 & 255u), aux = (int)((w0 >> 8) & 255u);
         const uint32_t creg = (w0 >> 16) & 255u, cregv = w0 >> 24;
         const uint32_t cthr = w1 & 0xffffu, cthrv = w1 >> 16;
@@ -258,12 +268,12 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             if (((uint32_t)blk & cb) != cbv) continue;
             const bool lane = cthr != 0;
             switch (aux) {
-            case 0: reg_op<R, RB, 0>(a, kind, creg, lane, on, c, coef + 4); break;
-            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, lane, on, c, coef + 4); break;
-            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, lane, on, c, coef + 4); break;
-            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, lane, on, c, coef + 4); break;
-            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, lane, on, c, coef + 4); break;
-            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, lane, on, c, coef + 4); break;
+            case 0: reg_op<R, RB, 0>(a, kind, creg, lane, on, c0, coef); break;
+            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, lane, on, c0, coef); break;
+            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, lane, on, c0, coef); break;
+            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, lane, on, c0, coef); break;
+            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, lane, on, c0, coef); break;
+            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, lane, on, c0, coef); break;
             }
             static_assert(RB <= 6, "register positions above 5 are not dispatched");
             continue;
@@ -307,7 +317,7 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
 #pragma unroll
             for (int j = 0; j < NR; j++) scale(a[j], tab[j]);
             pc += aux * SLOT;
-            next = *(const uint4*)pc;
+            read_next();
             continue;
         }
         if (kind == SLOT_TABMASK) {
@@ -317,12 +327,12 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             for (int j = 0; j < NR; j++)
                 if ((jm >> j) & 1) scale(a[j], tab[j]);
             pc += aux * SLOT;
-            next = *(const uint4*)pc;
+            read_next();
             continue;
         }
         if (kind == SLOT_SCALE) {
 #pragma unroll
-            for (int j = 0; j < NR; j++) scale(a[j], c[0], c[1]);
+            for (int j = 0; j < NR; j++) scale(a[j], c0, c1);
             continue;
         }
         if (kind == SLOT_LANEMUL) {
@@ -349,13 +359,13 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             fill();
             __syncthreads();
             pc = win;
-            next = *(const uint4*)pc;
+            read_next();
             continue;
         }
         if (kind == SLOT_END) break;
         if (((uint32_t)blk & cb) != cbv) continue;
         if (kind == SLOT_LANE) {
-            const double fr = on ? (double)c[0] : 1.0, fi = on ? (double)c[1] : 0.0;
+            const double fr = on ? (double)c0 : 1.0, fi = on ? (double)c1 : 0.0;
             const double x = lx, y = ly;
             lx = fr * x - fi * y;
             ly = fr * y + fi * x;
@@ -365,7 +375,7 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             for (int j = 0; j < NR; j++)
                 if ((j & creg) == cregv) { a[j].x *= f; a[j].y *= f; }
         } else {   // SLOT_MIX
-            const R fr = on ? c[0] : R(1), fi = on ? c[1] : R(0);
+            const R fr = on ? c0 : R(1), fi = on ? c1 : R(0);
 #pragma unroll
             for (int j = 0; j < NR; j++)
                 if ((j & creg) == cregv) scale(a[j], fr, fi);

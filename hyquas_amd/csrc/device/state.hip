@@ -228,44 +228,45 @@ __global__ __launch_bounds__(EZ_THREADS) void k_expect_z(const cplx<R>* __restri
         if (col < NCOL) sh[wave][col] = r;
     }
     __syncthreads();
-    const int o = threadIdx.x;
-    if (o >= RED_Z_STRIDE) return;
-    // row column o: qubit q's bit (pair = 0) or the pair q, q+1
-    const bool pair = o > RED_MAXQ;
-    const int q = o == 0 ? -1 : pair ? o - 1 - RED_MAXQ : o - 1;
-    int col = 0;            // thread column summed over the waves with weight 1 ...
-    int wmask = -1;         // ... or, >= 0: over the waves whose index has odd parity under it
-    bool zero = false;
-    constexpr int LANE0 = PAIR ? 1 : 0;   // qubit of lane bit 0
-    if (q < 0) {
-        col = 0;
-    } else if (q + (pair ? 1 : 0) >= n) {
-        zero = true;
-    } else if (q >= EZ_CHUNK_BITS + LB) {
-        const uint64_t c = blk << l;      // constant over the block
-        const uint64_t y = pair ? c ^ (c >> 1) : c;
-        zero = !((y >> (q - EZ_CHUNK_BITS)) & 1);
-    } else if (q >= EZ_CHUNK_BITS) {
-        col = 20 + (pair ? LB : 0) + (q - EZ_CHUNK_BITS);
-    } else if (!pair) {
-        if (q >= 9) wmask = 1 << (q - 9);
-        else if (q >= 7) col = 12 + (q - 6);
-        else if (PAIR && q == 0) col = 12;
-        else if (!PAIR && q == 6) col = 12;
-        else col = 1 + (q - LANE0);
-    } else {
-        if (q == 12) col = 19;
-        else if (q >= 9) wmask = 3 << (q - 9);
-        else if (q == 8) col = 18;
-        else if (q == 7) col = 15;
-        else if (PAIR) col = q == 6 ? 17 : q == 0 ? 16 : 7 + (q - 1);
-        else col = q == 6 ? 16 : q == 5 ? 17 : 7 + q;
+    const int waves = (int)(blockDim.x >> 6);
+    for (int o = threadIdx.x; o < RED_Z_STRIDE; o += (int)blockDim.x) {
+        // row column o: qubit q's bit (pair = 0) or the pair q, q+1
+        const bool pair = o > RED_MAXQ;
+        const int q = o == 0 ? -1 : pair ? o - 1 - RED_MAXQ : o - 1;
+        int col = 0;            // thread column summed over the waves with weight 1 ...
+        int wmask = -1;         // ... or, >= 0: over the waves whose index has odd parity under it
+        bool zero = false;
+        constexpr int LANE0 = PAIR ? 1 : 0;   // qubit of lane bit 0
+        if (q < 0) {
+            col = 0;
+        } else if (q + (pair ? 1 : 0) >= n) {
+            zero = true;
+        } else if (q >= EZ_CHUNK_BITS + LB) {
+            const uint64_t c = blk << l;      // constant over the block
+            const uint64_t y = pair ? c ^ (c >> 1) : c;
+            zero = !((y >> (q - EZ_CHUNK_BITS)) & 1);
+        } else if (q >= EZ_CHUNK_BITS) {
+            col = 20 + (pair ? LB : 0) + (q - EZ_CHUNK_BITS);
+        } else if (!pair) {
+            if (q >= 9) wmask = 1 << (q - 9);
+            else if (q >= 7) col = 12 + (q - 6);
+            else if (PAIR && q == 0) col = 12;
+            else if (!PAIR && q == 6) col = 12;
+            else col = 1 + (q - LANE0);
+        } else {
+            if (q == 12) col = 19;
+            else if (q >= 9) wmask = 3 << (q - 9);
+            else if (q == 8) col = 18;
+            else if (q == 7) col = 15;
+            else if (PAIR) col = q == 6 ? 17 : q == 0 ? 16 : 7 + (q - 1);
+            else col = q == 6 ? 16 : q == 5 ? 17 : 7 + q;
+        }
+        double r = 0;
+        if (!zero)
+            for (int w = 0; w < waves; w++)
+                if (wmask < 0 || (__popc(w & wmask) & 1)) r += sh[w][col];
+        out[blk * RED_Z_STRIDE + o] = r;
     }
-    double r = 0;
-    if (!zero)
-        for (int w = 0; w < EZ_THREADS / 64; w++)
-            if (wmask < 0 || (__popc(w & wmask) & 1)) r += sh[w][col];
-    out[blk * RED_Z_STRIDE + o] = r;
 }
 
 template <typename RA, typename RB>
@@ -622,8 +623,10 @@ static hq_status launch_expect_z(hq_state s, double* rows, double* fin)
     const unsigned g = 1u << (cb - l);
     static_assert(RED_Z_BLOCKS == 1 << 8, "block bits");
     double* part = g > 1 ? rows : fin;
+    // states below one chunk: a wave per 512 amplitudes
+    const unsigned threads = s->n >= EZ_CHUNK_BITS ? EZ_THREADS : 64u << std::max(0, s->n - 9);
 #define HQ_EZ(RV, LBV)                                                                                          \
-    hipLaunchKernelGGL((k_expect_z<RV, LBV>), dim3(g), dim3(EZ_THREADS), 0, s->stream, (const cplx<RV>*)s->data, \
+    hipLaunchKernelGGL((k_expect_z<RV, LBV>), dim3(g), dim3(threads), 0, s->stream, (const cplx<RV>*)s->data, \
                        s->n, l, part)
     if (s->precision == HQ_C128) {
         if (l == 0) HQ_EZ(double, 0);
