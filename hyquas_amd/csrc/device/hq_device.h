@@ -171,20 +171,30 @@ struct ShmSlot {
 };
 static_assert(sizeof(ShmSlot) == 16, "ShmSlot layout");
 
+// Kinds below SLOT_DIRECT_END are 8 P + SlotDirect for register bit P: the
+// frequent updates, without register or block conditions, reached by one
+// switch.  A dispatch step is a compare and a branch, some 40 cycles of a lone
+// wave; the general path takes twice as many of them.
+enum SlotDirect : uint8_t {
+    DIRECT_HADD, DIRECT_ROTA, DIRECT_ROTB, DIRECT_RXA, DIRECT_RXB,
+    DIRECT_PHASE,        // |1> half *= (m[0], m[1])
+    DIRECT_LPHASE,       // the same where the thread-bit condition holds
+    DIRECT_LSWAP,        // X where it holds
+};
 enum SlotKind : uint8_t {
-    // pair updates: the ShmClass value (SHM_SWAP..SHM_GEN, SHM_HADD..SHM_RXB)
-    SLOT_CSWAP = 32,     // SHM_SWAP under a thread-bit control
-    SLOT_SCALE = 33,     // every amplitude *= (m[0], m[1])
-    SLOT_TAB = 34,       // complex table of the 2^RB register indices in the next `aux` slots
-    SLOT_TABMASK = 35,   // the same; only register indices in cblkv:cblk are multiplied
-    SLOT_MIX = 36,
-    SLOT_MIXSIGN = 37,   // factor -1
-    SLOT_LANE = 38,
-    SLOT_LANETAB = 39,   // the lane's factor = thread's entry of the lane table cblk (of this program)
-    SLOT_LANEMUL = 40,   // every amplitude *= the lane's factor
-    SLOT_XCHG = 41,      // LDS exchange into the next stage's split
-    SLOT_REFILL = 42,    // copy the next window of slots to LDS
-    SLOT_END = 43,
+    SLOT_DIRECT_END = 48,
+    SLOT_PAIR = 64,      // + ShmClass (SHM_SWAP..SHM_GEN): pair update under any controls, target bit aux
+    SLOT_CSWAP = 95,     // SHM_SWAP under a thread-bit control and others
+    SLOT_SCALE,          // every amplitude *= (m[0], m[1])
+    SLOT_TAB,            // complex table of the 2^RB register indices in the next `aux` slots
+    SLOT_MIX,
+    SLOT_MIXSIGN,        // factor -1
+    SLOT_LANE,
+    SLOT_LANETAB,        // the lane's factor = thread's entry of the lane table cblk (of this program)
+    SLOT_LANEMUL,        // every amplitude *= the lane's factor
+    SLOT_XCHG,           // LDS exchange into the next stage's split
+    SLOT_REFILL,         // copy the next window of slots to LDS
+    SLOT_END,
 };
 
 constexpr int SHM_WINDOW_BYTES = 7680;   // 96 slots of complex128, 160 of complex64

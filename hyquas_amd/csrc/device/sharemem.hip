@@ -848,17 +848,22 @@ struct Encoder {
             const ShmOp& o = P.ops[i];
             switch (o.cls) {
             case SHM_TAB: {
+                // factors on the |1> half of one register bit
+                const uint32_t d = o.jdep;
+                if (!(d & (d - 1)) && !(o.jmask & 1) && !((o.jprod >> d) & 1)) {
+                    ShmSlot h{};
+                    h.kind = (uint8_t)(8 * __builtin_ctz(d) + DIRECT_PHASE);
+                    op(h, &P.tabs[2 * (o.tab + d)], 2);
+                    break;
+                }
                 const size_t bytes = ((size_t)1 << P.rb) * sizeof(Factor<R, PRECISE>);
                 const size_t more = (bytes + SLOT - 1) / SLOT;
                 std::vector<Factor<R, PRECISE>> t((size_t)1 << P.rb);
                 for (size_t j = 0; j < t.size(); j++)
                     t[j] = Factor<R, PRECISE>::of(P.tabs[2 * (o.tab + j)], P.tabs[2 * (o.tab + j) + 1]);
                 ShmSlot h{};
-                // per-index branches pay when at least half of the indices keep their amplitude
-                const bool mask = 2 * __builtin_popcountll(o.jmask) <= (1 << P.rb);
-                h.kind = mask ? SLOT_TABMASK : SLOT_TAB;
+                h.kind = SLOT_TAB;
                 h.aux = (uint8_t)more;
-                if (mask) { h.cblk = (uint32_t)o.jmask; h.cblkv = (uint32_t)(o.jmask >> 32); }
                 room(1 + more);
                 put(h, nullptr, 0);
                 const size_t at = slots.size();
@@ -867,7 +872,10 @@ struct Encoder {
                 break;
             }
             case SHM_MIX:
-                op(head(o, (o.flags & SHM_FLAG_REAL) && o.m[0] == -1.0 ? SLOT_MIXSIGN : SLOT_MIX), o.m, 2);
+                if (!o.cblk && o.creg == o.cregv && !(o.creg & (o.creg - 1)))
+                    op(head(o, 8 * __builtin_ctz(o.creg) + DIRECT_LPHASE), o.m, 2);
+                else
+                    op(head(o, (o.flags & SHM_FLAG_REAL) && o.m[0] == -1.0 ? SLOT_MIXSIGN : SLOT_MIX), o.m, 2);
                 break;
             case SHM_LANE:
                 if (o.cblk) op(head(o, SLOT_LANE), o.m, 2);
@@ -881,10 +889,17 @@ struct Encoder {
                 }
                 break;
             case SHM_SWAP:
-                op(head(o, o.cthr ? (int)SLOT_CSWAP : (int)SHM_SWAP), nullptr, 0);
+                if (o.cthr && !o.creg && !o.cblk) op(head(o, 8 * o.tpos + DIRECT_LSWAP), nullptr, 0);
+                else op(head(o, o.cthr ? (int)SLOT_CSWAP : SLOT_PAIR + SHM_SWAP), nullptr, 0);
                 break;
+            // the factored forms come from uncontrolled gates
+            case SHM_HADD: op(head(o, 8 * o.tpos + DIRECT_HADD), nullptr, 0); break;
+            case SHM_ROTA: op(head(o, 8 * o.tpos + DIRECT_ROTA), o.m, 1); break;
+            case SHM_ROTB: op(head(o, 8 * o.tpos + DIRECT_ROTB), o.m, 1); break;
+            case SHM_RXA: op(head(o, 8 * o.tpos + DIRECT_RXA), o.m, 1); break;
+            case SHM_RXB: op(head(o, 8 * o.tpos + DIRECT_RXB), o.m, 1); break;
             default:
-                op(head(o, o.cls), o.m, 8);
+                op(head(o, SLOT_PAIR + o.cls), o.m, 8);
                 break;
             }
         }

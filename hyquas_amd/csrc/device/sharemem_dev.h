@@ -44,14 +44,11 @@ __device__ __forceinline__ void reg_pairs(cplx<R> (&a)[1 << RB], uint32_t creg, 
         }
         return;
     }
-    // the factored forms come from uncontrolled gates only
-    if constexpr (CLS < SHM_HADD) {
 #pragma unroll
-        for (int j = 0; j < (1 << RB); j++) {
-            if (j & (1 << P)) continue;
-            if ((j & creg) != creg) continue;
-            pair_update<CLS, R>(a[j], a[j | (1 << P)], m);
-        }
+    for (int j = 0; j < (1 << RB); j++) {
+        if (j & (1 << P)) continue;
+        if ((j & creg) != creg) continue;
+        pair_update<CLS, R>(a[j], a[j | (1 << P)], m);
     }
 }
 
@@ -71,10 +68,34 @@ __device__ __forceinline__ void lane_swap(cplx<R> (&a)[1 << RB], uint32_t creg, 
     }
 }
 
-// c0: the first coefficient, coef: all of them in LDS (a matrix's real parts,
-// then its imaginary ones); lane: some thread-bit control, `on` where it holds
+// SlotDirect updates of register bit P; `on`: the lane's thread-bit condition
 template <typename R, int RB, int P>
-__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool lane, bool on, R c0,
+__device__ __forceinline__ void direct_op(cplx<R> (&a)[1 << RB], int op, bool on, R c0, R c1)
+{
+    R m[8];
+    m[0] = c0;
+    m[6] = c0;
+    m[7] = c1;
+    switch (op) {
+    case DIRECT_HADD: reg_pairs<R, RB, SHM_HADD, P>(a, 0, m); break;
+    case DIRECT_ROTA: reg_pairs<R, RB, SHM_ROTA, P>(a, 0, m); break;
+    case DIRECT_ROTB: reg_pairs<R, RB, SHM_ROTB, P>(a, 0, m); break;
+    case DIRECT_RXA: reg_pairs<R, RB, SHM_RXA, P>(a, 0, m); break;
+    case DIRECT_RXB: reg_pairs<R, RB, SHM_RXB, P>(a, 0, m); break;
+    case DIRECT_PHASE: reg_pairs<R, RB, SHM_PHASE, P>(a, 0, m); break;
+    case DIRECT_LPHASE:
+        m[6] = on ? c0 : R(1);
+        m[7] = on ? c1 : R(0);
+        reg_pairs<R, RB, SHM_PHASE, P>(a, 0, m);
+        break;
+    default: lane_swap<R, RB, P>(a, 0, on); break;
+    }
+}
+
+// the other pair updates; coef: the matrix's real parts, then its imaginary
+// ones, in LDS; lane: some thread-bit control, `on` where it holds
+template <typename R, int RB, int P>
+__device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t creg, bool lane, bool on,
                                        const R* coef)
 {
     R m[8];
@@ -87,18 +108,12 @@ __device__ __forceinline__ void reg_op(cplx<R> (&a)[1 << RB], int kind, uint32_t
                 if (imag || !(i & 1)) m[i] = on ? m[i] : (i == 0 || i == 6) ? R(1) : R(0);
         }
     };
-    m[0] = c0;
     switch (kind) {
-    case SHM_SWAP: reg_pairs<R, RB, SHM_SWAP, P>(a, creg, m); break;
-    case SHM_Y: reg_pairs<R, RB, SHM_Y, P>(a, creg, m); break;
-    case SHM_REAL: matrix(false); reg_pairs<R, RB, SHM_REAL, P>(a, creg, m); break;
-    case SHM_RX: matrix(true); reg_pairs<R, RB, SHM_RX, P>(a, creg, m); break;
-    case SHM_GEN: matrix(true); reg_pairs<R, RB, SHM_GEN, P>(a, creg, m); break;
-    case SHM_HADD: reg_pairs<R, RB, SHM_HADD, P>(a, creg, m); break;
-    case SHM_ROTA: reg_pairs<R, RB, SHM_ROTA, P>(a, creg, m); break;
-    case SHM_ROTB: reg_pairs<R, RB, SHM_ROTB, P>(a, creg, m); break;
-    case SHM_RXA: reg_pairs<R, RB, SHM_RXA, P>(a, creg, m); break;
-    case SHM_RXB: reg_pairs<R, RB, SHM_RXB, P>(a, creg, m); break;
+    case SLOT_PAIR + SHM_SWAP: reg_pairs<R, RB, SHM_SWAP, P>(a, creg, m); break;
+    case SLOT_PAIR + SHM_Y: reg_pairs<R, RB, SHM_Y, P>(a, creg, m); break;
+    case SLOT_PAIR + SHM_REAL: matrix(false); reg_pairs<R, RB, SHM_REAL, P>(a, creg, m); break;
+    case SLOT_PAIR + SHM_RX: matrix(true); reg_pairs<R, RB, SHM_RX, P>(a, creg, m); break;
+    case SLOT_PAIR + SHM_GEN: matrix(true); reg_pairs<R, RB, SHM_GEN, P>(a, creg, m); break;
     default: lane_swap<R, RB, P>(a, creg, on); break;
     }
 }
@@ -264,16 +279,32 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
         // Every branch below is uniform over the block: a lane whose
         // thread-bit condition does not hold gets the identity's coefficients
         // or keeps its values by selects instead of leaving the op.
+        if (kind < SLOT_DIRECT_END) {
+            switch (kind) {
+#define HQ_DIRECT(PV)                                                                          \
+    case 8 * PV + 0: case 8 * PV + 1: case 8 * PV + 2: case 8 * PV + 3: case 8 * PV + 4:        \
+    case 8 * PV + 5: case 8 * PV + 6: case 8 * PV + 7:                                          \
+        if constexpr (RB > PV) direct_op<R, RB, PV>(a, kind & 7, on, c0, c1);                   \
+        break;
+                HQ_DIRECT(0) HQ_DIRECT(1) HQ_DIRECT(2) HQ_DIRECT(3) HQ_DIRECT(4)
+            default:
+                if constexpr (RB > 5) direct_op<R, RB, 5>(a, kind & 7, on, c0, c1);
+                break;
+#undef HQ_DIRECT
+            }
+            static_assert(RB <= 6, "register positions above 5 are not dispatched");
+            continue;
+        }
         if (kind <= SLOT_CSWAP) {
             if (((uint32_t)blk & cb) != cbv) continue;
             const bool lane = cthr != 0;
             switch (aux) {
-            case 0: reg_op<R, RB, 0>(a, kind, creg, lane, on, c0, coef); break;
-            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, lane, on, c0, coef); break;
-            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, lane, on, c0, coef); break;
-            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, lane, on, c0, coef); break;
-            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, lane, on, c0, coef); break;
-            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, lane, on, c0, coef); break;
+            case 0: reg_op<R, RB, 0>(a, kind, creg, lane, on, coef); break;
+            case 1: if constexpr (RB > 1) reg_op<R, RB, 1>(a, kind, creg, lane, on, coef); break;
+            case 2: if constexpr (RB > 2) reg_op<R, RB, 2>(a, kind, creg, lane, on, coef); break;
+            case 3: if constexpr (RB > 3) reg_op<R, RB, 3>(a, kind, creg, lane, on, coef); break;
+            case 4: if constexpr (RB > 4) reg_op<R, RB, 4>(a, kind, creg, lane, on, coef); break;
+            default: if constexpr (RB > 5) reg_op<R, RB, 5>(a, kind, creg, lane, on, coef); break;
             }
             static_assert(RB <= 6, "register positions above 5 are not dispatched");
             continue;
@@ -316,16 +347,6 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
             const Factor<R, PRECISE>* __restrict__ tab = (const Factor<R, PRECISE>*)pc;
 #pragma unroll
             for (int j = 0; j < NR; j++) scale(a[j], tab[j]);
-            pc += aux * SLOT;
-            read_next();
-            continue;
-        }
-        if (kind == SLOT_TABMASK) {
-            const Factor<R, PRECISE>* __restrict__ tab = (const Factor<R, PRECISE>*)pc;
-            const uint64_t jm = (uint64_t)cbv << 32 | cb;
-#pragma unroll
-            for (int j = 0; j < NR; j++)
-                if ((jm >> j) & 1) scale(a[j], tab[j]);
             pc += aux * SLOT;
             read_next();
             continue;
