@@ -457,8 +457,14 @@ static hq_status launch_mfma(hq_state s, const R* ure, const R* uim, const void*
 
 // Column tile width: complex128 (three products, three accumulators per
 // column block, the next tile's B held in registers) takes 32-column tiles to
-// stay within 256 registers (two waves per SIMD)
-template <typename R> constexpr int dense_nt(int mq) { return sizeof(R) == 8 || mq == 7 ? 32 : 64; }
+// stay within 256 registers (two waves per SIMD); complex64 at K = 64 takes
+// them for the LDS: 34 KiB instead of 67 lets four blocks share a CU, whose
+// loads, products and stores overlap (28 qubits: 1.21 -> 1.17 ms a pass, 113 ->
+// 118 TFLOP/s; K = 16 and 32 are HBM-bound and lose 1-3 % with shorter tiles)
+template <typename R> constexpr int dense_nt(int mq) { return sizeof(R) == 8 || mq >= 6 ? 32 : 64; }
+// columns of the smallest state the MFMA form takes (K = 64 in complex64 also
+// fits half of it; such states keep the double-precision sums of the simple form)
+template <typename R> constexpr int dense_min_cols(int mq) { return sizeof(R) == 8 || mq == 7 ? 32 : 64; }
 
 template <typename R>
 static hq_status launch_mfma_masks(hq_state s, const R* ure, const R* uim, int mq, const void* in, void* out,
@@ -483,7 +489,7 @@ static hq_status launch_dense_t(hq_state s, const void* d_mat, int mq, void* in,
     const R* uim = ure + K * K;
     // MFMA path: the matrix qubits are the lowest, the tile columns the next
     const int nt = mq >= 4 && mq <= 7 ? dense_nt<R>(mq) : 0;
-    if (nt && s->amps >= K * nt) {
+    if (nt && s->amps >= K * (uint64_t)dense_min_cols<R>(mq)) {
         DenseMasks dm;
         dm.rows = K - 1;
         dm.cols = (uint64_t)(nt - 1) << mq;
@@ -506,8 +512,8 @@ hq_status launch_dense(hq_state s, const void* d_mat, int mq, void* in, void* ou
 int dense_at_min_qubits(int precision, int mq)
 {
     if (mq < 4 || mq > 7) return 1 << 20;
-    const int nt = precision == HQ_C128 ? dense_nt<double>(mq) : dense_nt<float>(mq);
-    return mq + __builtin_ctz((unsigned)nt);
+    const int cols = precision == HQ_C128 ? dense_min_cols<double>(mq) : dense_min_cols<float>(mq);
+    return mq + __builtin_ctz((unsigned)cols);
 }
 
 // U on the qubits at the set bits of `rows` (row index bit j = the j-th
