@@ -619,10 +619,11 @@ static void append_jit(JobPlan* jp, const ShmPlan& plan, const std::vector<doubl
 static hq_status add_group(JobPlan* jp, int n, int precision, const std::vector<hq_gate>& hg, uint64_t mask,
                            bool first, bool last, uint64_t zero_mask, KernelCache* kc)
 {
-    // many circuits fill the chip together: the single-state rule for few
-    // blocks (n - tile small) does not apply here
+    // a whole-state group is a chain of ops in one block; tiles of larger
+    // circuits fill the chip together, so the rule for few blocks does not
+    // apply to them
     const int tile = __builtin_popcountll((unsigned long long)mask);
-    const int irb = interpreter_rb(precision, tile, 64);
+    const int irb = interpreter_rb(precision, tile, tile == n ? n : 64);
     // an engine returns sums over a circuit's qubits, which merged factors in
     // one float serve; its passes are bound by the operations they save
     ShmPlan plan;

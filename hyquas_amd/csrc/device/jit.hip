@@ -568,15 +568,16 @@ struct Emitter {
         if (nst > 1) o << "    __shared__ C lds[" << (1 << (split ? K - 1 : K)) << "];\n";
         o << "    const unsigned t = threadIdx.x;\n";
         if (batch) {
-            o << "    unsigned lo_ = 0, hi_ = count;\n";
-            o << "    const unsigned long long bid = blockIdx.x;\n";
-            o << "    while (hi_ - lo_ > 1) { const unsigned mid = (lo_ + hi_) >> 1; "
-                 "if (items[mid].first_block <= bid) lo_ = mid; else hi_ = mid; }\n";
+            // circuits of one kernel have one size: item and tile by shift and
+            // mask (a search of the table cost a chain of loads per block)
+            const uint32_t nbb = P.hdr.num_block_bits;
+            o << "    const unsigned lo_ = blockIdx.x >> " << nbb << ";\n";
+            o << "    if (lo_ >= count) return;\n";
             o << "    HQ_G C* __restrict__ psi = (HQ_G C*)items[lo_].psi;\n";
             o << "    const HQ_G R* __restrict__ cf = (const HQ_G R*)items[lo_].cf;\n";
             if (readout) o << "    HQ_G double* __restrict__ part = (HQ_G double*)items[lo_].part;\n";
             o << "    const unsigned mode = items[lo_].mode;\n";
-            o << "    const unsigned long long b = bid - items[lo_].first_block;\n";
+            o << "    const unsigned long long b = blockIdx.x & " << hex32((1u << nbb) - 1) << ";\n";
         } else if (bmap == 2)
             o << "    const unsigned long long b = (unsigned long long)(blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);\n";
         else if (bmap == 1)
