@@ -41,7 +41,7 @@ namespace hq {
 
 struct BatchItem {
     uint64_t psi;          // state of the circuit (cplx<R>*)
-    uint64_t prog;         // group program (ShmHeader blob)
+    uint64_t prog;         // group program (ShmProg header, slots, lane tables)
     uint64_t part;         // per-tile partial readouts, 3 doubles per tile (TILE_READ)
     uint64_t first_block;  // first grid block of this item
     uint32_t n;
@@ -1738,6 +1738,7 @@ hq_status hq_state_topk(hq_state s, int k, uint64_t* idx, double* prob)
     const auto lv = topk_levels(s->amps);
     const size_t cand = lv.size() > 1 ? lv[1].count * sizeof(Cand) : 0;
     // candidates stay on the device, the result goes straight to pinned memory
+    std::lock_guard<std::mutex> lock(s->ws_mu);
     hq_status st = ensure_ws(s, cand, TOPK * sizeof(Cand));
     if (st != HQ_OK) return st;
     const Cand* res = (const Cand*)s->h_ws;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -58,6 +59,7 @@ struct hq_state_s {
     char* d_ws = nullptr;     // readout workspace (device, pinned host), see ensure_ws
     char* h_ws = nullptr;
     size_t ws_dev = 0, ws_host = 0;   // bytes
+    std::mutex ws_mu;         // held by a readout from ensure_ws until it has its results
     bool profiling = false;
     std::vector<hq::ProfileEntry> prof;
     std::vector<hipEvent_t> free_events;
@@ -70,7 +72,7 @@ hq_status prof_begin(hq_state s, int kind, int* slot);
 hq_status prof_end(hq_state s, int slot);
 
 // Room for a readout in the state's workspace (grown on demand, freed with
-// the state); contents do not outlive a call.
+// the state); contents do not outlive a call, which holds ws_mu.
 hq_status ensure_ws(hq_state s, size_t dev, size_t host);
 // Gives back workspace beyond `keep` bytes (no work of the state may use it).
 void trim_ws(hq_state s, size_t keep);

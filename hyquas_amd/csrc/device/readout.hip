@@ -159,11 +159,15 @@ static hq_status sample(hq_state s, int shots, uint64_t seed, uint64_t* out)
 {
     const uint64_t chunks = (s->amps + SAMPLE_CHUNK - 1) / SAMPLE_CHUNK;
     const size_t batch = (size_t)std::min(shots, SAMPLE_BATCH);
-    const bool with_parts = chunks * SAMPLE_PARTS <= SAMPLE_MAX_PARTS;
+    bool with_parts = chunks * SAMPLE_PARTS <= SAMPLE_MAX_PARTS;
     // device: prefix, uniforms, shots, part sums; pinned: uniforms, shots, prefix
-    const size_t dev = (chunks + 2 * batch + (with_parts ? chunks * SAMPLE_PARTS : 0)) * 8;
-    const size_t host = (chunks + 2 * batch) * 8;
-    hq_status st = ensure_ws(s, dev, host);
+    const size_t dev = (chunks + 2 * batch) * 8, host = dev;
+    hq_status st = ensure_ws(s, dev + (with_parts ? chunks * SAMPLE_PARTS * 8 : 0), host);
+    if (st != HQ_OK && with_parts) {   // no room beside the state: the waves sum the parts themselves
+        (void)hipGetLastError();
+        with_parts = false;
+        st = ensure_ws(s, dev, host);
+    }
     if (st != HQ_OK) return st;
     double* d_prefix = (double*)s->d_ws;
     double* d_u = d_prefix + chunks;
@@ -208,6 +212,7 @@ extern "C" hq_status hq_state_sample(hq_state s, int shots, uint64_t seed, uint6
     HQ_CHECK(s && (out || shots == 0), HQ_ERR_ARG, "hq_state_sample: null argument");
     HQ_CHECK(shots >= 0 && shots <= (1 << 24), HQ_ERR_ARG, "hq_state_sample: shots must be in [0, 2^24]");
     if (shots == 0) return HQ_OK;
+    std::lock_guard<std::mutex> lock(s->ws_mu);
     const hq_status st = sample(s, shots, seed, out);
     // after an error some of the call's work may still be queued
     if (st != HQ_OK && st != HQ_ERR_STATE) (void)hipStreamSynchronize(s->stream);

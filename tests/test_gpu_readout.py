@@ -130,3 +130,17 @@ def test_norm_and_measure_elements(gpu, n, prec):
     for q in sorted({0, min(1, n - 1), n // 2, n - 1}):
         assert abs(s.measure_zero(q) - p.reshape(-1, 2, 1 << q)[:, 0].sum()) <= 1e-13, (n, q)
     s.close()
+
+
+def test_threads_share_a_state(gpu):
+    """Samples and top lists of one state drawn from several threads at a time
+    are those drawn one after another (both use the state's workspace)."""
+    from concurrent.futures import ThreadPoolExecutor
+    s, _ = _state(gpu, 16, 0, 6)
+    jobs = [(k, seed) for seed in range(6) for k in (3, 16)]
+    run = lambda j: (s.topk(j[0]), s.sample(500 + 4000 * (j[1] % 3), j[1]).tolist())
+    want = [run(j) for j in jobs]
+    s.sync()
+    with ThreadPoolExecutor(4) as ex:
+        assert list(ex.map(run, jobs * 2)) == want * 2
+    s.close()
