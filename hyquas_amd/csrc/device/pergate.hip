@@ -1,15 +1,17 @@
-// pergate.hip -- the plain method: one HBM pass per gate.
+// pergate.hip -- the plain method: gates one after another, without a plan.
 //
 // Replaces kernelExecSimple and its 19 gate kernels (src/kernelSimple.cu:40-446).
 // Differences by design: one templated kernel per update form instead of one
 // per gate type; threads enumerate only the pairs whose controls are set
 // (the reference launches 2^(n-1) threads and idles the others); 64-bit
-// indexing so n >= 33 works.
+// indexing so n >= 33 works; consecutive gates share a pass over the state
+// where the tile of one thread and its wave holds their targets.
 
 #include "hq_ops.h"
 
 #include <algorithm>
 #include <cmath>
+#include <new>
 
 namespace hq {
 
@@ -142,6 +144,401 @@ static hq_status launch_plain_gate(hq_state s, const hq_gate& g)
     return HQ_OK;
 }
 
+// ---- runs of gates in one pass -------------------------------------------------------------
+// One gate a pass is bound by HBM (20 qubits and less: by launches, 4 to 6 us each).
+// Here a thread holds 16 amplitudes, four register bits of the index above the
+// wave's six lane bits (index bits 0 to 5, so that every access is a whole run
+// of 64 amplitudes), and a run of gates whose targets are among those ten bits
+// is applied in order; diagonal gates and controls may sit anywhere.  Register
+// targets are pair updates, lane targets one exchange with the partner lane.
+// Every branch is on the run's fields and uniform; controls select.  Random
+// layers, a gate on average, before and after: 10 qubits 3.1 -> 0.74 us, 20
+// qubits complex128 6.2 -> 1.38, 25 qubits 147 -> 17.6 (complex64 62 -> 8.0),
+// 30 qubits 4 890 -> 669.  A pass of 28 or 30 qubits runs at 4.5 TB/s with 11
+// gates; a state of few waves is bound by the chain of a run's gates.
+constexpr int RUN_MAX_RB = 4, RUN_LANES = 6, RUN_GATES = 32;
+constexpr int RUN_MIN_QUBITS = RUN_MAX_RB + RUN_LANES;
+// Up to here 8 amplitudes a thread: fewer gates fit a pass, but a pass is a
+// chain of its gates by one wave or none per SIMD (600 to 300 gates of random
+// layers, us, 8 against 16 amplitudes: 10 qubits 213 / 284, 17 qubits
+// complex64 365 / 434, 20 qubits complex128 840 / 783, 28 qubits 35 600 / 27 400).
+constexpr int RUN_SMALL_QUBITS = 18;
+
+// Passes over the state that gates must cost one by one to share a pass: one
+// of 16 strided runs takes 1.0 to 1.35 of a plain pass, by the strides (28
+// qubits complex128: one H 1.58 ms, two in a run 1.61 to 2.11; two CNOTs, half
+// a pass each, 1.59 one by one and 2.12 in a run, three 2.39 and 2.14).
+constexpr double RUN_MIN_SHARE = 1.35;
+
+enum RunForm : uint32_t { RUN_SWAP, RUN_REAL, RUN_RX, RUN_GEN, RUN_LSWAP, RUN_LREAL, RUN_LGEN, RUN_DIAG };
+
+struct RunFields {
+    uint64_t omask;      // controls outside the register bits
+    uint64_t tbit;       // RUN_DIAG: target outside the register bits; lane forms: the lane's target bit
+    uint32_t form;       // RunForm
+    uint32_t pos;        // register bit of the target; lane forms: its lane bit
+    uint32_t rmask;      // controls among the register bits
+    uint32_t rbit;       // RUN_DIAG: target among the register bits
+
+    __device__ __forceinline__ RunFields uniform() const
+    {
+        RunFields u;
+        const uint32_t* from = (const uint32_t*)this;
+        uint32_t* to = (uint32_t*)&u;
+#pragma unroll
+        for (int i = 0; i < 8; i++) to[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)from[i]);
+        return u;
+    }
+};
+static_assert(sizeof(RunFields) == 32, "RunFields layout");
+
+template <typename R>
+struct alignas(16) RunGate {
+    R m[8];
+    RunFields f;
+};
+
+template <typename R>
+struct Run {
+    RunGate<R> g[RUN_GATES + 1];   // (the last is only read ahead)
+    int num;
+    int pos[RUN_MAX_RB];     // index bit of each register bit, ascending
+};
+static_assert(sizeof(Run<double>) < 4000, "kernel arguments");
+
+template <typename R>
+__device__ __forceinline__ cplx<R> pick(bool c, cplx<R> a, cplx<R> b)
+{
+    cplx<R> r;
+    r.x = c ? a.x : b.x;
+    r.y = c ? a.y : b.y;
+    return r;
+}
+
+// register target P; lane: the lane's controls hold
+template <int CLS, int P, bool CTRL, int RB, typename R>
+__device__ __forceinline__ void run_pairs(cplx<R> (&a)[1 << RB], const R* m, bool lane, uint32_t rmask)
+{
+#pragma unroll
+    for (int j = 0; j < (1 << RB); j++) {
+        if (j & (1 << P)) continue;
+        cplx<R> x = a[j], y = a[j | (1 << P)];
+        pair_update<CLS, R>(x, y, m);
+        const bool on = !CTRL || (lane && ((uint32_t)j & rmask) == rmask);
+        a[j] = pick(on, x, a[j]);
+        a[j | (1 << P)] = pick(on, y, a[j | (1 << P)]);
+    }
+}
+
+template <int P, bool CTRL, int RB, typename R>
+__device__ __forceinline__ void run_reg(cplx<R> (&a)[1 << RB], uint32_t form, const R* m, bool lane, uint32_t rmask)
+{
+    if constexpr (P < RB) {
+    if (form == RUN_SWAP) run_pairs<SHM_SWAP, P, CTRL, RB, R>(a, m, lane, rmask);
+    else if (form == RUN_REAL) run_pairs<SHM_REAL, P, CTRL, RB, R>(a, m, lane, rmask);
+    else if (form == RUN_RX) run_pairs<SHM_RX, P, CTRL, RB, R>(a, m, lane, rmask);
+    else run_pairs<SHM_GEN, P, CTRL, RB, R>(a, m, lane, rmask);
+    }
+}
+
+// x of the lane whose index differs in bit BIT; hi: the lane's bit
+template <int BIT>
+__device__ __forceinline__ uint32_t partner32(uint32_t x, bool hi)
+{
+    if constexpr (BIT == 0) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true);   // quad 1 0 3 2
+    if constexpr (BIT == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xf, 0xf, true);   // quad 2 3 0 1
+    if constexpr (BIT == 2)   // half rows mirrored (xor 7), then quads (xor 3)
+        return (uint32_t)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, true), 0x1B, 0xf,
+                                                  0xf, true);
+    if constexpr (BIT == 3) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x128, 0xf, 0xf, true);  // row rotated by 8
+    // (first: every lane's value at bit clear, second: at bit set)
+    if constexpr (BIT == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return hi ? r[0] : r[1];
+    }
+    if constexpr (BIT == 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return hi ? r[0] : r[1];
+    }
+}
+template <int BIT>
+__device__ __forceinline__ float partner(float x, bool hi)
+{
+    return __uint_as_float(partner32<BIT>(__float_as_uint(x), hi));
+}
+template <int BIT>
+__device__ __forceinline__ double partner(double x, bool hi)
+{
+    return __hiloint2double((int)partner32<BIT>((uint32_t)__double2hiint(x), hi),
+                            (int)partner32<BIT>((uint32_t)__double2loint(x), hi));
+}
+template <int BIT, int N, typename R>
+__device__ __forceinline__ void partners(const cplx<R>* a, cplx<R>* p, bool hi)
+{
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        p[j].x = partner<BIT>(a[j].x, hi);
+        p[j].y = partner<BIT>(a[j].y, hi);
+    }
+}
+
+template <int RB, typename R>
+__global__ __launch_bounds__(256) void k_run(cplx<R>* __restrict__ psi, const Run<R> run)
+{
+    constexpr int NR = 1 << RB;
+    uint64_t base = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < RB; k++) {
+        const int p = run.pos[k];
+        base = ((base >> p) << (p + 1)) | (base & (((uint64_t)1 << p) - 1));
+    }
+    cplx<R>* const at = psi + base;
+    uint64_t off[NR];
+    cplx<R> a[NR];
+#pragma unroll
+    for (int j = 0; j < NR; j++) {
+        off[j] = 0;
+#pragma unroll
+        for (int k = 0; k < RB; k++) if ((j >> k) & 1) off[j] |= (uint64_t)1 << run.pos[k];
+        a[j] = at[off[j]];
+    }
+    auto apply = [&](const R* m, const RunFields& g) {
+        const uint32_t rmask = g.rmask;
+        const bool lane = (base & g.omask) == g.omask;
+        if (g.form <= RUN_GEN) {
+            if ((g.omask | rmask) != 0) {
+                switch (g.pos) {
+                case 0: run_reg<0, true, RB, R>(a, g.form, m, lane, rmask); break;
+                case 1: run_reg<1, true, RB, R>(a, g.form, m, lane, rmask); break;
+                case 2: run_reg<2, true, RB, R>(a, g.form, m, lane, rmask); break;
+                default: run_reg<3, true, RB, R>(a, g.form, m, lane, rmask); break;
+                }
+            } else {
+                switch (g.pos) {
+                case 0: run_reg<0, false, RB, R>(a, g.form, m, lane, rmask); break;
+                case 1: run_reg<1, false, RB, R>(a, g.form, m, lane, rmask); break;
+                case 2: run_reg<2, false, RB, R>(a, g.form, m, lane, rmask); break;
+                default: run_reg<3, false, RB, R>(a, g.form, m, lane, rmask); break;
+                }
+            }
+        } else if (g.form == RUN_DIAG) {
+            // factor of the lane's amplitudes with the register target clear and set
+            const bool hi = (base & g.tbit) != 0;
+            const R lr = lane ? (hi ? m[6] : m[0]) : R(1), li = lane ? (hi ? m[7] : m[1]) : R(0);
+            const R hr = lane ? m[6] : R(1), hi_i = lane ? m[7] : R(0);
+            if ((rmask | g.rbit) == 0) {
+#pragma unroll
+                for (int j = 0; j < NR; j++) {
+                    const R x = a[j].x, y = a[j].y;
+                    a[j].x = lr * x - li * y;
+                    a[j].y = lr * y + li * x;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NR; j++) {
+                    const bool set = ((uint32_t)j & g.rbit) != 0, on = ((uint32_t)j & rmask) == rmask;
+                    const R fr = on ? (set ? hr : lr) : R(1), fi = on ? (set ? hi_i : li) : R(0);
+                    const R x = a[j].x, y = a[j].y;
+                    a[j].x = fr * x - fi * y;
+                    a[j].y = fr * y + fi * x;
+                }
+            }
+        } else {
+            // a lane's amplitude and its partner's, in the order (own, other)
+            const bool hi = (base & g.tbit) != 0;
+            const R or_ = hi ? m[6] : m[0], oi = hi ? m[7] : m[1], pr = hi ? m[4] : m[2], pi = hi ? m[5] : m[3];
+#pragma unroll
+            for (int h = 0; h < NR; h += NR / 2) {
+                cplx<R> p[NR / 2];
+                switch (g.pos) {
+                case 0: partners<0, NR / 2>(a + h, p, hi); break;
+                case 1: partners<1, NR / 2>(a + h, p, hi); break;
+                case 2: partners<2, NR / 2>(a + h, p, hi); break;
+                case 3: partners<3, NR / 2>(a + h, p, hi); break;
+                case 4: partners<4, NR / 2>(a + h, p, hi); break;
+                default: partners<5, NR / 2>(a + h, p, hi); break;
+                }
+                if (g.form == RUN_LREAL) {
+#pragma unroll
+                    for (int j = 0; j < NR / 2; j++) {
+                        p[j].x = or_ * a[h + j].x + pr * p[j].x;
+                        p[j].y = or_ * a[h + j].y + pr * p[j].y;
+                    }
+                } else if (g.form == RUN_LGEN) {
+#pragma unroll
+                    for (int j = 0; j < NR / 2; j++) {
+                        const cplx<R> o = a[h + j], t = p[j];
+                        p[j].x = or_ * o.x - oi * o.y + (pr * t.x - pi * t.y);
+                        p[j].y = or_ * o.y + oi * o.x + (pr * t.y + pi * t.x);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < NR / 2; j++) {
+                    const bool on = lane && ((uint32_t)(h + j) & rmask) == rmask;
+                    a[h + j] = pick(on, p[j], a[h + j]);
+                }
+            }
+        }
+    };
+    if constexpr (RB < RUN_MAX_RB) {
+        // Few waves: the gates go to LDS in one latency instead of one per
+        // gate.  (With 16 amplitudes a thread the barrier costs more than
+        // that at size: 30 qubits 7.9 against 7.5 ms a pass.)
+        __shared__ RunGate<R> gates[RUN_GATES];
+        for (uint32_t t = threadIdx.x; t < (uint32_t)run.num * (sizeof(RunGate<R>) / 16); t += blockDim.x)
+            ((uint4*)gates)[t] = ((const uint4*)run.g)[t];
+        __syncthreads();
+        for (int q = 0; q < run.num; q++) apply(gates[q].m, gates[q].f.uniform());
+    } else {
+        RunGate<R> next = run.g[0];
+        for (int q = 0; q < run.num; q++) {
+            const RunGate<R> g = next;
+            next = run.g[q + 1];     // read while this one is applied
+            apply(g.m, g.f);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NR; j++) at[off[j]] = a[j];
+}
+
+// Share of the state that k_plain moves for a gate: the pairs whose controls
+// are set, half of each for a phase
+static double plain_share(const hq_gate& g)
+{
+    double f = classify_gate(g) == SHM_PHASE ? 0.5 : 1.0;
+    if (g.control >= 0) f *= 0.5;
+    if (g.control2 >= 0) f *= 0.5;
+    return f;
+}
+
+static bool run_diagonal(int cls) { return cls == SHM_DIAG || cls == SHM_PHASE; }
+
+struct PlainGate {
+    int index;           // in the call's array
+    bool done;
+    uint64_t qubits;     // target and controls
+    uint64_t reg;        // the register bit it needs, 0 for lane targets and diagonal gates
+    double share;
+};
+
+// The gates of the next pass, in order: those among the next RUN_AHEAD that
+// share no qubit with a gate left out before them (so that they commute with
+// it) and whose targets fit.  1350 gates of random layers on 30 qubits need 89
+// passes, 190 without looking past the first gate that does not fit.
+constexpr size_t RUN_AHEAD = 256;
+
+static void next_run(int rb, std::vector<PlainGate>& list, size_t first, uint64_t all, std::vector<int>* members,
+                     uint64_t* regs, double* share)
+{
+    members->clear();
+    *regs = 0;
+    *share = 0;
+    uint64_t blocked = 0;
+    const size_t end = std::min(list.size(), first + RUN_AHEAD);
+    for (size_t i = first; i < end && blocked != all && (int)members->size() < RUN_GATES; i++) {
+        PlainGate& g = list[i];
+        if (g.done) continue;
+        if ((g.qubits & blocked) || __builtin_popcountll(*regs | g.reg) > rb) {
+            blocked |= g.qubits;
+            continue;
+        }
+        *regs |= g.reg;
+        g.done = true;
+        members->push_back(g.index);
+        *share += g.share;
+    }
+}
+
+template <int RB, typename R>
+static hq_status launch_run(hq_state s, const hq_gate* gates, const std::vector<int>& members, uint64_t regs)
+{
+    // register bits without a target: the highest free ones
+    for (int q = s->n - 1; __builtin_popcountll(regs) < RB; q--) regs |= (uint64_t)1 << q;
+    Run<R> run = {};
+    int bit_of[64], k = 0;
+    for (int q = 0; q < s->n; q++) {
+        bit_of[q] = -1;
+        if (regs >> q & 1) { run.pos[k] = q; bit_of[q] = k++; }
+    }
+    run.num = 0;
+    for (int i : members) {
+        const hq_gate& g = gates[i];
+        const int cls = classify_gate(g);
+        RunGate<R>& rg = run.g[run.num++];
+        RunFields& o = rg.f;
+        for (int j = 0; j < 8; j++) rg.m[j] = (R)g.mat[j];
+        o.omask = o.tbit = 0;
+        o.pos = o.rmask = o.rbit = 0;
+        for (int c : {g.control, g.control2}) {
+            if (c < 0) continue;
+            if (bit_of[c] >= 0) o.rmask |= 1u << bit_of[c];
+            else o.omask |= (uint64_t)1 << c;
+        }
+        const int rb = bit_of[g.target];
+        if (run_diagonal(cls)) {
+            o.form = RUN_DIAG;
+            if (cls == SHM_PHASE) { rg.m[0] = R(1); rg.m[1] = R(0); }
+            if (rb >= 0) o.rbit = 1u << rb;
+            else o.tbit = (uint64_t)1 << g.target;
+        } else if (rb >= 0) {
+            o.form = cls == SHM_SWAP ? RUN_SWAP : cls == SHM_REAL ? RUN_REAL : cls == SHM_RX ? RUN_RX : RUN_GEN;
+            o.pos = (uint32_t)rb;
+        } else {
+            o.form = cls == SHM_SWAP ? RUN_LSWAP : cls == SHM_REAL ? RUN_LREAL : RUN_LGEN;
+            o.pos = (uint32_t)g.target;
+            o.tbit = (uint64_t)1 << g.target;
+        }
+    }
+    const uint64_t threads = s->amps >> RB, block = std::min<uint64_t>(threads, 256);
+    hipLaunchKernelGGL((k_run<RB, R>), dim3((unsigned)(threads / block)), dim3((unsigned)block), 0, s->stream,
+                       (cplx<R>*)s->data, run);
+    HQ_HIP(hipGetLastError());
+    return HQ_OK;
+}
+
+template <typename R>
+static hq_status apply_plain(hq_state s, const hq_gate* gates, int num)
+{
+    if (s->n < RUN_MIN_QUBITS || num == 1) {
+        for (int i = 0; i < num; i++) {
+            if (gates[i].type == HQ_ID) continue;
+            hq_status st = launch_plain_gate<R>(s, gates[i]);
+            if (st != HQ_OK) return st;
+        }
+        return HQ_OK;
+    }
+    std::vector<PlainGate> list;
+    list.reserve((size_t)num);
+    for (int i = 0; i < num; i++) {
+        const hq_gate& g = gates[i];
+        if (g.type == HQ_ID) continue;
+        PlainGate p{i, false, (uint64_t)1 << g.target, 0, plain_share(g)};
+        for (int c : {g.control, g.control2})
+            if (c >= 0) p.qubits |= (uint64_t)1 << c;
+        if (g.target >= RUN_LANES && !run_diagonal(classify_gate(g))) p.reg = (uint64_t)1 << g.target;
+        list.push_back(p);
+    }
+    const uint64_t all = ((uint64_t)1 << s->n) - 1;
+    // a launch costs what 20 MB of traffic do, in passes over the state
+    const double launch = 20e6 / (2.0 * (double)s->amps * sizeof(cplx<R>));
+    const int rb = s->n <= RUN_SMALL_QUBITS ? 3 : 4;
+    std::vector<int> members;
+    for (size_t first = 0;;) {
+        while (first < list.size() && list[first].done) first++;
+        if (first == list.size()) return HQ_OK;
+        uint64_t regs;
+        double share;
+        next_run(rb, list, first, all, &members, &regs, &share);
+        hq_status st = HQ_OK;
+        if (members.size() > 1 && share + (double)(members.size() - 1) * launch > RUN_MIN_SHARE) {
+            st = rb == 3 ? launch_run<3, R>(s, gates, members, regs) : launch_run<4, R>(s, gates, members, regs);
+        } else {
+            for (size_t k = 0; k < members.size() && st == HQ_OK; k++) st = launch_plain_gate<R>(s, gates[members[k]]);
+        }
+        if (st != HQ_OK) return st;
+    }
+}
+
 }  // namespace hq
 
 using namespace hq;
@@ -157,10 +554,13 @@ extern "C" hq_status hq_apply_gates_plain(hq_state s, const hq_gate* gates, int 
     int slot;
     hq_status st = prof_begin(s, 0, &slot);
     if (st != HQ_OK) return st;
-    for (int i = 0; i < num_gates; i++) {
-        if (gates[i].type == HQ_ID) continue;
-        st = s->precision == HQ_C128 ? launch_plain_gate<double>(s, gates[i]) : launch_plain_gate<float>(s, gates[i]);
-        if (st != HQ_OK) return st;
+    try {
+        st = s->precision == HQ_C128 ? apply_plain<double>(s, gates, num_gates)
+                                     : apply_plain<float>(s, gates, num_gates);
+    } catch (const std::bad_alloc&) {
+        set_error("hq_apply_gates_plain: out of host memory");
+        return HQ_ERR_OOM;
     }
+    if (st != HQ_OK) return st;
     return prof_end(s, slot);
 }

@@ -133,8 +133,10 @@ hq_status hq_state_info(hq_state s, int *num_qubits, int *precision);
 /* Whether the state was created with a work buffer (TransMM groups need one). */
 hq_status hq_state_has_buffer(hq_state s, int *has_buffer);
 
-/* Plain method: one HBM pass per gate, in order (kernelExecSimple,
- * src/kernelSimple.cu:335-446).  Asynchronous. */
+/* Plain method: the gates one after another, without a plan (kernelExecSimple,
+ * src/kernelSimple.cu:335-446, which makes one HBM pass per gate; here gates
+ * whose targets fit a wave's tile share a pass, in order up to gates without a
+ * common qubit).  Asynchronous. */
 hq_status hq_apply_gates_plain(hq_state s, const hq_gate *gates, int num_gates);
 
 /* OShareMem group: compile the gates (physical qubits) into a device-resident
