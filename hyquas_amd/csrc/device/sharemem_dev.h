@@ -178,16 +178,18 @@ __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const c
     constexpr int WIN_BYTES = shm_window_slots<R>() * SLOT;
     constexpr int PIECES = SHM_WINDOW_COPY / (16 * NT);
     const HQ_GLOBAL char* __restrict__ slots = prog + SHM_PROG_HEADER;
-    uint4 piece[PIECES];
+    // (a native vector: uint4's copies of unread pieces went to scratch memory in half of the shapes)
+    typedef uint32_t Piece __attribute__((ext_vector_type(4)));
+    Piece piece[PIECES];
     auto fetch = [&](uint32_t from) {
 #pragma unroll
         for (int i = 0; i < PIECES; i++)
             if (i == 0 || from + (uint32_t)(i * NT) * 16u < nbytes)
-                piece[i] = *(const HQ_GLOBAL uint4*)(slots + from + (uint32_t)(i * NT + tid) * 16u);
+                piece[i] = *(const HQ_GLOBAL Piece*)(slots + from + (uint32_t)(i * NT + tid) * 16u);
     };
     auto fill = [&]() {
 #pragma unroll
-        for (int i = 0; i < PIECES; i++) *(uint4*)(win + (uint32_t)(i * NT + tid) * 16u) = piece[i];
+        for (int i = 0; i < PIECES; i++) *(Piece*)(win + (uint32_t)(i * NT + tid) * 16u) = piece[i];
     };
 
     cplx<R> a[NR];
