@@ -152,10 +152,10 @@ static hq_status launch_plain_gate(hq_state s, const hq_gate& g)
 // is applied in order; diagonal gates and controls may sit anywhere.  Register
 // targets are pair updates, lane targets one exchange with the partner lane.
 // Every branch is on the run's fields and uniform; controls select.  Random
-// layers, a gate on average, before and after: 10 qubits 3.1 -> 0.74 us, 20
-// qubits complex128 6.2 -> 1.38, 25 qubits 147 -> 17.6 (complex64 62 -> 8.0),
-// 30 qubits 4 890 -> 669.  A pass of 28 or 30 qubits runs at 4.5 TB/s with 11
-// gates; a state of few waves is bound by the chain of a run's gates.
+// layers, a gate on average, before and after: 10 qubits 3.1 -> 0.69 us, 20
+// qubits complex128 6.2 -> 1.31, 25 qubits 147 -> 16.8 (complex64 62 -> 7.5),
+// 30 qubits 4 890 -> 647.  A pass of 30 qubits runs at 4.7 TB/s with 11 gates;
+// a state of few waves is bound by the chain of a run's gates.
 constexpr int RUN_MAX_RB = 4, RUN_LANES = 6, RUN_GATES = 32;
 constexpr int RUN_MIN_QUBITS = RUN_MAX_RB + RUN_LANES;
 // Up to here 8 amplitudes a thread: fewer gates fit a pass, but a pass is a
@@ -170,7 +170,7 @@ constexpr int RUN_SMALL_QUBITS = 18;
 // a pass each, 1.59 one by one and 2.12 in a run, three 2.39 and 2.14).
 constexpr double RUN_MIN_SHARE = 1.35;
 
-enum RunForm : uint32_t { RUN_SWAP, RUN_REAL, RUN_RX, RUN_GEN, RUN_LSWAP, RUN_LREAL, RUN_LGEN, RUN_DIAG };
+enum RunForm : uint32_t { RUN_SWAP, RUN_REAL, RUN_RX, RUN_GEN, RUN_LSWAP, RUN_LREAL, RUN_LRX, RUN_LGEN, RUN_DIAG };
 
 struct RunFields {
     uint64_t omask;      // controls outside the register bits
@@ -178,7 +178,8 @@ struct RunFields {
     uint32_t form;       // RunForm
     uint32_t pos;        // register bit of the target; lane forms: its lane bit
     uint32_t rmask;      // controls among the register bits
-    uint32_t rbit;       // RUN_DIAG: target among the register bits
+    uint32_t rbit : 31;  // RUN_DIAG: target among the register bits
+    uint32_t phase : 1;  // RUN_DIAG: the factor is 1 where the target is clear
 
     __device__ __forceinline__ RunFields uniform() const
     {
@@ -238,6 +239,25 @@ __device__ __forceinline__ void run_reg(cplx<R> (&a)[1 << RB], uint32_t form, co
     else if (form == RUN_REAL) run_pairs<SHM_REAL, P, CTRL, RB, R>(a, m, lane, rmask);
     else if (form == RUN_RX) run_pairs<SHM_RX, P, CTRL, RB, R>(a, m, lane, rmask);
     else run_pairs<SHM_GEN, P, CTRL, RB, R>(a, m, lane, rmask);
+    }
+}
+
+// amplitudes with register bit P clear *= l, set *= h (P < 0: all *= l); phase: l is 1
+template <int RB, int P, typename R>
+__device__ __forceinline__ void run_scale(cplx<R> (&a)[1 << RB], R lr, R li, R hr, R hi, bool phase)
+{
+    if constexpr (P < RB) {
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            if (half == 0 && phase) continue;
+#pragma unroll
+            for (int j = 0; j < (1 << RB); j++) {
+                if (P < 0 ? half != 0 : ((j >> (P < 0 ? 0 : P)) & 1) != half) continue;
+                const R x = a[j].x, y = a[j].y, fr = half ? hr : lr, fi = half ? hi : li;
+                a[j].x = fr * x - fi * y;
+                a[j].y = fr * y + fi * x;
+            }
+        }
     }
 }
 
@@ -326,12 +346,13 @@ __global__ __launch_bounds__(256) void k_run(cplx<R>* __restrict__ psi, const Ru
             const bool hi = (base & g.tbit) != 0;
             const R lr = lane ? (hi ? m[6] : m[0]) : R(1), li = lane ? (hi ? m[7] : m[1]) : R(0);
             const R hr = lane ? m[6] : R(1), hi_i = lane ? m[7] : R(0);
-            if ((rmask | g.rbit) == 0) {
-#pragma unroll
-                for (int j = 0; j < NR; j++) {
-                    const R x = a[j].x, y = a[j].y;
-                    a[j].x = lr * x - li * y;
-                    a[j].y = lr * y + li * x;
+            if (rmask == 0) {
+                switch (g.rbit) {
+                case 0: run_scale<RB, -1>(a, lr, li, hr, hi_i, false); break;
+                case 1: run_scale<RB, 0>(a, lr, li, hr, hi_i, g.phase != 0); break;
+                case 2: run_scale<RB, 1>(a, lr, li, hr, hi_i, g.phase != 0); break;
+                case 4: run_scale<RB, 2>(a, lr, li, hr, hi_i, g.phase != 0); break;
+                default: run_scale<RB, 3>(a, lr, li, hr, hi_i, g.phase != 0); break;
                 }
             } else {
 #pragma unroll
@@ -364,6 +385,13 @@ __global__ __launch_bounds__(256) void k_run(cplx<R>* __restrict__ psi, const Ru
                         p[j].x = or_ * a[h + j].x + pr * p[j].x;
                         p[j].y = or_ * a[h + j].y + pr * p[j].y;
                     }
+                } else if (g.form == RUN_LRX) {
+#pragma unroll
+                    for (int j = 0; j < NR / 2; j++) {
+                        const cplx<R> t = p[j];
+                        p[j].x = or_ * a[h + j].x - pi * t.y;
+                        p[j].y = or_ * a[h + j].y + pi * t.x;
+                    }
                 } else if (g.form == RUN_LGEN) {
 #pragma unroll
                     for (int j = 0; j < NR / 2; j++) {
@@ -372,10 +400,15 @@ __global__ __launch_bounds__(256) void k_run(cplx<R>* __restrict__ psi, const Ru
                         p[j].y = or_ * o.y + oi * o.x + (pr * t.y + pi * t.x);
                     }
                 }
+                if ((g.omask | rmask) == 0) {
 #pragma unroll
-                for (int j = 0; j < NR / 2; j++) {
-                    const bool on = lane && ((uint32_t)(h + j) & rmask) == rmask;
-                    a[h + j] = pick(on, p[j], a[h + j]);
+                    for (int j = 0; j < NR / 2; j++) a[h + j] = p[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < NR / 2; j++) {
+                        const bool on = lane && ((uint32_t)(h + j) & rmask) == rmask;
+                        a[h + j] = pick(on, p[j], a[h + j]);
+                    }
                 }
             }
         }
@@ -468,7 +501,7 @@ static hq_status launch_run(hq_state s, const hq_gate* gates, const std::vector<
         RunFields& o = rg.f;
         for (int j = 0; j < 8; j++) rg.m[j] = (R)g.mat[j];
         o.omask = o.tbit = 0;
-        o.pos = o.rmask = o.rbit = 0;
+        o.pos = o.rmask = o.rbit = o.phase = 0;
         for (int c : {g.control, g.control2}) {
             if (c < 0) continue;
             if (bit_of[c] >= 0) o.rmask |= 1u << bit_of[c];
@@ -477,14 +510,14 @@ static hq_status launch_run(hq_state s, const hq_gate* gates, const std::vector<
         const int rb = bit_of[g.target];
         if (run_diagonal(cls)) {
             o.form = RUN_DIAG;
-            if (cls == SHM_PHASE) { rg.m[0] = R(1); rg.m[1] = R(0); }
+            if (cls == SHM_PHASE) { rg.m[0] = R(1); rg.m[1] = R(0); o.phase = 1; }
             if (rb >= 0) o.rbit = 1u << rb;
             else o.tbit = (uint64_t)1 << g.target;
         } else if (rb >= 0) {
             o.form = cls == SHM_SWAP ? RUN_SWAP : cls == SHM_REAL ? RUN_REAL : cls == SHM_RX ? RUN_RX : RUN_GEN;
             o.pos = (uint32_t)rb;
         } else {
-            o.form = cls == SHM_SWAP ? RUN_LSWAP : cls == SHM_REAL ? RUN_LREAL : RUN_LGEN;
+            o.form = cls == SHM_SWAP ? RUN_LSWAP : cls == SHM_REAL ? RUN_LREAL : cls == SHM_RX ? RUN_LRX : RUN_LGEN;
             o.pos = (uint32_t)g.target;
             o.tbit = (uint64_t)1 << g.target;
         }
