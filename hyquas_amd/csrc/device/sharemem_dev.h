@@ -138,10 +138,11 @@ __device__ __forceinline__ void zsums(uint64_t idx, int n, double* z, double* zz
 // and dispatch: read from HBM through the scalar cache, each op's fields were
 // three dependent misses.  Slots are copied to
 // LDS a window at a time, together with the tile's loads, and the next slot is
-// read while one executes.  With diagonal gates merged on top, passes of the
-// 17-qubit complex64 and 20-qubit complex128 random circuits (32 and 256
-// blocks) went from 61 and 67.5 us to 37 and 38 us, the 174 gates of a
-// 10-qubit ansatz (one wave) from 132 to 51 us.
+// read while one executes.  With diagonal gates merged, uniform branches, one
+// switch for the frequent updates and 8 amplitudes a thread on top, passes of
+// the 17-qubit complex64 and 20-qubit complex128 random circuits (32 and 256
+// blocks) went from 61 and 67.5 us to 24 and 31 us, the 174 gates of a
+// 10-qubit ansatz from 132 to 34.5 us.
 template <typename R, int RB, int TB, bool PRECISE>
 __device__ __forceinline__ void tile_pass(cplx<R>* __restrict__ psi_any, const char* __restrict__ prog_any,
                                           uint64_t blk, cplx<R>* __restrict__ lds, char* __restrict__ win,
