@@ -251,7 +251,10 @@ struct Emitter {
         return true;
     }
 
-    // factor of a diagonal op: literals, or two runtime coefficients
+    // Factor of a diagonal op: literals, or two runtime coefficients, loaded
+    // here (kr, ki) for every lane.  A load inside a lane's `pc ? .. : 1` is a
+    // branch to the compiler, with copies of every amplitude at its join (QFT,
+    // complex64: 100 spilled registers in a kernel; 24 qubits 246 us so, 208).
     void factor(const ShmOp& op, std::string* fr, std::string* fi)
     {
         if (op.flags & SHM_FLAG_CONST) {
@@ -262,8 +265,9 @@ struct Emitter {
         const size_t base = coef->size();
         coef->push_back(op.m[0]);
         coef->push_back(op.m[1]);
-        *fr = "cf[" + std::to_string(base) + "]";
-        *fi = "cf[" + std::to_string(base + 1) + "]";
+        o << "      const R kr = cf[" << base << "], ki = cf[" << base + 1 << "];\n";
+        *fr = "kr";
+        *fi = "ki";
     }
 
     // by the sum of two floats (precise complex64 plans): four operations more
@@ -351,10 +355,11 @@ struct Emitter {
         }
         const bool real = op.flags & SHM_FLAG_REAL;
         std::string fr, fi, pc;
+        o << "    {\n";
         factor(op, &fr, &fi);
         if (op.cblk) pc = "(b & " + hex64(op.cblk) + ") == " + hex64(op.cblkv);
         if (op.cthr) pc += std::string(pc.empty() ? "" : " && ") + "(t & " + hex32(op.cthr) + ") == " + hex32(op.cthrv);
-        o << "    {\n      const bool pc = " << pc << ";\n      const R fr = pc ? " << fr << " : (R)1;\n";
+        o << "      const bool pc = " << pc << ";\n      const R fr = pc ? " << fr << " : (R)1;\n";
         if (real) {
             o << "      " << lx << " *= fr;";
             if (lane == LANE_CPLX) o << " " << ly << " *= fr;";

@@ -4,7 +4,7 @@ import re
 
 import pytest
 
-from helpers import CNOT, H, to_oracle
+from helpers import CNOT, CU1, H, RZ, to_oracle
 
 N, MASK = 13, (1 << 13) - 1
 
@@ -26,3 +26,15 @@ def test_x_under_a_thread_bit_control(hq, prec, variant):
     assert "const bool pc" in src
     assert (len(selects) > 0) == (prec == 1)
     assert (len(updates) > 0) == (prec == 0)
+
+
+@pytest.mark.parametrize("variant", [0, 1, 4, 20])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_factors_of_diagonal_gates_are_loaded_outside_conditions(hq, prec, variant):
+    """A coefficient loaded where a lane's condition selects it is a branch, with
+    copies of every amplitude at its join."""
+    spec = [(H, q, -1) for q in range(N)]
+    spec += [(CU1, t, c, (0.1 + t + c,)) for t in range(N) for c in range(t)] + [(RZ, q, -1, (0.3,)) for q in range(N)]
+    src = _source(hq, spec, prec, variant)
+    assert "? kr : (R)1" in src
+    assert not re.search(r"\? *cf\[", src)
