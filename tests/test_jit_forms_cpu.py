@@ -38,3 +38,17 @@ def test_factors_of_diagonal_gates_are_loaded_outside_conditions(hq, prec, varia
     src = _source(hq, spec, prec, variant)
     assert "? kr : (R)1" in src
     assert not re.search(r"\? *cf\[", src)
+
+
+@pytest.mark.parametrize("variant", [0, 1, 4, 20])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_diagonal_gates_across_block_bits_do_not_branch(hq, prec, variant):
+    """A gate on a register bit and a block bit touches half a thread's
+    amplitudes: its factor is selected by the block, without a branch around them."""
+    n = 18
+    spec = [(H, q, -1) for q in range(N)]
+    spec += [(CU1, t, c, (0.1 + t + c,)) for t in range(N) for c in range(N, n)]
+    spec += [(CU1, c, t, (0.2 + t + c,)) for t in range(N) for c in range(N, n)] + [(H, q, -1) for q in range(N)]
+    src = _source(hq, spec, prec, variant, n)
+    assert re.search(r"pc = \(b & 0x[0-9a-f]+ull\) == 0x[0-9a-f]+ull;", src)
+    assert "if ((b & " not in src
