@@ -436,12 +436,11 @@ struct Emitter {
         default: break;
         }
         // X, CNOT and CCX have no coefficients.  Under a thread-bit control
-        // they are selects in complex64, half the operations of the update
-        // with per-lane 0 and 1, and that update in complex128, where both
-        // forms take eight (30 qubits, 30 random layers: 156.9 ms by selects, 152.1;
-        // 24 qubits, 24 layers: 1.75 and 1.64).  Measured on complex64 circuits
-        // of 23 to 31 qubits the two are within 3 % of each other either way.
-        const bool lane_update = op.cls == SHM_SWAP && op.cthr && !f32;
+        // they are the update with per-lane 0 and 1: by selects, fewer operations
+        // in complex64 and as many in complex128, 24 qubits take 1.00 ms instead of
+        // 0.97 (complex64, 24 random layers) and 1.75 instead of 1.64 (complex128),
+        // 30 qubits complex128 with 30 layers 156.0 instead of 151.1.
+        const bool lane_update = op.cls == SHM_SWAP && op.cthr;
         const int cls = lane_update ? (int)SHM_REAL : (int)op.cls;
         std::vector<std::string> m = lane_update ? std::vector<std::string>{"(R)0", "", "(R)1", "", "(R)1", "", "(R)0", ""}
                                      : op.cls == SHM_SWAP ? std::vector<std::string>(8) : coeffs(op);
@@ -468,7 +467,7 @@ struct Emitter {
                 }
             }
         }
-        const bool rename = identity_ok_renaming && !blockc && !op.cthr;
+        const bool rename = identity_ok_renaming && !blockc;
         // the shear forms come from uncontrolled gates only; a per-lane
         // identity select would not express the identity for them
         if (op.cthr && (op.cls == SHM_SHEAR || op.cls == SHM_SHEARX))
@@ -482,10 +481,6 @@ struct Emitter {
                 switch (cls) {
                 case SHM_SWAP:
                     if (rename) std::swap(name[j], name[jh]);
-                    else if (op.cthr)
-                        o << "      { const C lo = " << r(j) << ", hi = " << r(jh) << "; "
-                          << r(j) << ".x = pc ? hi.x : lo.x; " << r(j) << ".y = pc ? hi.y : lo.y; "
-                          << r(jh) << ".x = pc ? lo.x : hi.x; " << r(jh) << ".y = pc ? lo.y : hi.y; }\n";
                     else o << "      { const C tmp = " << r(j) << "; " << r(j) << " = " << r(jh) << "; " << r(jh) << " = tmp; }\n";
                     break;
                 case SHM_Y:

@@ -16,16 +16,12 @@ def _source(hq, spec, prec=0, variant=0, n=N, mask=MASK):
 @pytest.mark.parametrize("variant", [0, 1, 4, 20])
 @pytest.mark.parametrize("prec", [0, 1])
 def test_x_under_a_thread_bit_control(hq, prec, variant):
-    """Selects in complex64, in complex128 the 2x2 update with per-lane 0 and 1:
-    both take eight operations a pair there, and the kernels of 22 to 25 qubits
-    were 2 to 4 % slower by selects."""
+    """The 2x2 update with per-lane 0 and 1: by selects, the kernels of 22 to 31
+    qubits were up to 4 % slower."""
     spec = [(H, q, -1) for q in range(N)] + [(CNOT, t, c) for t in range(4) for c in range(6, 12)]
     src = _source(hq, spec, prec, variant)
-    selects = re.findall(r"= pc \? hi\.x : lo\.x", src)
-    updates = re.findall(r"const R m0 = pc \? \(R\)0 : \(R\)1", src)
-    assert "const bool pc" in src
-    assert (len(selects) > 0) == (prec == 1)
-    assert (len(updates) > 0) == (prec == 0)
+    assert re.search(r"const R m0 = pc \? \(R\)0 : \(R\)1", src)
+    assert not re.search(r"= pc \? hi\.x : lo\.x", src)
 
 
 @pytest.mark.parametrize("variant", [0, 1, 4, 20])
