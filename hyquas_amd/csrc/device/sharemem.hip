@@ -872,7 +872,8 @@ struct Encoder {
                 break;
             }
             case SHM_MIX:
-                if (!o.cblk && o.creg == o.cregv && !(o.creg & (o.creg - 1)))
+                // (a factor on no register bit is every amplitude's)
+                if (!o.cblk && o.creg && o.creg == o.cregv && !(o.creg & (o.creg - 1)))
                     op(head(o, 8 * __builtin_ctz(o.creg) + DIRECT_LPHASE), o.m, 2);
                 else
                     op(head(o, (o.flags & SHM_FLAG_REAL) && o.m[0] == -1.0 ? SLOT_MIXSIGN : SLOT_MIX), o.m, 2);
