@@ -59,7 +59,7 @@ struct hq_state_s {
     char* d_ws = nullptr;     // readout workspace (device, pinned host), see ensure_ws
     char* h_ws = nullptr;
     size_t ws_dev = 0, ws_host = 0;   // bytes
-    std::mutex ws_mu;         // held by a readout from ensure_ws until it has its results
+    std::mutex ws_mu;         // held by a readout from its use of d_red, h_red or the workspace until it has its results
     bool profiling = false;
     std::vector<hq::ProfileEntry> prof;
     std::vector<hipEvent_t> free_events;

@@ -346,6 +346,9 @@ static hq_status noalloc_scratch(int device, double** out)
     return HQ_OK;
 }
 
+// Room in the state's reduction buffers; the caller holds ws_mu until it has read
+// its results out of h_red (growing frees the buffers, and every readout writes
+// to their start).
 static hq_status ensure_red(hq_state s, size_t doubles)
 {
     if (s->red_cap >= doubles) return HQ_OK;
@@ -554,6 +557,7 @@ hq_status hq_state_get_amp(hq_state s, uint64_t index, double* re, double* im)
 {
     HQ_CHECK(s && re && im, HQ_ERR_ARG, "hq_state_get_amp: null argument");
     HQ_CHECK(index < s->amps, HQ_ERR_ARG, "hq_state_get_amp: index out of range");
+    std::lock_guard<std::mutex> lock(s->ws_mu);
     hq_status st = ensure_red(s, 2);
     if (st != HQ_OK) return st;
     HQ_HIP(hipMemcpyAsync(s->h_red, (char*)s->data + index * s->amp_bytes, s->amp_bytes,
@@ -580,6 +584,7 @@ static hq_status sum_partials(hq_state s, int count, int stride, int offset, dou
 
 static hq_status run_norm(hq_state s, int target, double* out)
 {
+    std::lock_guard<std::mutex> lock(s->ws_mu);
     hq_status st = ensure_red(s, RED_BLOCKS);
     if (st != HQ_OK) return st;
     unsigned g = grid_for(s->amps, RED_THREADS, RED_BLOCKS);
@@ -662,6 +667,7 @@ hq_status hq_expect_z(hq_state s, double* z, double* zz)
 {
     HQ_CHECK(s, HQ_ERR_ARG, "hq_expect_z: null state");
     HQ_CHECK(s->n <= RED_MAXQ, HQ_ERR_UNSUPPORTED, "hq_expect_z: at most 36 qubits");
+    std::lock_guard<std::mutex> lock(s->ws_mu);
     hq_status st = ensure_red(s, (size_t)RED_Z_BLOCKS * RED_Z_STRIDE);
     if (st != HQ_OK) return st;
     // the sums go straight to the pinned buffer: no copy to wait for
@@ -697,6 +703,7 @@ hq_status hq_state_inner(hq_state a, hq_state b, double* re, double* im)
     HQ_CHECK(a->n == b->n, HQ_ERR_ARG, "hq_state_inner: qubit counts differ");
     HQ_HIP(hipStreamSynchronize(b->stream));
     unsigned g = grid_for(a->amps, RED_THREADS, RED_BLOCKS);
+    std::lock_guard<std::mutex> lock(a->ws_mu);
     hq_status st = ensure_red(a, 2 * (size_t)g);
     if (st != HQ_OK) return st;
     if (a->precision == HQ_C128 && b->precision == HQ_C128)

@@ -144,3 +144,26 @@ def test_threads_share_a_state(gpu):
     with ThreadPoolExecutor(4) as ex:
         assert list(ex.map(run, jobs * 2)) == want * 2
     s.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_threads_read_a_fresh_state(gpu, prec):
+    """Every kind of readout of one state from several threads at a time, the
+    first of them growing its buffers, gives what one thread gets."""
+    from concurrent.futures import ThreadPoolExecutor
+    n = 15
+    kinds = [lambda s: s.norm2(), lambda s: s.get_amp(12345), lambda s: [x.tolist() for x in map(np.asarray, s.expect_z())],
+             lambda s: s.measure_zero(3), lambda s: s.inner(s), lambda s: s.measure_zero(n - 1),
+             lambda s: s.get_amp(7), lambda s: [np.asarray(x).tolist() for x in s.topk(16)],
+             lambda s: s.sample(300, 2).tolist()]
+    ref, _ = _state(gpu, n, prec, 12)
+    want = [k(ref) for k in kinds]
+    ref.close()
+    for first in range(len(kinds)):
+        s, _ = _state(gpu, n, prec, 12)
+        order = [(first + i) % len(kinds) for i in range(len(kinds))] * 4
+        with ThreadPoolExecutor(4) as ex:
+            got = list(ex.map(lambda k: kinds[k](s), order))
+        s.close()
+        for k, g in zip(order, got):
+            assert g == want[k], (first, k)
