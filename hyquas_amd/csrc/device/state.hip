@@ -57,14 +57,16 @@ __device__ inline double block_sum(double v, double* sh)
 // Kahan-compensated FP64 accumulation of |a_i|^2 over a subset (bit `target`
 // clear when target >= 0: the subset's elements are numbered, nothing of the
 // rest is read), one partial per block (measure<>/reduce<>,
-// kernelSimple.cu:448-495).  Four independent 16-byte loads per thread and
-// step: one 8-byte load at a time read a 2 GiB complex64 state at 3.4 TB/s, this
-// reads it at 5.4 TB/s.
+// kernelSimple.cu:448-495).  Bound by HBM: independent 16-byte loads per thread and
+// step.  Complex64 takes four (one 8-byte load at a time read a 2 GiB state in 0.65
+// ms, this in 0.42), complex128 two (26 and 28 qubits: one load 206 and 866 us,
+// two 197 and 774, four 217 and 836; 24 qubits 53, 54.5 and 56).
 template <typename R>
 __global__ __launch_bounds__(RED_THREADS) void k_norm(const cplx<R>* __restrict__ a, uint64_t n_amps, int target,
                                                       double* __restrict__ out)
 {
     constexpr int E = 16 / (2 * (int)sizeof(R));   // amplitudes per 16-byte element
+    constexpr int U = E == 2 ? 4 : 2;              // loads per thread and step
     struct alignas(16) Elem { cplx<R> v[E]; };
     __shared__ double sh[16];
     double s = 0, c = 0;
@@ -83,12 +85,12 @@ __global__ __launch_bounds__(RED_THREADS) void k_norm(const cplx<R>* __restrict_
     auto at = [&](uint64_t i) { return tb < 0 ? i : (i >> tb) << (tb + 1) | (i & (((uint64_t)1 << tb) - 1)); };
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; i + 3 * stride < elems; i += 4 * stride) {
-        Elem v[4];
+    for (; i + (U - 1) * stride < elems; i += U * stride) {
+        Elem v[U];
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = src[at(i + (uint64_t)k * stride)];
+        for (int k = 0; k < U; k++) v[k] = src[at(i + (uint64_t)k * stride)];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < U; k++) {
             add(v[k].v[0]);
             if constexpr (E == 2) { if (!inside) add(v[k].v[1]); }
         }
