@@ -188,12 +188,11 @@ struct RunFields {
 
     __device__ __forceinline__ RunFields uniform() const
     {
-        RunFields u;
-        const uint32_t* from = (const uint32_t*)this;
-        uint32_t* to = (uint32_t*)&u;
+        struct Words { uint32_t w[8]; };
+        Words u = __builtin_bit_cast(Words, *this);
 #pragma unroll
-        for (int i = 0; i < 8; i++) to[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)from[i]);
-        return u;
+        for (int i = 0; i < 8; i++) u.w[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)u.w[i]);
+        return __builtin_bit_cast(RunFields, u);
     }
 };
 static_assert(sizeof(RunFields) == 32, "RunFields layout");
@@ -460,7 +459,7 @@ __global__ __launch_bounds__(256) void k_run(cplx<R>* __restrict__ psi, const Ru
         // that at size: 30 qubits 7.9 against 7.5 ms a pass.)
         __shared__ RunGate<R> gates[RUN_GATES];
         for (uint32_t t = threadIdx.x; t < (uint32_t)run.num * (sizeof(RunGate<R>) / 16); t += blockDim.x)
-            ((uint4*)gates)[t] = ((const uint4*)run.g)[t];
+            __builtin_memcpy((char*)gates + 16 * t, (const char*)run.g + 16 * t, 16);
         __syncthreads();
         for (int q = 0; q < run.num; q++) apply(gates[q].m, gates[q].f.uniform());
     } else {
