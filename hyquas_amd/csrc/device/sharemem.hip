@@ -465,7 +465,7 @@ private:
     {
         const uint32_t m = to_reg(t.tmask), v = to_reg(t.tval);
         for (int j = 0; j < nr_; j++)
-            if ((j & m) == v) { table_[j] *= t.f; used_[j] += t.real ? 0x100 : t.gates; }
+            if ((j & m) == v) { table_[j] *= t.f; used_[j] += t.real ? SIGN : (uint64_t)t.gates; }
         tdep_ |= m;
         tactive_ = true;
     }
@@ -482,7 +482,7 @@ private:
         o.jdep = tdep_;
         for (int j = 0; j < nr_; j++) {
             if (used_[j]) o.jmask |= 1ull << j;
-            if (precise_ && (used_[j] & 0xff) > 1) o.jprod |= 1ull << j;
+            if (precise_ && (used_[j] & (SIGN - 1)) > 1) o.jprod |= 1ull << j;
             tabs_->push_back(table_[j].real());
             tabs_->push_back(table_[j].imag());
         }
@@ -545,7 +545,8 @@ private:
     uint32_t regset_ = 0;
     int reg_[SHM_MAX_TILE], thr_[SHM_MAX_TILE];
     std::vector<std::complex<double>> table_;
-    std::vector<int> used_;     // gates in each entry (signs count 0x100 each)
+    static constexpr uint64_t SIGN = 1ull << 32;
+    std::vector<uint64_t> used_;   // gates in each entry, signs counted in the upper half
     uint32_t tdep_ = 0;
     bool tactive_ = false;
     std::complex<double> scale_{1.0, 0.0};

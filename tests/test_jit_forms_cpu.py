@@ -48,3 +48,13 @@ def test_diagonal_gates_across_block_bits_do_not_branch(hq, prec, variant):
     src = _source(hq, spec, prec, variant, n)
     assert re.search(r"pc = \(b & 0x[0-9a-f]+ull\) == 0x[0-9a-f]+ull;", src)
     assert "if ((b & " not in src
+
+
+@pytest.mark.parametrize("gates", [1, 2, 255, 256, 257, 258])
+def test_products_of_many_factors_keep_two_floats(hq, gates):
+    """A table entry of a complex64 program that is a product of several gates'
+    factors is held as two floats, however many they are."""
+    # between two H the target is a register bit, and the gates stay in one table
+    spec = [(H, 0, -1)] + [(RZ, 0, -1, (0.01 * (i + 1),)) for i in range(gates)] + [(H, 0, -1)]
+    src = _source(hq, spec, 1)
+    assert bool(re.search(r"const R ex\d+ = cf\[", src)) == (gates > 1)
