@@ -151,11 +151,13 @@ static hq_status launch_plain_gate(hq_state s, const hq_gate& g)
 // of 64 amplitudes), and a run of gates whose targets are among those ten bits
 // is applied in order; diagonal gates and controls may sit anywhere.  Register
 // targets are pair updates, lane targets one exchange with the partner lane.
-// Every branch is on the run's fields and uniform; controls select.  Random
-// layers, a gate on average, before and after: 10 qubits 3.1 -> 0.69 us, 20
-// qubits complex128 6.2 -> 1.31, 25 qubits 147 -> 16.8 (complex64 62 -> 7.5),
-// 30 qubits 4 890 -> 647.  A pass of 30 qubits runs at 4.7 TB/s with 11 gates;
-// a state of few waves is bound by the chain of a run's gates.
+// Branches are on the run's fields and uniform, but for the lanes a diagonal
+// gate skips; controls select.  Random layers, a gate on average, one by one and
+// in runs: 10 qubits (20 layers) 3.1 and 0.66 us, 20 qubits complex128 (20) 6.2 and
+// 1.34, 25 qubits (8) 147 and 15.5 (complex64 62 and 7.1), 30 qubits (30 layers) 4 890
+// and 507.  Those 1350 gates of 30 qubits are 88 runs of 15 gates on average, 7.7 ms
+// each (4.5 TB/s), and two single gates; a state of few waves is bound by the
+// chain of a run's gates (20 qubits: 26 us for 21).
 constexpr int RUN_MAX_RB = 4, RUN_LANES = 6, RUN_GATES = 32;
 constexpr int RUN_MIN_QUBITS = RUN_MAX_RB + RUN_LANES;
 // Up to here 8 amplitudes a thread: fewer gates fit a pass, but a pass is a
@@ -496,7 +498,7 @@ struct PlainGate {
 
 // The gates of the next pass, in order: those among the next RUN_AHEAD that
 // share no qubit with a gate left out before them (so that they commute with
-// it) and whose targets fit.  1350 gates of random layers on 30 qubits need 89
+// it) and whose targets fit.  1350 gates of random layers on 30 qubits need 90
 // passes, 190 without looking past the first gate that does not fit.
 constexpr size_t RUN_AHEAD = 256;
 

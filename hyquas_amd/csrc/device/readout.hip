@@ -12,8 +12,9 @@
 // parts and the part's amplitudes.  A thread walking its chunk amplitude by
 // amplitude took 1.56 ms for 100 000 shots of 25 qubits (and 0.8 ms for 4096,
 // the latency of one walk), beside 5 ms of searches on the host; this search
-// reads two lines a shot: 58 us and 7 us (the part sums add 40 us to the 87 us
-// pass over 512 MiB).
+// reads 512 B of part sums, one part (1 KiB in complex128) and three probes of
+// the prefix a lane and shot, one dependent step after another: 58 us and 6.4 us,
+// after 128 us for the sums (87 without the part sums, 512 MiB).
 
 #include "hq_device.h"
 #include "reduce_dev.h"
