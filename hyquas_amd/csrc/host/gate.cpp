@@ -271,23 +271,6 @@ Rng::Rng(uint64_t seed)
     for (int i = 0; i < 4; i++) s[i] = splitmix64(x);
 }
 
-static inline uint64_t rotl(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
-
-uint64_t Rng::next()
-{
-    const uint64_t result = rotl(s[1] * 5, 7) * 9;
-    const uint64_t t = s[1] << 17;
-    s[2] ^= s[0];
-    s[3] ^= s[1];
-    s[1] ^= s[2];
-    s[0] ^= s[3];
-    s[2] ^= t;
-    s[3] = rotl(s[3], 45);
-    return result;
-}
-
-double Rng::uniform() { return (double)(next() >> 11) * 0x1.0p-53; }
-
 uint64_t Rng::below(uint64_t m) { return ((next() >> 11) * m) >> 53; }
 
 }  // namespace hq

@@ -93,8 +93,25 @@ namespace hq {
 struct Rng {
     uint64_t s[4];
     explicit Rng(uint64_t seed);
-    uint64_t next();
-    double uniform();            // [0, 1)
+    // inline: a sample's uniforms are drawn while its sums run on the device and
+    // take longer (100 000 of 25 qubits; as calls between the library's files
+    // their time moved by a tenth with the code's placement in the library)
+    uint64_t next()
+    {
+        const uint64_t result = rotl(s[1] * 5, 7) * 9;
+        const uint64_t t = s[1] << 17;
+        s[2] ^= s[0];
+        s[3] ^= s[1];
+        s[1] ^= s[2];
+        s[0] ^= s[3];
+        s[2] ^= t;
+        s[3] = rotl(s[3], 45);
+        return result;
+    }
+    double uniform() { return (double)(next() >> 11) * 0x1.0p-53; }   // [0, 1)
     uint64_t below(uint64_t m);  // [0, m), m < 2^11
+
+private:
+    static uint64_t rotl(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
 };
 }  // namespace hq
