@@ -480,6 +480,8 @@ hq_status hq_state_topk(hq_state s, int k, uint64_t *idx, double *prob);
  * shot k is the smallest i with sum_{j<=i} |a_j|^2 > u_k * sum_j |a_j|^2, u_k
  * the k-th uniform of the portable generator seeded with `seed`.  No
  * counterpart in the reference (it reads P(q = 0), src/kernelSimple.cu:497-516).
+ * The state keeps the workspace of its readouts, for samples at most 128 MiB of
+ * device and 128 MiB of pinned host memory, until it is destroyed.
  * Synchronous. */
 hq_status hq_state_sample(hq_state s, int shots, uint64_t seed, uint64_t *out);
 
