@@ -330,8 +330,8 @@ hq_status build_sharemem_programs(hq_state s, const std::vector<SharememRequest>
     std::vector<std::vector<hq_program>> built(variants, std::vector<hq_program>(reqs.size(), nullptr));
     // complex64 kernels of large states keep diagonal gates apart: <Z_q> there
     // is of the order of what one rounding of a merged factor moves it by
-    // (ShmPlan::precise), and the pass is not bound by the operations saved
-    // (31 qubits, 18 groups: 128 ms merged, 126 ms apart)
+    // (ShmPlan::precise).  That costs 2 to 5 % of a run (26 qubits 3.61 ms apart,
+    // 3.42 merged as two floats; 31 qubits, 18 groups: 125.7 and 123.0 ms)
     const bool apart = jit && s->precision == HQ_C64;
     auto destroy_all = [&]() {
         for (auto& v : built)
